@@ -274,6 +274,29 @@ int qmoe_moe_gate_up_swiglu_tiles_topk(const uint16_t* x, const float* logits,
                                        int64_t I, uint16_t* h, int32_t* idx,
                                        float* scores, void* stream);
 
+/* The same two decode launches with the layer's sigmoid-gated shared expert
+ * (qwen3_5_moe/language.py:81-89: sigmoid(x . sh_gate) * SwiGLU-MLP(x)) as one
+ * more slot per token: h [T, top_k + 1, I], idx and scores [T, top_k + 1], the
+ * last slot the shared expert's (id num_experts, score sigmoid(x . sh_gate) in
+ * fp32).  sh_wp / sh_sb are its tile-layout gate_up (paired row order) and down
+ * weights, one expert of the routed experts' shape; sh_gate bf16 [K].  The down
+ * call takes slots = top_k + 1 (<= 16) and sums all of them in fp32 into one
+ * bf16 rounding. */
+int qmoe_moe_gate_up_swiglu_tiles_topk_shared(
+    const uint16_t* x, const float* logits, int norm, int64_t T, int64_t top_k,
+    int64_t K, const uint32_t* wp, const uint32_t* sb, int32_t num_experts,
+    int64_t I, const uint32_t* sh_wp, const uint32_t* sh_sb,
+    const uint16_t* sh_gate, uint16_t* h, int32_t* idx, float* scores,
+    void* stream);
+int qmoe_moe_down_wsum_tiles_shared(const uint16_t* h, const int32_t* idx,
+                                    const float* scores, int64_t T,
+                                    int64_t slots, int64_t I,
+                                    const uint32_t* wp, const uint32_t* sb,
+                                    int32_t num_experts, int64_t D,
+                                    const uint32_t* sh_wp,
+                                    const uint32_t* sh_sb, uint16_t* y,
+                                    void* stream);
+
 /* ------------------------------------------------------------------ int8 --
  * int8-activation x int4-weight gate_up (replaces
  * titan/kernels/moe_gather_int8.py:132-182 quantize_activations and

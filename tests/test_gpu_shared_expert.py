@@ -1,0 +1,95 @@
+"""The shared expert as one more slot of the decode kernels
+(qmoe_moe_gate_up_swiglu_tiles_topk_shared, qmoe_moe_down_wsum_tiles_shared)
+against the id-taking kernels and a 64-bit product."""
+
+import pytest
+import torch
+
+from titan_amd import ops
+from titan_amd.moe_block import SharedExpert, SparseMoeBlock
+
+pytestmark = pytest.mark.gpu
+
+
+def _quant(g, lead, K, dev):
+    w = torch.randint(-2 ** 31, 2 ** 31, (*lead, K // 8), dtype=torch.int32, device=dev, generator=g)
+    s = (0.004 + 0.004 * torch.rand(*lead, K // 64, device=dev, generator=g)).to(torch.bfloat16)
+    return w, s, (-7.5 * s.float()).to(torch.bfloat16)
+
+
+def _deq64(q):
+    w, s, b = q
+    shifts = torch.arange(0, 32, 4, device=w.device, dtype=torch.int32)
+    c = ((w.unsqueeze(-1) >> shifts) & 15).reshape(*w.shape[:-1], -1).double()
+    return c * s.double().repeat_interleave(64, -1) + b.double().repeat_interleave(64, -1)
+
+
+def _close_bf16(y, ref):
+    """One bf16 rounding (2^-9 of a value) of sums in fp32: n * 2^-24 of the
+    sum of magnitudes, far below 2^-14 of the largest output."""
+    err = (y.double() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * ref.abs() + 2.0 ** -14 * ref.abs().max()).all()), float(err.max())
+
+
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("T,k,H,E", [(1, 10, 2048, 256), (2, 1, 2048, 3), (16, 15, 4096, 300), (3, 4, 6144, 5),
+                                     (5, 2, 8192, 64)])
+def test_shared_slot_decode(dev, T, k, H, E, norm):
+    print(f"[case] shared slot T={T} k={k} H={H} E={E} norm={norm}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T * 100 + k)
+    I = 512
+    gu, dn = _quant(g, (E, 2 * I), H, dev), _quant(g, (E, H), I, dev)
+    sgu, sdn = _quant(g, (1, 2 * I), H, dev), _quant(g, (1, H), I, dev)
+    gate = (torch.randn(1, H, device=dev, generator=g) * H ** -0.5).to(torch.bfloat16)
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    logits = torch.randn(T, E, device=dev, generator=g)
+    tw, stw = ops.repack_tiles(*gu, swiglu_pairs=True), ops.repack_tiles(*sgu, swiglu_pairs=True)
+    td, std = ops.repack_tiles(*dn), ops.repack_tiles(*sdn)
+    h, idx, sc = ops.gate_up_silu_tiles_topk_shared(x, tw, logits, k, stw, gate, norm)
+    h0, idx0, sc0 = ops.gate_up_silu_tiles_topk(x, tw, logits, k, norm)
+    assert torch.equal(h[:, :k], h0) and torch.equal(idx[:, :k], idx0) and torch.equal(sc[:, :k], sc0)
+    zeros = torch.zeros(T, 1, dtype=torch.int32, device=dev)
+    assert torch.equal(h[:, k:], ops.gate_up_silu_tiles(x, stw, zeros))
+    assert bool((idx[:, k] == E).all())
+    z = x.double() @ gate.double().t()
+    # the logit's fp32 sum is within K * 2^-24 of sum |x w|; the sigmoid's slope is at most 1/4
+    bound = 0.25 * H * 2.0 ** -24 * (x.double().abs() @ gate.double().abs().t()) + 4 * 2.0 ** -24
+    assert bool(((sc[:, k:].double() - torch.sigmoid(z)).abs() <= bound).all())
+    y = ops.down_wsum_tiles_shared(h, td, idx, sc, std)
+    ref = torch.zeros(T, H, dtype=torch.float64, device=dev)
+    dn64, sdn64 = _deq64(dn) if E <= 5 else None, _deq64(sdn)[0]
+    for t in range(T):
+        for j in range(k):
+            e = int(idx[t, j])
+            we = dn64[e] if dn64 is not None else _deq64(tuple(q[e] for q in dn))
+            ref[t] += sc[t, j].double() * (we @ h[t, j].double())
+        ref[t] += sc[t, k].double() * (sdn64 @ h[t, k].double())
+    _close_bf16(y, ref)
+
+
+@pytest.mark.parametrize("T", [1, 6, 7, 16])
+@pytest.mark.parametrize("k,S", [(10, 512), (16, 512), (10, 768)])
+def test_block_with_shared_expert_matches_its_parts(dev, T, k, S):
+    """The block over every dispatch of its shared expert (a slot of the
+    decode kernels, k at their limit, another width) against the routed part
+    and the shared part on their own."""
+    print(f"[case] block with shared expert T={T} k={k} S={S}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T + k + S)
+    E, H, I = 32, 2048, 512
+    gu, dn = _quant(g, (E, 2 * I), H, dev), _quant(g, (E, H), I, dev)
+    sgu, sdn = _quant(g, (1, 2 * S), H, dev), _quant(g, (1, H), S, dev)
+    gate = (torch.randn(1, H, device=dev, generator=g) * H ** -0.5).to(torch.bfloat16)
+    router = (torch.randn(E, H, device=dev, generator=g) * H ** -0.5).to(torch.bfloat16)
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    block = SparseMoeBlock(router, gu, dn, k, shared=SharedExpert(sgu, sdn, gate))
+    y = block(x)
+    idx, sc = block.route(x)
+    routed = block.experts(x, idx, sc).double()
+    gate_up = x.double() @ _deq64(sgu)[0].t()
+    a, u = gate_up.chunk(2, dim=-1)
+    shared = (torch.nn.functional.silu(a) * u) @ _deq64(sdn)[0].t()
+    shared = torch.sigmoid(x.double() @ gate.double().t()) * shared
+    ref = routed + shared
+    # the routed part's bf16 rounding, h's, and the sum's: 3 * 2^-9 of the
+    # parts' magnitudes, the block's own bar of 2^-7 of max|y|
+    assert bool(((y.double() - ref).abs() <= 2.0 ** -7 * ref.abs().max()).all())

@@ -14,6 +14,7 @@
 // This is the factored affine form of the reference decode kernels
 // (engine/patches/decode-fusion/fused_kernels.py:57-79), with the codes fed
 // to the dot unit two at a time.
+#include <limits.h>
 #include <stdarg.h>
 
 #include <stdlib.h>
@@ -189,6 +190,11 @@ struct QmvArgs {
   int32_t* topk_idx = nullptr;
   float* topk_scores = nullptr;
   int topk_norm = 1;
+  // with a shared expert (SH): its tile-layout weights, and the dense row
+  // whose product with x, through a sigmoid, is its score
+  const uint32_t* sh_w = nullptr;
+  const uint32_t* sh_sb = nullptr;
+  const uint16_t* sh_gate = nullptr;
 };
 
 // The expert of pair pr = t * k + j of the tiled SwiGLU form: experts[pr], or
@@ -197,7 +203,15 @@ struct QmvArgs {
 // wave of the token's first column block and last slot, j = k - 1, also
 // writes the token's k ids and scores: it runs the whole selection here, keeps
 // it in ts, and computes and stores the scores in pair_topk_store, which the
-// kernel calls once its weight loads are in flight.  Wave-uniform.
+// kernel calls once its weight loads are in flight.  Wave-uniform.  SH: every
+// token has a (k + 1)-th slot, the shared expert (kSharedSlot returned), and
+// the ids and scores have k + 1 entries per token.  A decode block's time is
+// its number of dependent launches (~2-4 us each, whatever their few KiB), and
+// the shared expert run apart took 13 of its 18: in a graph of six layers
+// (256 experts, top-10, hidden 2048, 8-bit router) the block with a shared
+// expert went from 38.8 to 15.5 us a layer at one token, 56.3 to 29.3 at four.
+constexpr int kSharedSlot = INT_MIN;
+
 template <int PER>
 struct PairTopk {
   bool writer = false;
@@ -206,14 +220,16 @@ struct PairTopk {
   uint32_t key_j = 0;
 };
 
-template <int PER>
+template <int PER, bool SH = false>
 __device__ __forceinline__ int pair_expert(const QmvArgs& a, uint32_t pr, uint32_t t, bool first_block,
                                            PairTopk<PER>& ts) {
   if constexpr (PER == 0) {
     return a.experts[pr];
   } else {
-    const int k = (int)a.x_div;
-    const int j = __builtin_amdgcn_readfirstlane((int)(pr - t * (uint32_t)k));
+    const int slots = (int)a.x_div;
+    const int k = SH ? slots - 1 : slots;
+    const int j = __builtin_amdgcn_readfirstlane((int)(pr - t * (uint32_t)slots));
+    if (SH && j == k) return kSharedSlot;
     const float* lp = a.logits + (int64_t)t * a.num_experts;
     ts.writer = first_block && j == k - 1;
     if (!ts.writer) return qmoe_topk::wave_topk_last<PER>(lp, a.num_experts, j + 1);
@@ -222,17 +238,46 @@ __device__ __forceinline__ int pair_expert(const QmvArgs& a, uint32_t pr, uint32
   }
 }
 
-template <int PER>
+template <int PER, bool SH = false>
 __device__ __forceinline__ void pair_topk_store(const QmvArgs& a, uint32_t t, const PairTopk<PER>& ts) {
   if constexpr (PER > 0) {
     if (!ts.writer) return;
-    const int k = (int)a.x_div;
+    const int slots = (int)a.x_div;
+    const int k = SH ? slots - 1 : slots;
     const float sc = qmoe_topk::wave_topk_scores<PER>(ts.v, k, a.topk_norm, ts.key_j);
     const int lane = threadIdx.x & 63;
     if (lane < k) {
-      a.topk_idx[(int64_t)t * k + lane] = ts.idx;
-      a.topk_scores[(int64_t)t * k + lane] = sc;
+      a.topk_idx[(int64_t)t * slots + lane] = ts.idx;
+      a.topk_scores[(int64_t)t * slots + lane] = sc;
     }
+  }
+}
+
+// The shared expert's score of token t (language.py:81-89): sigmoid(x . gate)
+// in fp32, from the x row the wave holds (lane l: elements v*2048 + 32l ..),
+// written to the token's last slot with id num_experts (the routed experts end
+// below it; the down kernel goes by the slot).
+template <int NV>
+__device__ __forceinline__ void shared_score_store(const QmvArgs& a, uint32_t t, const uint4 (&xa)[NV][4]) {
+  const int lane = threadIdx.x & 63;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const uint4* gp = reinterpret_cast<const uint4*>(a.sh_gate + v * 2048 + lane * 32);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint4 gq = gp[q];
+      acc[q] = dot2_bf16(xa[v][q].x, gq.x, acc[q]);
+      acc[q] = dot2_bf16(xa[v][q].y, gq.y, acc[q]);
+      acc[q] = dot2_bf16(xa[v][q].z, gq.z, acc[q]);
+      acc[q] = dot2_bf16(xa[v][q].w, gq.w, acc[q]);
+    }
+  }
+  const float z = qmoe_topk::wave_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
+  if (lane == 0) {
+    const int64_t o = ((int64_t)t + 1) * a.x_div - 1;
+    a.topk_idx[o] = a.num_experts;
+    a.topk_scores[o] = 1.0f / (1.0f + expf(-z));
   }
 }
 
@@ -857,7 +902,7 @@ __global__ __launch_bounds__(64) void qmv64_tiled_kernel(QmvArgs a) {
 // XCD-contiguously (xcd_item), so the row groups sharing a scale|bias chunk
 // run on one XCD.  Per lane and row the arithmetic and the reduction tree are
 // those of qmv64_kernel's fused form, so the result is bit-identical to it.
-template <int NV, int RG, int PER = 0>
+template <int NV, int RG, int PER = 0, bool SH = false>
 __global__ __launch_bounds__(64) void qmv64_paired_kernel(QmvArgs a) {
   static_assert(RG == 4 || RG == 8, "four or eight indices per wave");
   const int lane = threadIdx.x;
@@ -875,8 +920,11 @@ __global__ __launch_bounds__(64) void qmv64_paired_kernel(QmvArgs a) {
   for (int v = 0; v < NV; ++v)
 #pragma unroll
     for (int q = 0; q < 4; ++q) xa[v][q] = reinterpret_cast<const uint4*>(xrow + v * 2048 + lane * 32)[q];
-  if constexpr (PER > 0) e = pair_expert<PER>(a, r, xr, i0 == 0, ts);
-  e = min(max(e, 0), a.num_experts - 1);
+  if constexpr (PER > 0) e = pair_expert<PER, SH>(a, r, xr, i0 == 0, ts);
+  const bool shared = SH && e == kSharedSlot;  // wave-uniform
+  const uint32_t* wbase = shared ? a.sh_w : a.w;
+  const uint32_t* sbbase = shared ? a.sh_sb : a.sb;
+  e = shared ? 0 : min(max(e, 0), a.num_experts - 1);
   const int G = 32 * NV;
   const int NC = a.n_w / 64;
   const int c = i0 >> 5, l0 = i0 & 31;
@@ -889,7 +937,7 @@ __global__ __launch_bounds__(64) void qmv64_paired_kernel(QmvArgs a) {
   for (int v = 0; v < NV; ++v)
 #pragma unroll
     for (int t = 0; t < RG / 4; ++t) {
-      const uint32_t* base = a.sb + (chunk0 + v * 32) * 64 + l0 + 4 * t;
+      const uint32_t* base = sbbase + (chunk0 + v * 32) * 64 + l0 + 4 * t;
       sg[v][t] = *reinterpret_cast<const uint4*>(base);
       su[v][t] = *reinterpret_cast<const uint4*>(base + 32);
     }
@@ -898,11 +946,12 @@ __global__ __launch_bounds__(64) void qmv64_paired_kernel(QmvArgs a) {
   for (int q = 0; q < RG; ++q)
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const uint4* units = reinterpret_cast<const uint4*>(a.w) + ((chunk0 + v * 32) * 4 + h) * 32 + l0 + q;
+      const uint4* units = reinterpret_cast<const uint4*>(wbase) + ((chunk0 + v * 32) * 4 + h) * 32 + l0 + q;
       wg[q][v] = load_nt(units);       // half j = 0: gate
       wu[q][v] = load_nt(units + 64);  // half j = 1: up, two 32-unit halves further
     }
-  pair_topk_store<PER>(a, xr, ts);  // while the weights are in flight
+  pair_topk_store<PER, SH>(a, xr, ts);  // while the weights are in flight
+  if (SH && shared && i0 == 0) shared_score_store<NV>(a, xr, xa);
   XChunk xc[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
@@ -962,7 +1011,7 @@ __global__ __launch_bounds__(64) void qmv64_paired_kernel(QmvArgs a) {
 // nibble pairs, and the chunk's sum) and each lane reads the chunk of its
 // (g, h) per step.  Per lane the affine chunk arithmetic is qmv64_kernel's;
 // the row sums close over the eight group slots with three DPP steps.
-template <int NV, int RG, int PER = 0>
+template <int NV, int RG, int PER = 0, bool SH = false>
 __global__ __launch_bounds__(64) void qmv64_paired_lines_kernel(QmvArgs a) {
   static_assert(RG == 4 || RG == 8, "four or eight indices per wave");
   constexpr int NCH = 64 * NV;   // 32-element chunks of x
@@ -988,8 +1037,11 @@ __global__ __launch_bounds__(64) void qmv64_paired_lines_kernel(QmvArgs a) {
   for (int v = 0; v < NV; ++v)
 #pragma unroll
     for (int q = 0; q < 4; ++q) xa[v][q] = reinterpret_cast<const uint4*>(xrow + v * 2048 + lane * 32)[q];
-  if constexpr (PER > 0) e = pair_expert<PER>(a, pr, xr, i0 == 0, ts);
-  e = min(max(e, 0), a.num_experts - 1);
+  if constexpr (PER > 0) e = pair_expert<PER, SH>(a, pr, xr, i0 == 0, ts);
+  const bool shared = SH && e == kSharedSlot;  // wave-uniform
+  const uint32_t* wbase = shared ? a.sh_w : a.w;
+  const uint32_t* sbbase = shared ? a.sh_sb : a.sb;
+  e = shared ? 0 : min(max(e, 0), a.num_experts - 1);
   const int G = 32 * NV;
   const int NC = a.n_w / 64;
   const int c = i0 >> 5, l0 = i0 & 31;
@@ -999,7 +1051,7 @@ __global__ __launch_bounds__(64) void qmv64_paired_lines_kernel(QmvArgs a) {
   uint4 wv[NP][2][NJ];  // [step][h][row half]
 #pragma unroll
   for (int pp = 0; pp < NP; ++pp) {
-    const uint32_t* sbc = a.sb + (cbase + 8 * pp + sl) * 64 + l0 + rr;
+    const uint32_t* sbc = sbbase + (cbase + 8 * pp + sl) * 64 + l0 + rr;
 #pragma unroll
     for (int jj = 0; jj < NJ; ++jj) sbw[pp][jj] = sbc[32 * (jr + jj)];
   }
@@ -1010,9 +1062,10 @@ __global__ __launch_bounds__(64) void qmv64_paired_lines_kernel(QmvArgs a) {
 #pragma unroll
       for (int jj = 0; jj < NJ; ++jj) {
         const int64_t chunk = cbase + 8 * pp + sl;
-        wv[pp][h][jj] = load_nt(reinterpret_cast<const uint4*>(a.w) + ((chunk * 2 + jr + jj) * 2 + h) * 32 + l0 + rr);
+        wv[pp][h][jj] = load_nt(reinterpret_cast<const uint4*>(wbase) + ((chunk * 2 + jr + jj) * 2 + h) * 32 + l0 + rr);
       }
-  pair_topk_store<PER>(a, xr, ts);  // while the weights are in flight
+  pair_topk_store<PER, SH>(a, xr, ts);  // while the weights are in flight
+  if (SH && shared && i0 == 0) shared_score_store<NV>(a, xr, xa);
   // stage x: lane l writes chunk v*64 + l (elements v*2048 + 32l ..)
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
@@ -1085,6 +1138,9 @@ struct DownArgs {
   int num_experts, D;
   uint16_t* y;  // [T, D]
   const uint32_t* sb;  // tile layout: scale|bias words (w then holds the tile-layout codes)
+  // with a shared expert (SH): slot k - 1 of every token reads these weights
+  const uint32_t* sh_w = nullptr;
+  const uint32_t* sh_sb = nullptr;
 };
 
 // One block per group of 64/LPR output rows; wave t handles token t and walks
@@ -1222,7 +1278,7 @@ __global__ __launch_bounds__(64 * kPairMaxK) void down_pair_kernel(DownArgs a) {
 // wave instead, each touching eight chunks, cost 17-23% of the kernel at 8
 // and 16 tokens.  Eight lanes per line with two h chunks per lane measured
 // slower: every wave then reads twice the h row.)
-template <int R>
+template <int R, bool SH = false>
 __global__ __launch_bounds__(64 * kPairMaxK) void down_pair_tiled_kernel(DownArgs a) {
   constexpr int NI = R / 4;
   __shared__ float red[kPairMaxK][R];
@@ -1237,13 +1293,16 @@ __global__ __launch_bounds__(64 * kPairMaxK) void down_pair_tiled_kernel(DownArg
   const int64_t p = (int64_t)t * a.k + j;
   XChunk hc;
   load_x_chunk(a.h + p * 512 + l * 32, hc);
-  int e = a.idx[p];
+  const bool shared = SH && __builtin_amdgcn_readfirstlane(j) == a.k - 1;
+  int e = shared ? 0 : a.idx[p];
   e = min(max(e, 0), a.num_experts - 1);
+  const uint32_t* wbase = shared ? a.sh_w : a.w;
+  const uint32_t* sbbase = shared ? a.sh_sb : a.sb;
   const float sc = a.scores[p];
   static_assert(R == 8 || R == 16, "rows per wave");
   // D % 64 == 0 and d0 % R == 0: the wave's rows lie in one 64-row chunk
   const int64_t chunk = ((int64_t)e * NCd + (d0 >> 6)) * 8 + g;
-  const uint32_t* sbg = a.sb + chunk * 64 + (d0 & 63);
+  const uint32_t* sbg = sbbase + chunk * 64 + (d0 & 63);
   uint4 sq;
   uint32_t s1;
   if constexpr (NI == 4) sq = *reinterpret_cast<const uint4*>(sbg + 4 * rg);
@@ -1252,7 +1311,7 @@ __global__ __launch_bounds__(64 * kPairMaxK) void down_pair_tiled_kernel(DownArg
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int row = d0 + 4 * i + rg;
-    wq[i] = *(reinterpret_cast<const uint4*>(a.w) + ((chunk * 2 + ((row >> 5) & 1)) * 2 + h) * 32 + (row & 31));
+    wq[i] = *(reinterpret_cast<const uint4*>(wbase) + ((chunk * 2 + ((row >> 5) & 1)) * 2 + h) * 32 + (row & 31));
   }
   uint32_t sbw[NI];  // the scale|bias word of row d0 + 4i + rg, group g
   if constexpr (NI == 4) {
@@ -1491,7 +1550,7 @@ int launch_qmv_tiled(const QmvArgs& a, hipStream_t st) {
   return qmoe::launch_status("qmv64_tiled_kernel");
 }
 
-template <int RG, int PER = 0>
+template <int RG, int PER = 0, bool SH = false>
 int launch_qmv_paired_rg(QmvArgs a, hipStream_t st) {
   const int64_t nblk = a.n_out / RG;
   const int64_t blocks = a.n_pairs * nblk;
@@ -1502,12 +1561,12 @@ int launch_qmv_paired_rg(QmvArgs a, hipStream_t st) {
   a.x_divf = make_fastdiv((uint32_t)a.x_div);
   dim3 grid((unsigned)blocks), block(64);
   switch (a.K / 2048) {
-    case 1: qmv64_paired_kernel<1, RG, PER><<<grid, block, 0, st>>>(a); break;
-    case 2: qmv64_paired_kernel<2, RG, PER><<<grid, block, 0, st>>>(a); break;
+    case 1: qmv64_paired_kernel<1, RG, PER, SH><<<grid, block, 0, st>>>(a); break;
+    case 2: qmv64_paired_kernel<2, RG, PER, SH><<<grid, block, 0, st>>>(a); break;
     default:
       if constexpr (RG == 4) {
-        if (a.K / 2048 == 3) qmv64_paired_kernel<3, 4, PER><<<grid, block, 0, st>>>(a);
-        else qmv64_paired_kernel<4, 4, PER><<<grid, block, 0, st>>>(a);
+        if (a.K / 2048 == 3) qmv64_paired_kernel<3, 4, PER, SH><<<grid, block, 0, st>>>(a);
+        else qmv64_paired_kernel<4, 4, PER, SH><<<grid, block, 0, st>>>(a);
       } else {
         return qmoe::fail(QMOE_ERR_UNSUPPORTED, "K=%d: %d indices per wave take K <= 4096", a.K, RG);
       }
@@ -1524,7 +1583,7 @@ int launch_qmv_paired_rg(QmvArgs a, hipStream_t st) {
 #define QMOE_PAIRED_LINES_RG 4
 #endif
 
-template <int PER = 0>
+template <int PER = 0, bool SH = false>
 int launch_qmv_paired(const QmvArgs& a, hipStream_t st) {
   if (a.K <= 4096) {
     // line reads with x staged in LDS (K = 2048 or 4096)
@@ -1538,11 +1597,11 @@ int launch_qmv_paired(const QmvArgs& a, hipStream_t st) {
     b.blk_div = make_fastdiv((uint32_t)nblk);
     b.x_divf = make_fastdiv((uint32_t)a.x_div);
     dim3 grid((unsigned)blocks), block(64);
-    if (a.K == 2048) qmv64_paired_lines_kernel<1, RG, PER><<<grid, block, 0, st>>>(b);
-    else qmv64_paired_lines_kernel<2, RG, PER><<<grid, block, 0, st>>>(b);
+    if (a.K == 2048) qmv64_paired_lines_kernel<1, RG, PER, SH><<<grid, block, 0, st>>>(b);
+    else qmv64_paired_lines_kernel<2, RG, PER, SH><<<grid, block, 0, st>>>(b);
     return qmoe::launch_status("qmv64_paired_lines_kernel");
   }
-  return launch_qmv_paired_rg<4, PER>(a, st);
+  return launch_qmv_paired_rg<4, PER, SH>(a, st);
 }
 
 int check_tiled(int64_t K, int64_t rows_per_expert, const void* x, const void* wp, const void* sb) {
@@ -1709,9 +1768,14 @@ extern "C" int qmoe_moe_gate_up_swiglu_tiles(const uint16_t* x, const int32_t* i
   return launch_qmv_paired(a, qmoe::as_stream(stream));
 }
 
-extern "C" int qmoe_moe_down_wsum_tiles(const uint16_t* h, const int32_t* idx, const float* scores, int64_t T,
-                                        int64_t top_k, int64_t I, const uint32_t* wp, const uint32_t* sb,
-                                        int32_t num_experts, int64_t D, uint16_t* y, void* stream) {
+namespace {
+
+// The tile-layout down kernel over k slots per token, the last one the shared
+// expert's when SH.
+template <bool SH>
+int down_wsum_tiles(const uint16_t* h, const int32_t* idx, const float* scores, int64_t T, int64_t top_k, int64_t I,
+                    const uint32_t* wp, const uint32_t* sb, int32_t num_experts, int64_t D, const uint32_t* sh_wp,
+                    const uint32_t* sh_sb, uint16_t* y, void* stream) {
   if (T < 0 || top_k <= 0 || D <= 0 || num_experts <= 0) return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
   if (T == 0) return QMOE_OK;
   if (!h || !idx || !scores || !wp || !sb || !y) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
@@ -1723,13 +1787,35 @@ extern "C" int qmoe_moe_down_wsum_tiles(const uint16_t* h, const int32_t* idx, c
   if (!qmoe::aligned16(h) || !qmoe::aligned16(wp) || !qmoe::aligned16(sb))
     return qmoe::fail(QMOE_ERR_UNSUPPORTED, "h, wp and sb must be 16-byte aligned");
   DownArgs a{h, idx, scores, (int)T, (int)top_k, (int)I, 64, wp, nullptr, nullptr, num_experts, (int)D, y, sb};
+  if (SH) {
+    if (!sh_wp || !sh_sb) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+    if (!qmoe::aligned16(sh_wp) || !qmoe::aligned16(sh_sb))
+      return qmoe::fail(QMOE_ERR_UNSUPPORTED, "the shared weights must be 16-byte aligned");
+    a.sh_w = sh_wp;
+    a.sh_sb = sh_sb;
+  }
   hipStream_t st = qmoe::as_stream(stream);
   // rows per wave as for the MLX-layout kernel: 8 for one token, 16 from two on
   const int R = T == 1 ? 8 : 16;
   dim3 grid((unsigned)(D / R), (unsigned)T), block((unsigned)(64 * top_k));
-  if (R == 8) down_pair_tiled_kernel<8><<<grid, block, 0, st>>>(a);
-  else down_pair_tiled_kernel<16><<<grid, block, 0, st>>>(a);
+  if (R == 8) down_pair_tiled_kernel<8, SH><<<grid, block, 0, st>>>(a);
+  else down_pair_tiled_kernel<16, SH><<<grid, block, 0, st>>>(a);
   return qmoe::launch_status("down_pair_tiled_kernel");
+}
+
+}  // namespace
+
+extern "C" int qmoe_moe_down_wsum_tiles(const uint16_t* h, const int32_t* idx, const float* scores, int64_t T,
+                                        int64_t top_k, int64_t I, const uint32_t* wp, const uint32_t* sb,
+                                        int32_t num_experts, int64_t D, uint16_t* y, void* stream) {
+  return down_wsum_tiles<false>(h, idx, scores, T, top_k, I, wp, sb, num_experts, D, nullptr, nullptr, y, stream);
+}
+
+extern "C" int qmoe_moe_down_wsum_tiles_shared(const uint16_t* h, const int32_t* idx, const float* scores, int64_t T,
+                                               int64_t slots, int64_t I, const uint32_t* wp, const uint32_t* sb,
+                                               int32_t num_experts, int64_t D, const uint32_t* sh_wp,
+                                               const uint32_t* sh_sb, uint16_t* y, void* stream) {
+  return down_wsum_tiles<true>(h, idx, scores, T, slots, I, wp, sb, num_experts, D, sh_wp, sh_sb, y, stream);
 }
 
 namespace {
@@ -1745,12 +1831,14 @@ int check_topk(const float* logits, int64_t top_k, int32_t num_experts, int* per
   *per = num_experts <= 256 ? 4 : 16;
   return QMOE_OK;
 }
-}  // namespace
 
-extern "C" int qmoe_moe_gate_up_swiglu_tiles_topk(const uint16_t* x, const float* logits, int norm, int64_t T,
-                                                  int64_t top_k, int64_t K, const uint32_t* wp, const uint32_t* sb,
-                                                  int32_t num_experts, int64_t I, uint16_t* h, int32_t* idx,
-                                                  float* scores, void* stream) {
+// The tile-layout gate_up decode kernel that selects its experts, with the
+// shared expert as every token's slot top_k when SH.
+template <bool SH>
+int gate_up_tiles_topk(const uint16_t* x, const float* logits, int norm, int64_t T, int64_t top_k, int64_t K,
+                       const uint32_t* wp, const uint32_t* sb, int32_t num_experts, int64_t I, const uint32_t* sh_wp,
+                       const uint32_t* sh_sb, const uint16_t* sh_gate, uint16_t* h, int32_t* idx, float* scores,
+                       void* stream) {
   if (T < 0 || top_k <= 0 || I <= 0 || num_experts <= 0) return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
   if (T == 0) return QMOE_OK;
   if (!x || !wp || !sb || !h || !idx || !scores) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
@@ -1760,14 +1848,42 @@ extern "C" int qmoe_moe_gate_up_swiglu_tiles_topk(const uint16_t* x, const float
   if (I % 32) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "I=%lld: the paired layout needs I %% 32 == 0", (long long)I);
   rc = check_tiled(K, 2 * I, x, wp, sb);
   if (rc) return rc;
-  QmvArgs a{x, K, nullptr, top_k, nullptr, T * top_k, (int)K, 64, wp, nullptr, nullptr, num_experts, (int)I,
+  if (SH) {
+    if (!sh_wp || !sh_sb || !sh_gate) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+    if (!qmoe::aligned16(sh_wp) || !qmoe::aligned16(sh_sb) || !qmoe::aligned16(sh_gate))
+      return qmoe::fail(QMOE_ERR_UNSUPPORTED, "the shared weights must be 16-byte aligned");
+  }
+  const int64_t slots = top_k + (SH ? 1 : 0);
+  QmvArgs a{x, K, nullptr, slots, nullptr, T * slots, (int)K, 64, wp, nullptr, nullptr, num_experts, (int)I,
             (int)(2 * I), h, sb};
+  a.sh_w = sh_wp;
+  a.sh_sb = sh_sb;
+  a.sh_gate = sh_gate;
   a.logits = logits;
   a.topk_idx = idx;
   a.topk_scores = scores;
   a.topk_norm = norm ? 1 : 0;
   hipStream_t st = qmoe::as_stream(stream);
-  return per == 4 ? launch_qmv_paired<4>(a, st) : launch_qmv_paired<16>(a, st);
+  return per == 4 ? launch_qmv_paired<4, SH>(a, st) : launch_qmv_paired<16, SH>(a, st);
+}
+}  // namespace
+
+extern "C" int qmoe_moe_gate_up_swiglu_tiles_topk(const uint16_t* x, const float* logits, int norm, int64_t T,
+                                                  int64_t top_k, int64_t K, const uint32_t* wp, const uint32_t* sb,
+                                                  int32_t num_experts, int64_t I, uint16_t* h, int32_t* idx,
+                                                  float* scores, void* stream) {
+  return gate_up_tiles_topk<false>(x, logits, norm, T, top_k, K, wp, sb, num_experts, I, nullptr, nullptr, nullptr, h,
+                                   idx, scores, stream);
+}
+
+extern "C" int qmoe_moe_gate_up_swiglu_tiles_topk_shared(const uint16_t* x, const float* logits, int norm, int64_t T,
+                                                         int64_t top_k, int64_t K, const uint32_t* wp,
+                                                         const uint32_t* sb, int32_t num_experts, int64_t I,
+                                                         const uint32_t* sh_wp, const uint32_t* sh_sb,
+                                                         const uint16_t* sh_gate, uint16_t* h, int32_t* idx,
+                                                         float* scores, void* stream) {
+  return gate_up_tiles_topk<true>(x, logits, norm, T, top_k, K, wp, sb, num_experts, I, sh_wp, sh_sb, sh_gate, h, idx,
+                                  scores, stream);
 }
 
 #ifdef QMOE_QMV_STAMPS

@@ -25,7 +25,9 @@ softmax to bf16 first and breaks bf16 ties arbitrarily
 near-ties; everything after the selection has the same semantics.
 
 The optional shared expert (language.py:81-89: a dense SwiGLU MLP gated by
-sigmoid(x w_gate)) runs through the same kernels as a one-expert table.
+sigmoid(x w_gate)) is one more slot of the two decode kernels when it has the
+routed experts' shape, so the decode block stays three launches; otherwise it
+runs through the same kernels as a one-expert table.
 
 Resident weights (``resident``): by default one copy, in the tile layout --
 the block repacks gate_up (in the gate/up-paired row order) and down at
@@ -151,6 +153,11 @@ class SparseMoeBlock:
             if self.resident == "tiles" and tile_decode_supported(self.hidden, S, group_size, bits):
                 self._shared_decode_tiles = True
                 self.shared = SharedExpert(None, None, shared.gate_weight)
+        # a shared expert of the routed experts' shape is one more slot of the
+        # decode kernels (qmoe_moe_*_shared)
+        self._shared_slot = (self.decode_tiles and self._shared_decode_tiles and self.top_k < TILE_DECODE_MAX_K
+                             and self._shared_tiles[0].N == self.gu_tiles.N
+                             and shared.gate_weight.numel() == self.hidden)
 
     @property
     def nbytes(self) -> int:
@@ -229,6 +236,11 @@ class SparseMoeBlock:
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         H = x.shape[-1]
         x2 = x.reshape(-1, H).to(torch.bfloat16).contiguous()
+        if self._shared_slot and self.decodes_with_topk(x2.shape[0]):
+            gu_t, dn_t = self._shared_tiles
+            h, idx, scores = ops.gate_up_silu_tiles_topk_shared(x2, self.gu_tiles, self.route_logits(x2), self.top_k,
+                                                                gu_t, self.shared.gate_weight, self.norm)
+            return ops.down_wsum_tiles_shared(h, self.down_tiles, idx, scores, dn_t).reshape(x.shape)
         if self.decodes_with_topk(x2.shape[0]):
             h, idx, scores = ops.gate_up_silu_tiles_topk(x2, self.gu_tiles, self.route_logits(x2), self.top_k,
                                                          self.norm)

@@ -411,6 +411,47 @@ def gate_up_silu_tiles_topk(x: torch.Tensor, tw: TileWeights, logits: torch.Tens
     return h, idx, scores
 
 
+def gate_up_silu_tiles_topk_shared(x: torch.Tensor, tw: TileWeights, logits: torch.Tensor, top_k: int,
+                                   shared: TileWeights, gate: torch.Tensor, norm: bool = True):
+    """:func:`gate_up_silu_tiles_topk` with the shared expert's SwiGLU in the
+    same launch, as slot ``top_k`` of every token: (h [T, k + 1, I], idx and
+    scores [T, k + 1]), the last score sigmoid(x . gate).  For
+    :func:`down_wsum_tiles_shared`."""
+    if not tw.swiglu_pairs or not shared.swiglu_pairs:
+        raise ValueError("the decode SwiGLU kernel needs weights repacked with swiglu_pairs=True")
+    x, gate = _bf16(x, "x"), _bf16(gate, "gate")
+    T, K = x.shape
+    if (shared.num_experts, shared.N, shared.K) != (1, tw.N, tw.K) or K != tw.K or gate.numel() != K:
+        raise ValueError("x, the shared expert and its gate must have the routed experts' shape")
+    lg = _logits(logits, T, tw.num_experts, x.device)
+    I = tw.N // 2
+    h = torch.empty(T, top_k + 1, I, dtype=torch.bfloat16, device=x.device)
+    idx = torch.empty(T, top_k + 1, dtype=torch.int32, device=x.device)
+    scores = torch.empty(T, top_k + 1, dtype=torch.float32, device=x.device)
+    _lib.call("qmoe_moe_gate_up_swiglu_tiles_topk_shared", x.data_ptr(), lg.data_ptr(), int(bool(norm)), T, top_k, K,
+              tw.wp.data_ptr(), tw.sb.data_ptr(), tw.num_experts, I, shared.wp.data_ptr(), shared.sb.data_ptr(),
+              gate.data_ptr(), h.data_ptr(), idx.data_ptr(), scores.data_ptr(), _stream(x))
+    return h, idx, scores
+
+
+def down_wsum_tiles_shared(h: torch.Tensor, tw: TileWeights, idx: torch.Tensor, scores: torch.Tensor,
+                           shared: TileWeights) -> torch.Tensor:
+    """:func:`down_wsum_tiles` whose last slot per token is the shared expert's."""
+    if tw.swiglu_pairs or shared.swiglu_pairs:
+        raise ValueError("down weights are repacked in their own row order (swiglu_pairs=False)")
+    h = _bf16(h, "h")
+    T, slots, I = h.shape
+    if (shared.num_experts, shared.N, shared.K) != (1, tw.N, tw.K) or I != tw.K:
+        raise ValueError("h and the shared expert must have the routed experts' shape")
+    idx = _i32(idx, "idx", h.device)
+    sc = _f32(scores, "scores", h.device)
+    y = torch.empty(T, tw.N, dtype=torch.bfloat16, device=h.device)
+    _lib.call("qmoe_moe_down_wsum_tiles_shared", h.data_ptr(), idx.data_ptr(), sc.data_ptr(), T, slots, I,
+              tw.wp.data_ptr(), tw.sb.data_ptr(), tw.num_experts, tw.N, shared.wp.data_ptr(), shared.sb.data_ptr(),
+              y.data_ptr(), _stream(h))
+    return y
+
+
 def gemm_supported(K: int, N: int, group_size: int, bits: int) -> bool:
     return bits == 4 and group_size == 64 and K % 128 == 0 and N % 256 == 0
 
@@ -686,7 +727,7 @@ def router_logits(x: torch.Tensor, router, group_size: int = GROUP, bits: int = 
 __all__ = [
     "GROUP", "BITS", "QmoeError", "QmoeUnsupported", "TileTable", "TileWeights", "Routing", "build_tiles", "route",
     "repack_tiles", "gather_qmm_sorted_tiles", "gather_qmm_int8_sorted_tiles", "router_topk", "router_logits", "gather_qmm_swiglu_sorted_tiles", "swiglu_pair_order", "gather_qmv_tiles", "gate_up_silu_tiles",
-    "down_wsum_tiles", "gate_up_silu_tiles_topk",
+    "down_wsum_tiles", "gate_up_silu_tiles_topk", "gate_up_silu_tiles_topk_shared", "down_wsum_tiles_shared",
     "max_tiles", "tile_rows", "unpack", "dequantize", "gather_qmv", "gather_qmm_sorted", "gather_qmm",
     "gemm_supported", "quantized_matmul", "gate_up_silu", "down_wsum", "moe_weighted_sum",
     "quantize_act_int8", "gather_qmm_int8_sorted",
