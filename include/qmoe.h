@@ -86,6 +86,22 @@ int qmoe_route(const int32_t* ids, int64_t n_pairs, int32_t num_experts,
                int32_t* tile_exp, int32_t* ntiles, int64_t max_tiles,
                void* workspace, size_t workspace_bytes, void* stream);
 
+/* The routing step of a whole MoE block over ids [T, top_k] (n_pairs = T *
+ * top_k): qmoe_route's sort and tables with x_rows [n_pairs + shared_rows] in
+ * the place of order and sorted_ids -- x_rows[i] = the token of sorted row i,
+ * pair / top_k, what the gate_up GEMM gathers by.  With shared_rows > 0 a
+ * shared expert is expert num_experts of the tables, with rows n_pairs ..
+ * n_pairs + shared_rows - 1 (x_rows[n_pairs + t] = t): offsets then holds
+ * num_experts + 2 entries, and max_tiles >= ceil(n_pairs/tile_rows) +
+ * num_experts + ceil(shared_rows/tile_rows) suffices.  num_experts <= 2048;
+ * workspace as for qmoe_route. */
+int qmoe_route_block(const int32_t* ids, int64_t n_pairs, int32_t top_k,
+                     int32_t num_experts, int32_t shared_rows,
+                     int32_t tile_rows, int32_t* x_rows, int32_t* inv_order,
+                     int32_t* offsets, int32_t* tile_row, int32_t* tile_exp,
+                     int32_t* ntiles, int64_t max_tiles, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
 /* qmoe_route without a caller workspace.  No counterpart in the reference:
  * this is for callers that cannot allocate device memory (code under HIP
  * graph capture, serving loops or harnesses that forbid hipMalloc).  The
@@ -352,6 +368,25 @@ int qmoe_gather_qmm_swiglu_sorted_tiles(const uint16_t* x, const int32_t* x_rows
                                         const int32_t* ntiles, int64_t max_tiles,
                                         uint16_t* h, void* stream);
 
+/* qmoe_gather_qmm_sorted_tiles, or with swiglu != 0
+ * qmoe_gather_qmm_swiglu_sorted_tiles, over a tile table of num_experts + 1
+ * experts (qmoe_route_block with shared rows) whose last one is the tensor
+ * (sh_wp, sh_sb), one expert of the same N and K. */
+int qmoe_gather_qmm_sorted_tiles_shared(
+    const uint16_t* x, const int32_t* x_rows, int64_t n_rows, int64_t K,
+    const uint32_t* wp, const uint32_t* sb, const uint32_t* sh_wp,
+    const uint32_t* sh_sb, int32_t num_experts, int64_t N, int swiglu,
+    const int32_t* offsets, const int32_t* tile_row, const int32_t* tile_exp,
+    const int32_t* ntiles, int64_t max_tiles, uint16_t* out, void* stream);
+
+/* qmoe_weighted_sum with one more row per output row: scores [rows, top_k + 1],
+ * and scores[r, top_k] * shared[r, :] is added in fp32 (in the ops and clone
+ * modes to the rounded sum of the top_k slots), one bf16 rounding after it. */
+int qmoe_weighted_sum_shared(const uint16_t* xs, const int32_t* inv_order,
+                             const float* scores, int64_t rows, int64_t top_k,
+                             int64_t dim, int mode, const uint16_t* shared,
+                             uint16_t* out, void* stream);
+
 /* ---------------------------------------------------------------- router --
  * Top-k experts per token from fp32 router logits [T, E] (replaces the
  * reference's fused router_topk, engine/patches/decode-fusion/
@@ -363,6 +398,14 @@ int qmoe_gather_qmm_swiglu_sorted_tiles(const uint16_t* x, const int32_t* x_rows
  * NaN ranks below every number, after which ties go to the lower index). */
 int qmoe_router_topk(const float* logits, int64_t T, int64_t E, int64_t k,
                      int norm, int32_t* idx, float* scores, void* stream);
+
+/* qmoe_router_topk with scores [T, k + 1], scores[t, k] = sigmoid(x[t] . gate)
+ * in fp32: the shared expert's weight (qwen3_5_moe/language.py:81-89).  x [T, K]
+ * and gate [K] bf16, K % 8 == 0. */
+int qmoe_router_topk_shared(const float* logits, int64_t T, int64_t E,
+                            int64_t k, int norm, const uint16_t* x,
+                            const uint16_t* gate, int64_t K, int32_t* idx,
+                            float* scores, void* stream);
 
 /* Router logits in fp32 from an affine-quantized router weight [E, K*bits/32]
  * (replaces the fused router's quantized matvec,

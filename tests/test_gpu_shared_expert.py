@@ -1,5 +1,6 @@
 """The shared expert as one more slot of the decode kernels
-(qmoe_moe_gate_up_swiglu_tiles_topk_shared, qmoe_moe_down_wsum_tiles_shared)
+(qmoe_moe_gate_up_swiglu_tiles_topk_shared, qmoe_moe_down_wsum_tiles_shared) and
+one more expert of the sorted path (qmoe_route_block and the *_shared entry points)
 against the id-taking kernels and a 64-bit product."""
 
 import pytest
@@ -67,7 +68,7 @@ def test_shared_slot_decode(dev, T, k, H, E, norm):
     _close_bf16(y, ref)
 
 
-@pytest.mark.parametrize("T", [1, 6, 7, 16])
+@pytest.mark.parametrize("T", [1, 6, 7, 16, 17, 200])
 @pytest.mark.parametrize("k,S", [(10, 512), (16, 512), (10, 768)])
 def test_block_with_shared_expert_matches_its_parts(dev, T, k, S):
     """The block over every dispatch of its shared expert (a slot of the
@@ -93,3 +94,89 @@ def test_block_with_shared_expert_matches_its_parts(dev, T, k, S):
     # the routed part's bf16 rounding, h's, and the sum's: 3 * 2^-9 of the
     # parts' magnitudes, the block's own bar of 2^-7 of max|y|
     assert bool(((y.double() - ref).abs() <= 2.0 ** -7 * ref.abs().max()).all())
+
+
+@pytest.mark.parametrize("T,k,E", [(1, 1, 1), (7, 10, 256), (64, 64, 100), (409, 10, 512), (410, 10, 256),
+                                   (129, 3, 2048), (5, 4, 513), (3000, 10, 64)])
+def test_route_block_matches_route(dev, T, k, E):
+    """The block's routing on every path and edge of qmoe_route (one block,
+    count and scatter, an expert count of its limit), with and without the
+    shared expert's rows, against the plain tables."""
+    print(f"[case] route_block T={T} k={k} E={E}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T + k + E)
+    idx = torch.randint(-1, E + 1, (T, k), dtype=torch.int32, device=dev, generator=g)  # a few out of range
+    r = ops.route(idx, E)
+    n, nt = T * k, int(r.tiles.ntiles)
+    for shared in (False, True):
+        x_rows, inv, t = ops.route_block(idx, E, shared)
+        assert torch.equal(x_rows[:n], r.order // k) and torch.equal(inv[:n], r.inv_order)
+        assert torch.equal(t.offsets[:E + 1], r.tiles.offsets)
+        m = int(t.ntiles)
+        assert torch.equal(t.tile_row[:nt], r.tiles.tile_row[:nt]) and torch.equal(t.tile_exp[:nt], r.tiles.tile_exp[:nt])
+        if shared:
+            rows = torch.arange(0, T, 128, dtype=torch.int32, device=dev)
+            assert m == nt + rows.numel() and int(t.offsets[E + 1]) == n + T and t.rows == n + T
+            assert torch.equal(t.tile_row[nt:m], n + rows) and bool((t.tile_exp[nt:m] == E).all())
+            assert torch.equal(x_rows[n:n + T], torch.arange(T, dtype=torch.int32, device=dev))
+        else:
+            assert m == nt and t.rows == n
+
+
+@pytest.mark.parametrize("T,E", [(17, 4), (128, 3), (129, 3), (300, 40)])
+def test_gemm_with_shared_expert_is_the_two_gemms(dev, T, E):
+    """Both epilogues over a table whose last expert is a tensor of its own:
+    bit for bit the routed GEMM and the shared expert's own."""
+    print(f"[case] GEMM with shared rows T={T} E={E}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T + E)
+    k, H, I = 2, 512, 256
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    idx = torch.randint(0, E, (T, k), dtype=torch.int32, device=dev, generator=g)
+    x_rows, _, ts = ops.route_block(idx, E, shared=True)
+    _, _, t0 = ops.route_block(idx, E)
+    one = ops.build_tiles(torch.zeros(T, dtype=torch.int32, device=dev), 1)
+    for pairs in (True, False):
+        w, sw = _quant(g, (E, 2 * I), H, dev), _quant(g, (1, 2 * I), H, dev)
+        tw, stw = ops.repack_tiles(*w, swiglu_pairs=pairs), ops.repack_tiles(*sw, swiglu_pairs=pairs)
+        gemm = ops.gather_qmm_swiglu_sorted_tiles if pairs else ops.gather_qmm_sorted_tiles
+        y = ops.gather_qmm_sorted_tiles_shared(x, tw, stw, ts, x_rows=x_rows)
+        assert torch.equal(y[:T * k], gemm(x, tw, t0, x_rows=x_rows))
+        assert torch.equal(y[T * k:], gemm(x, stw, one))
+
+
+@pytest.mark.parametrize("mode", ["fast", "ops", "clone"])
+@pytest.mark.parametrize("T,k,D", [(1, 1, 8), (3, 8, 2056), (70, 10, 2048), (5, 17, 512)])
+def test_weighted_sum_with_shared_row(dev, mode, T, k, D):
+    print(f"[case] weighted sum with shared row T={T} k={k} D={D} {mode}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T + k)
+    xs = torch.randn(T * k, D, device=dev, generator=g).to(torch.bfloat16)
+    sh = torch.randn(T, D, device=dev, generator=g).to(torch.bfloat16)
+    sc = torch.rand(T, k + 1, device=dev, generator=g)
+    inv = torch.randperm(T * k, device=dev, generator=g).to(torch.int32)
+    y = ops.moe_weighted_sum_shared(xs, inv, sc, sh, mode)
+    if mode == "fast":
+        ref = (xs.double()[inv.long()].reshape(T, k, D) * sc[:, :k, None].double()).sum(1)
+        mag = (xs.double().abs()[inv.long()].reshape(T, k, D) * sc[:, :k, None].double()).sum(1)
+    else:  # the k-slot sum as that mode rounds it
+        ref = ops.moe_weighted_sum(xs, inv, sc[:, :k].contiguous(), (T, D), mode).double()
+        mag = ref.abs()
+    last = sc[:, k:].double() * sh.double()
+    err = (y.double() - (ref + last)).abs()
+    # one bf16 rounding, and k + 2 roundings of the sums in fp32
+    assert bool((err <= 2.0 ** -8 * (ref + last).abs() + (k + 2) * 2.0 ** -24 * (mag + last.abs())).all())
+
+
+@pytest.mark.parametrize("T,E,K", [(1, 8, 8), (5, 100, 2048), (300, 256, 2056), (9, 1000, 520)])
+def test_topk_with_shared_score(dev, T, E, K):
+    print(f"[case] top-k with shared score T={T} E={E} K={K}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T + E)
+    lg = torch.randn(T, E, device=dev, generator=g)
+    x = torch.randn(T, K, device=dev, generator=g).to(torch.bfloat16)
+    gate = (torch.randn(1, K, device=dev, generator=g) * K ** -0.5).to(torch.bfloat16)
+    k = min(E, 10)
+    for norm in (True, False):
+        idx, sc = ops.router_topk_shared(lg, k, x, gate, norm)
+        idx0, sc0 = ops.router_topk(lg, k, norm)
+        assert torch.equal(idx, idx0) and torch.equal(sc[:, :k], sc0)
+        z = x.double() @ gate.double().t()
+        bound = 0.25 * K * 2.0 ** -24 * (x.double().abs() @ gate.double().abs().t()) + 4 * 2.0 ** -24
+        assert bool(((sc[:, k:].double() - torch.sigmoid(z)).abs() <= bound).all())

@@ -70,6 +70,10 @@ SIGNATURES: dict[str, tuple] = {
     "qmoe_moe_gate_up_swiglu_tiles_topk": (INT, [P, P, INT, I64, I64, I64, P, P, I32, I64, P, P, P, P]),
     "qmoe_moe_gate_up_swiglu_tiles_topk_shared": (INT, [P, P, INT, I64, I64, I64, P, P, I32, I64, P, P, P, P, P, P, P]),
     "qmoe_moe_down_wsum_tiles_shared": (INT, [P, P, P, I64, I64, I64, P, P, I32, I64, P, P, P, P]),
+    "qmoe_route_block": (INT, [P, I64, I32, I32, I32, I32, P, P, P, P, P, P, I64, P, SZ, P]),
+    "qmoe_gather_qmm_sorted_tiles_shared": (INT, [P, P, I64, I64, P, P, P, P, I32, I64, INT, P, P, P, P, I64, P, P]),
+    "qmoe_weighted_sum_shared": (INT, [P, P, P, I64, I64, I64, INT, P, P, P]),
+    "qmoe_router_topk_shared": (INT, [P, I64, I64, I64, INT, P, P, I64, P, P, P]),
     "qmoe_quantize_act_int8": (INT, [P, I64, I64, P, P, P]),
     "qmoe_gather_qmm_int8_sorted": (INT, [P, P, P, I64, I64, P, P, P, I32, I64, INT, INT, P, P, P, P,
                                           I64, P, P]),

@@ -134,6 +134,10 @@ struct GemmArgs {
   const int32_t* tile_exp;
   const int32_t* ntiles;
   uint16_t* out;
+  // tile layout: the weights of the last expert, num_experts - 1, when they
+  // are a tensor of their own (the block's shared expert); null: in w and sb
+  const uint32_t* last_w = nullptr;
+  const uint32_t* last_sb = nullptr;
 };
 
 // fma(h, s, b) in fp32 with h the fp16 in the low (HI = false) or high half
@@ -530,10 +534,11 @@ __device__ __forceinline__ void run_unit(const GemmArgs& a, char* smem, int tile
   }
   if constexpr (TILED) {
     // chunk (e, c, g) of the tile layout, c = the wave's 64-column block
-    const int64_t chunk0 = ((int64_t)e * (a.N / 64) + nblk * kWaves + c.wave) * G;
-    c.b_base = reinterpret_cast<const char*>(a.w) + uniform64(chunk0 * 2048);
+    const bool last = a.last_w && e == a.num_experts - 1;  // block-uniform
+    const int64_t chunk0 = ((int64_t)(last ? 0 : e) * (a.N / 64) + nblk * kWaves + c.wave) * G;
+    c.b_base = reinterpret_cast<const char*>(last ? a.last_w : a.w) + uniform64(chunk0 * 2048);
     c.b_off[0] = c.b_off[1] = (uint32_t)c.lane * 16;
-    c.s_base = reinterpret_cast<const char*>(a.sb) + uniform64(chunk0 * 256);
+    c.s_base = reinterpret_cast<const char*>(last ? a.last_sb : a.sb) + uniform64(chunk0 * 256);
     c.s_off = (uint32_t)c.lane * 4;
     c.z_base = nullptr;
   } else {
@@ -681,20 +686,34 @@ extern "C" int qmoe_gather_qmm_sorted(const uint16_t* x, const int32_t* x_rows, 
   return launch_gemm(a, max_tiles, false, stream);
 }
 
+namespace {
+
+// The tile-layout GEMM, plain or with the SwiGLU epilogue; with last_wp the
+// table's last expert is that tensor and num_experts counts it.
+int gemm_tiles(const uint16_t* x, const int32_t* x_rows, int64_t n_rows, int64_t K, const uint32_t* wp,
+               const uint32_t* sb, const uint32_t* last_wp, const uint32_t* last_sb, int32_t num_experts, int64_t N,
+               const int32_t* offsets, const int32_t* tile_row, const int32_t* tile_exp, const int32_t* ntiles,
+               int64_t max_tiles, uint16_t* out, void* stream, bool swiglu) {
+  const int rc = check_common(x, n_rows, K, num_experts, N, offsets, tile_row, tile_exp, ntiles, max_tiles, out);
+  if (rc != QMOE_OK || n_rows == 0 || max_tiles == 0) return rc;
+  if (!wp || !sb) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+  if (K % 64) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "K=%lld: must be a multiple of 64", (long long)K);
+  if (!qmoe::aligned16(wp) || !qmoe::aligned16(sb) || !qmoe::aligned16(last_wp) || !qmoe::aligned16(last_sb))
+    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "wp and sb must be 16-byte aligned");
+  GemmArgs a{x, x_rows, n_rows, (int)K, wp, nullptr, nullptr, sb, num_experts, (int)N, offsets, tile_row,
+             tile_exp, ntiles, out, last_wp, last_sb};
+  return launch_gemm(a, max_tiles, true, stream, swiglu);
+}
+
+}  // namespace
+
 extern "C" int qmoe_gather_qmm_sorted_tiles(const uint16_t* x, const int32_t* x_rows, int64_t n_rows, int64_t K,
                                             const uint32_t* wp, const uint32_t* sb, int32_t num_experts,
                                             int64_t N, const int32_t* offsets, const int32_t* tile_row,
                                             const int32_t* tile_exp, const int32_t* ntiles, int64_t max_tiles,
                                             uint16_t* out, void* stream) {
-  const int rc = check_common(x, n_rows, K, num_experts, N, offsets, tile_row, tile_exp, ntiles, max_tiles, out);
-  if (rc != QMOE_OK || n_rows == 0 || max_tiles == 0) return rc;
-  if (!wp || !sb) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
-  if (K % 64) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "K=%lld: must be a multiple of 64", (long long)K);
-  if (!qmoe::aligned16(wp) || !qmoe::aligned16(sb))
-    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "wp and sb must be 16-byte aligned");
-  GemmArgs a{x, x_rows, n_rows, (int)K, wp, nullptr, nullptr, sb, num_experts, (int)N, offsets, tile_row,
-             tile_exp, ntiles, out};
-  return launch_gemm(a, max_tiles, true, stream);
+  return gemm_tiles(x, x_rows, n_rows, K, wp, sb, nullptr, nullptr, num_experts, N, offsets, tile_row, tile_exp,
+                    ntiles, max_tiles, out, stream, false);
 }
 
 extern "C" int qmoe_gather_qmm_swiglu_sorted_tiles(const uint16_t* x, const int32_t* x_rows, int64_t n_rows,
@@ -703,15 +722,21 @@ extern "C" int qmoe_gather_qmm_swiglu_sorted_tiles(const uint16_t* x, const int3
                                                    const int32_t* tile_row, const int32_t* tile_exp,
                                                    const int32_t* ntiles, int64_t max_tiles, uint16_t* h,
                                                    void* stream) {
-  const int rc = check_common(x, n_rows, K, num_experts, N, offsets, tile_row, tile_exp, ntiles, max_tiles, h);
-  if (rc != QMOE_OK || n_rows == 0 || max_tiles == 0) return rc;
-  if (!wp || !sb) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
-  if (K % 64) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "K=%lld: must be a multiple of 64", (long long)K);
-  if (!qmoe::aligned16(wp) || !qmoe::aligned16(sb))
-    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "wp and sb must be 16-byte aligned");
-  GemmArgs a{x, x_rows, n_rows, (int)K, wp, nullptr, nullptr, sb, num_experts, (int)N, offsets, tile_row,
-             tile_exp, ntiles, h};
-  return launch_gemm(a, max_tiles, true, stream, true);
+  return gemm_tiles(x, x_rows, n_rows, K, wp, sb, nullptr, nullptr, num_experts, N, offsets, tile_row, tile_exp,
+                    ntiles, max_tiles, h, stream, true);
+}
+
+extern "C" int qmoe_gather_qmm_sorted_tiles_shared(const uint16_t* x, const int32_t* x_rows, int64_t n_rows,
+                                                   int64_t K, const uint32_t* wp, const uint32_t* sb,
+                                                   const uint32_t* sh_wp, const uint32_t* sh_sb, int32_t num_experts,
+                                                   int64_t N, int swiglu, const int32_t* offsets,
+                                                   const int32_t* tile_row, const int32_t* tile_exp,
+                                                   const int32_t* ntiles, int64_t max_tiles, uint16_t* out,
+                                                   void* stream) {
+  if (!sh_wp || !sh_sb) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+  if (num_experts <= 0 || num_experts == INT32_MAX) return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
+  return gemm_tiles(x, x_rows, n_rows, K, wp, sb, sh_wp, sh_sb, num_experts + 1, N, offsets, tile_row, tile_exp,
+                    ntiles, max_tiles, out, stream, swiglu != 0);
 }
 
 namespace qmoe_gemm {

@@ -29,6 +29,20 @@ constexpr int kChunk = 1024;    // rows per histogram chunk
 constexpr int kCountThreads = 256;
 constexpr int kScanThreads = 1024;
 
+// What the MoE block's routing writes besides the tables (all off by default):
+// x_rows[sorted position] = the pair's token, pair / top_k, which the gate_up
+// GEMM gathers by, so that no launch computes it from `order`; and a shared
+// expert as expert E of `rows` more rows, one per token, after the n sorted
+// pairs: offsets[E + 1] = n + rows, its tiles last, x_rows[n + t] = t.  order
+// and sorted_ids may then be null.  With both, the sorted block with a shared
+// expert went from 20 launches to 7 (256 experts, top-10, hidden 2048): 16
+// tokens 115.8 -> 93.6 us, 96 tokens 199 -> 130 us, 4096 tokens 512 -> 408 us.
+struct BlockRows {
+  int32_t* x_rows = nullptr;
+  uint32_t top_k = 1;
+  int rows = 0;
+};
+
 __device__ __forceinline__ int clamp_id(int id, int E) { return id < 0 ? 0 : (id >= E ? E - 1 : id); }
 
 // ids[i], read from an index clamped into [0, n) (n > 0) so that the read is
@@ -304,14 +318,14 @@ __global__ __launch_bounds__(64 * kScanScatterWaves) void route_scan_scatter_ker
     const int32_t* __restrict__ ids, int64_t n, int E, int nbits, int nchunks, const int32_t* __restrict__ counts,
     int tile_rows, int32_t* __restrict__ order, int32_t* __restrict__ inv_order, int32_t* __restrict__ sorted_ids,
     int32_t* __restrict__ offsets, int32_t* __restrict__ tile_row, int32_t* __restrict__ tile_exp,
-    int32_t* __restrict__ ntiles, int64_t max_tiles, int32_t* __restrict__ bad) {
+    int32_t* __restrict__ ntiles, int64_t max_tiles, int32_t* __restrict__ bad, BlockRows br) {
   constexpr int W = kScanScatterWaves;
   constexpr int T = 64 * W;
   constexpr int kSteps = kChunk / 64 / W;
   extern __shared__ int sm[];
   int* run = sm;             // [W][E]: per-wave counts, then first slots
   int* base = sm + W * E;    // [E]: the chunk's first slot per expert
-  int* off = base + E;       // [E + 1]: the experts' offsets
+  int* off = base + E;       // [E + 2]: the experts' offsets (and the shared expert's end)
   __shared__ int lds[T / 64 + 1];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int c = blockIdx.x;
@@ -375,14 +389,20 @@ __global__ __launch_bounds__(64 * kScanScatterWaves) void route_scan_scatter_ker
       off[e] = r;
       r += t;
     }
-    if (tid == 0) off[E] = (int)n;
+    if (tid == 0) {
+      off[E] = (int)n;
+      off[E + 1] = (int)n + br.rows;
+    }
   }
   __syncthreads();
   for (int e = tid; e < E; e += T) base[e] += off[e];
   if (c == 0) {  // block-uniform
-    for (int e = tid; e <= E; e += T) offsets[e] = off[e];
-    emit_tiles<T>(off, E, tile_rows, tile_row, tile_exp, ntiles, max_tiles, lds);
+    const int Et = E + (br.rows > 0 ? 1 : 0);
+    for (int e = tid; e <= Et; e += T) offsets[e] = off[e];
+    emit_tiles<T>(off, Et, tile_rows, tile_row, tile_exp, ntiles, max_tiles, lds);
   }
+  if (br.x_rows)
+    for (int i = c * T + tid; i < br.rows; i += gridDim.x * T) br.x_rows[n + i] = i;
   uint64_t mv[kSteps];
 #pragma unroll
   for (int step = 0; step < kSteps; ++step) {
@@ -419,8 +439,9 @@ __global__ __launch_bounds__(64 * kScanScatterWaves) void route_scan_scatter_ker
     const int rank = __popcll(m & lt);
     if (valid) {
       const int dst = my[id] + rank;
-      order[dst] = (int32_t)i;
-      sorted_ids[dst] = id;
+      if (order) order[dst] = (int32_t)i;
+      if (sorted_ids) sorted_ids[dst] = id;
+      if (br.x_rows) br.x_rows[dst] = (int32_t)((uint32_t)i / br.top_k);
       inv_order[i] = dst;
     }
     __builtin_amdgcn_wave_barrier();  // every lane has read my[id] before the leader moves it
@@ -470,10 +491,10 @@ __global__ __launch_bounds__(kScanThreads) void route_fused_kernel(
     const int32_t* __restrict__ ids, int64_t n, int E, int nbits, int tile_rows, int32_t* __restrict__ order,
     int32_t* __restrict__ inv_order, int32_t* __restrict__ sorted_ids, int32_t* __restrict__ offsets,
     int32_t* __restrict__ tile_row, int32_t* __restrict__ tile_exp, int32_t* __restrict__ ntiles,
-    int64_t max_tiles, int32_t* __restrict__ bad) {
+    int64_t max_tiles, int32_t* __restrict__ bad, BlockRows br) {
   extern __shared__ int sm[];
   int* hist = sm;                          // [kFusedWaves][E + 1]; slot E counts out-of-range ids
-  int* off = sm + kFusedWaves * (E + 1);   // [E + 1]
+  int* off = sm + kFusedWaves * (E + 1);   // [E + 2]
   __shared__ int lds[kScanThreads];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int64_t seg = (n + kFusedWaves - 1) / kFusedWaves;
@@ -522,7 +543,11 @@ __global__ __launch_bounds__(kScanThreads) void route_fused_kernel(
   if (tid == 0) {
     off[E] = (int)n;
     offsets[E] = (int32_t)n;
+    off[E + 1] = (int)n + br.rows;
+    if (br.rows > 0) offsets[E + 1] = (int32_t)(n + br.rows);
   }
+  if (br.x_rows)
+    for (int i = tid; i < br.rows; i += kScanThreads) br.x_rows[n + i] = i;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
   for (int q = 0; q < kFusedSteps; ++q) {
@@ -540,8 +565,9 @@ __global__ __launch_bounds__(kScanThreads) void route_fused_kernel(
     const int rank = __popcll(m & lt);
     if (valid) {
       const int dst = my[id] + rank;
-      order[dst] = (int32_t)i;
-      sorted_ids[dst] = id;
+      if (order) order[dst] = (int32_t)i;
+      if (sorted_ids) sorted_ids[dst] = id;
+      if (br.x_rows) br.x_rows[dst] = (int32_t)((uint32_t)i / br.top_k);
       inv_order[i] = dst;
     }
     __builtin_amdgcn_wave_barrier();  // every lane has read my[id] before the leader moves it
@@ -549,7 +575,7 @@ __global__ __launch_bounds__(kScanThreads) void route_fused_kernel(
     __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
-  emit_tiles(off, E, tile_rows, tile_row, tile_exp, ntiles, max_tiles, lds);
+  emit_tiles(off, E + (br.rows > 0 ? 1 : 0), tile_rows, tile_row, tile_exp, ntiles, max_tiles, lds);
 }
 
 int64_t n_chunks(int64_t n) { return (n + kChunk - 1) / kChunk; }
@@ -558,7 +584,8 @@ int64_t n_chunks(int64_t n) { return (n + kChunk - 1) / kChunk; }
 // (word 0 unused when `bad` points elsewhere, then (E + 1) * chunks counts).
 int route_launch(const int32_t* ids, int64_t n_pairs, int32_t num_experts, int32_t tile_rows, int32_t* order,
                  int32_t* inv_order, int32_t* sorted_ids, int32_t* offsets, int32_t* tile_row, int32_t* tile_exp,
-                 int32_t* ntiles, int64_t max_tiles, int32_t* ws, int32_t* bad, hipStream_t st);
+                 int32_t* ntiles, int64_t max_tiles, int32_t* ws, int32_t* bad, hipStream_t st,
+                 BlockRows br = {});
 
 }  // namespace
 
@@ -591,16 +618,16 @@ namespace {
 
 int route_launch(const int32_t* ids, int64_t n_pairs, int32_t num_experts, int32_t tile_rows, int32_t* order,
                  int32_t* inv_order, int32_t* sorted_ids, int32_t* offsets, int32_t* tile_row, int32_t* tile_exp,
-                 int32_t* ntiles, int64_t max_tiles, int32_t* ws, int32_t* bad, hipStream_t st) {
+                 int32_t* ntiles, int64_t max_tiles, int32_t* ws, int32_t* bad, hipStream_t st, BlockRows br) {
   const int64_t nch = n_chunks(n_pairs);
   int32_t* counts = ws + 64;
   if (n_pairs <= kFusedMaxN && num_experts <= kFusedMaxE) {
     int nbits = 1;
     while ((1 << nbits) <= num_experts) ++nbits;  // ids in [0, E] (E is the sentinel)
-    const size_t shm = (size_t)(kFusedWaves + 1) * (num_experts + 1) * sizeof(int);
+    const size_t shm = ((size_t)(kFusedWaves + 1) * (num_experts + 1) + 1) * sizeof(int);
     route_fused_kernel<<<dim3(1), dim3(kScanThreads), shm, st>>>(ids, n_pairs, num_experts, nbits, tile_rows,
                                                                 order, inv_order, sorted_ids, offsets, tile_row,
-                                                                tile_exp, ntiles, max_tiles, bad);
+                                                                tile_exp, ntiles, max_tiles, bad, br);
     return qmoe::launch_status("route_fused_kernel");
   }
   int nbits = 1;
@@ -613,12 +640,12 @@ int route_launch(const int32_t* ids, int64_t n_pairs, int32_t num_experts, int32
     if (rc) return rc;
   }
   if (scan_in_scatter) {
-    // (W + 2) * E + 1 ints of LDS; one block even without rows (it writes
+    // (W + 2) * E + 2 ints of LDS; one block even without rows (it writes
     // the zero offsets and the empty tile list)
-    const size_t shm = ((size_t)(kScanScatterWaves + 2) * num_experts + 1) * sizeof(int);
+    const size_t shm = ((size_t)(kScanScatterWaves + 2) * num_experts + 2) * sizeof(int);
     route_scan_scatter_kernel<<<dim3((unsigned)(nch > 0 ? nch : 1)), dim3(64 * kScanScatterWaves), shm, st>>>(
         ids, n_pairs, num_experts, nbits, (int)nch, counts, tile_rows, order, inv_order, sorted_ids, offsets,
-        tile_row, tile_exp, ntiles, max_tiles, bad);
+        tile_row, tile_exp, ntiles, max_tiles, bad, br);
     return qmoe::launch_status("route_scan_scatter_kernel");
   }
   route_scan_kernel<<<dim3(1), dim3(kScanThreads), 0, st>>>(counts, n_pairs, num_experts, (int)nch, tile_rows,
@@ -631,6 +658,26 @@ int route_launch(const int32_t* ids, int64_t n_pairs, int32_t num_experts, int32
 }
 
 }  // namespace
+
+extern "C" int qmoe_route_block(const int32_t* ids, int64_t n_pairs, int32_t top_k, int32_t num_experts,
+                                int32_t shared_rows, int32_t tile_rows, int32_t* x_rows, int32_t* inv_order,
+                                int32_t* offsets, int32_t* tile_row, int32_t* tile_exp, int32_t* ntiles,
+                                int64_t max_tiles, void* workspace, size_t workspace_bytes, void* stream) {
+  if (n_pairs <= 0 || top_k <= 0 || num_experts <= 0 || shared_rows < 0 || tile_rows <= 0 || max_tiles <= 0)
+    return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
+  if (num_experts > kScanScatterMaxE)
+    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "num_experts=%d > %d", num_experts, kScanScatterMaxE);
+  if (n_pairs + shared_rows > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "too many pairs");
+  if (!ids || !x_rows || !inv_order || !offsets || !tile_row || !tile_exp || !ntiles)
+    return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+  const size_t need = qmoe_route_workspace_size(n_pairs, num_experts);
+  if (!workspace || workspace_bytes < need)
+    return qmoe::fail(QMOE_ERR_WORKSPACE, "route needs %zu workspace bytes", need);
+  int32_t* ws = static_cast<int32_t*>(workspace);
+  return route_launch(ids, n_pairs, num_experts, tile_rows, nullptr, inv_order, nullptr, offsets, tile_row, tile_exp,
+                      ntiles, max_tiles, ws, ws, qmoe::as_stream(stream),
+                      BlockRows{x_rows, (uint32_t)top_k, shared_rows});
+}
 
 extern "C" int qmoe_build_tiles(const int32_t* sorted_ids, int64_t n_rows, int32_t num_experts,
                                 int32_t tile_rows, int32_t* offsets, int32_t* tile_row, int32_t* tile_exp,

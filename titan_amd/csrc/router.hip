@@ -14,20 +14,74 @@ using qmoe_topk::kMaxK;
 using qmoe_topk::kMaxPer;
 using qmoe_topk::wave_sum;
 
-template <int PER>
+// SH: the token's row of scores has one more entry, the shared expert's
+// sigmoid(x[t] . gate) in fp32 (language.py:81-89).  The wave's share of the
+// product, K / 64 columns a lane, comes first: 5.9 against 4.5 us at 16 tokens
+// and 10.0 against 6.4 us at 4096 (16.8 MB of x), where a launch of its own
+// for the logits took 4.1 and 4.9 us and each of the eight passes that gated
+// and added the shared expert's rows 4 to 16 us more.
+template <int PER, bool SH>
 __global__ __launch_bounds__(256) void router_topk_kernel(const float* __restrict__ logits, int64_t T, int E, int k,
                                                          int norm, int32_t* __restrict__ idx,
-                                                         float* __restrict__ scores) {
+                                                         float* __restrict__ scores, const uint16_t* __restrict__ x,
+                                                         const uint16_t* __restrict__ gate, int K) {
   const int64_t t = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
   if (t >= T) return;
+  float z[4] = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (SH) {
+    const uint4* xp = reinterpret_cast<const uint4*>(x + t * K);
+    const uint4* gp = reinterpret_cast<const uint4*>(gate);
+    for (int u = lane; u < K / 8; u += 64) {
+      const uint4 xv = xp[u], gv = gp[u];
+      z[0] = dot2_bf16(xv.x, gv.x, z[0]);
+      z[1] = dot2_bf16(xv.y, gv.y, z[1]);
+      z[2] = dot2_bf16(xv.z, gv.z, z[2]);
+      z[3] = dot2_bf16(xv.w, gv.w, z[3]);
+    }
+  }
   int sel;
   float sc;
   qmoe_topk::wave_topk<PER>(logits + t * E, E, k, norm, sel, sc);
+  const int ss = SH ? k + 1 : k;
   if (lane < k) {
     idx[t * k + lane] = sel;
-    scores[t * k + lane] = sc;
+    scores[t * ss + lane] = sc;
   }
+  if constexpr (SH) {
+    const float zs = wave_sum((z[0] + z[1]) + (z[2] + z[3]));
+    if (lane == 0) scores[t * ss + k] = 1.0f / (1.0f + expf(-zs));
+  }
+}
+
+template <bool SH>
+int launch_router_topk(const float* logits, int64_t T, int64_t E, int64_t k, int norm, const uint16_t* x,
+                       const uint16_t* gate, int64_t K, int32_t* idx, float* scores, void* stream) {
+  if (T < 0 || E <= 0 || k <= 0) return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
+  if (k > E) return qmoe::fail(QMOE_ERR_INVALID, "k=%lld > E=%lld", (long long)k, (long long)E);
+  if (T == 0) return QMOE_OK;
+  if (!logits || !idx || !scores) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+  if (k > kMaxK || E > 64 * kMaxPer)
+    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "k=%lld, E=%lld: the router takes k <= %d, E <= %d", (long long)k,
+                      (long long)E, kMaxK, 64 * kMaxPer);
+  if (SH) {
+    if (!x || !gate || K <= 0) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+    if (K % 8 || K > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "K=%lld: must be a multiple of 8", (long long)K);
+    if (!qmoe::aligned16(x) || !qmoe::aligned16(gate))
+      return qmoe::fail(QMOE_ERR_UNSUPPORTED, "x and gate must be 16-byte aligned");
+  }
+  const int64_t blocks = (T + 3) / 4;
+  if (blocks > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "too many tokens");
+  const dim3 grid((unsigned)blocks), block(256);
+  hipStream_t st = qmoe::as_stream(stream);
+  const int per = (int)((E + 63) / 64);
+  const int e = (int)E, kk = (int)k, K32 = (int)K;
+  if (per <= 1) router_topk_kernel<1, SH><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores, x, gate, K32);
+  else if (per <= 2) router_topk_kernel<2, SH><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores, x, gate, K32);
+  else if (per <= 4) router_topk_kernel<4, SH><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores, x, gate, K32);
+  else if (per <= 8) router_topk_kernel<8, SH><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores, x, gate, K32);
+  else router_topk_kernel<16, SH><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores, x, gate, K32);
+  return qmoe::launch_status("router_topk_kernel");
 }
 
 // Router logits over a dense bf16 router weight: logits[t, e] = x[t] . W[e]
@@ -256,23 +310,11 @@ extern "C" int qmoe_router_logits_dense(const uint16_t* x, int64_t T, int64_t K,
 
 extern "C" int qmoe_router_topk(const float* logits, int64_t T, int64_t E, int64_t k, int norm, int32_t* idx,
                                 float* scores, void* stream) {
-  if (T < 0 || E <= 0 || k <= 0) return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
-  if (k > E) return qmoe::fail(QMOE_ERR_INVALID, "k=%lld > E=%lld", (long long)k, (long long)E);
-  if (T == 0) return QMOE_OK;
-  if (!logits || !idx || !scores) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
-  if (k > kMaxK || E > 64 * kMaxPer)
-    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "k=%lld, E=%lld: the router takes k <= %d, E <= %d", (long long)k,
-                      (long long)E, kMaxK, 64 * kMaxPer);
-  const int64_t blocks = (T + 3) / 4;
-  if (blocks > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "too many tokens");
-  const dim3 grid((unsigned)blocks), block(256);
-  hipStream_t st = qmoe::as_stream(stream);
-  const int per = (int)((E + 63) / 64);
-  const int e = (int)E, kk = (int)k;
-  if (per <= 1) router_topk_kernel<1><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores);
-  else if (per <= 2) router_topk_kernel<2><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores);
-  else if (per <= 4) router_topk_kernel<4><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores);
-  else if (per <= 8) router_topk_kernel<8><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores);
-  else router_topk_kernel<16><<<grid, block, 0, st>>>(logits, T, e, kk, norm, idx, scores);
-  return qmoe::launch_status("router_topk_kernel");
+  return launch_router_topk<false>(logits, T, E, k, norm, nullptr, nullptr, 0, idx, scores, stream);
+}
+
+extern "C" int qmoe_router_topk_shared(const float* logits, int64_t T, int64_t E, int64_t k, int norm,
+                                       const uint16_t* x, const uint16_t* gate, int64_t K, int32_t* idx,
+                                       float* scores, void* stream) {
+  return launch_router_topk<true>(logits, T, E, k, norm, x, gate, K, idx, scores, stream);
 }

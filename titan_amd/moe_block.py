@@ -13,7 +13,7 @@ engine/patches/decode-fusion/fused_kernels.py:232-371).
         top-k's own code, and writes them for the down kernel, so the decode
         block is three launches)
     prefill:
-        order, tiles = stable sort of the pairs       qmoe_route
+        x_rows, tiles = stable sort of the pairs      qmoe_route_block
         h   = SwiGLU gate_up grouped GEMM             qmoe_gather_qmm_swiglu_sorted_tiles
         yd  = down grouped GEMM over h                qmoe_gather_qmm_sorted_tiles
         y   = un-permute + weighted sum               qmoe_weighted_sum
@@ -25,9 +25,12 @@ softmax to bf16 first and breaks bf16 ties arbitrarily
 near-ties; everything after the selection has the same semantics.
 
 The optional shared expert (language.py:81-89: a dense SwiGLU MLP gated by
-sigmoid(x w_gate)) is one more slot of the two decode kernels when it has the
-routed experts' shape, so the decode block stays three launches; otherwise it
-runs through the same kernels as a one-expert table.
+sigmoid(x w_gate)), when it has the routed experts' shape, is one more slot of
+the two decode kernels and one more expert of the prefill's GEMMs, with its
+score from the top-k kernel and its rows added by the weighted sum, so it takes
+no launch of its own; otherwise it runs through the same kernels as a
+one-expert table.  Up to 16 tokens its weights are always the exact affine
+ones, so a sorted call that narrow runs it through the decode kernels.
 
 Resident weights (``resident``): by default one copy, in the tile layout --
 the block repacks gate_up (in the gate/up-paired row order) and down at
@@ -64,6 +67,8 @@ ROUTER_GEMV_MAX_T = 16
 # qmoe_moe_down_wsum_tiles takes at most this many experts per token (the
 # MLX-layout qmoe_moe_down_wsum takes up to 64)
 TILE_DECODE_MAX_K = 16
+# qmoe_route_block takes at most this many experts (qmoe_route up to 8192)
+ROUTE_BLOCK_MAX_E = 2048
 
 
 def tile_decode_supported(hidden: int, inter: int, group_size: int = ops.GROUP, bits: int = ops.BITS,
@@ -158,6 +163,14 @@ class SparseMoeBlock:
         self._shared_slot = (self.decode_tiles and self._shared_decode_tiles and self.top_k < TILE_DECODE_MAX_K
                              and self._shared_tiles[0].N == self.gu_tiles.N
                              and shared.gate_weight.numel() == self.hidden)
+        # and one more expert of the sorted path's GEMMs
+        self._shared_expert_rows = (self._shared_tiles is not None and self._shared_tiles[0].N == self.gu_tiles.N
+                                    and shared.gate_weight.numel() == self.hidden
+                                    and self.num_experts <= ROUTE_BLOCK_MAX_E)
+        if self._shared_expert_rows:  # constant ids and scores of the shared expert's decode kernels
+            dev = self.gu_tiles.wp.device
+            self._zeros = torch.zeros(16, 1, dtype=torch.int32, device=dev)
+            self._ones = torch.ones(16, 1, dtype=torch.float32, device=dev)
 
     @property
     def nbytes(self) -> int:
@@ -198,11 +211,43 @@ class SparseMoeBlock:
                 return ops.down_wsum_tiles(h, self.down_tiles, idx, scores)
             h = ops.gate_up_silu(x2, *self.gate_up, idx, self.group_size, self.bits)
             return ops.down_wsum(h, *self.down, idx, scores, self.group_size, self.bits)
-        r = ops.route(idx, self.num_experts)
-        lhs = torch.div(r.order, k, rounding_mode="floor").to(torch.int32)
-        h = ops.gather_qmm_swiglu_sorted_tiles(x2, self.gu_tiles, r.tiles, x_rows=lhs)
-        yd = ops.gather_qmm_sorted_tiles(h, self.down_tiles, r.tiles)
-        return ops.moe_weighted_sum(yd, r.inv_order, scores, (T, self.hidden), self.wsum_mode)
+        if self.num_experts > ROUTE_BLOCK_MAX_E:
+            r = ops.route(idx, self.num_experts)
+            x_rows, inv, tiles = torch.div(r.order, k, rounding_mode="floor").to(torch.int32), r.inv_order, r.tiles
+        else:
+            x_rows, inv, tiles = ops.route_block(idx, self.num_experts)
+        h = ops.gather_qmm_swiglu_sorted_tiles(x2, self.gu_tiles, tiles, x_rows=x_rows)
+        yd = ops.gather_qmm_sorted_tiles(h, self.down_tiles, tiles)
+        return ops.moe_weighted_sum(yd, inv, scores, (T, self.hidden), self.wsum_mode)
+
+    def _sorted_with_shared(self, x2: torch.Tensor) -> torch.Tensor:
+        """The sorted path with the shared expert in its launches."""
+        T, k = x2.shape[0], self.top_k
+        gu_t, dn_t = self._shared_tiles
+        gate = self.shared.gate_weight
+        idx, scores = ops.router_topk_shared(self.route_logits(x2), k, x2, gate, self.norm)
+        if T <= 16:
+            x_rows, inv, tiles = ops.route_block(idx, self.num_experts)
+            h = ops.gather_qmm_swiglu_sorted_tiles(x2, self.gu_tiles, tiles, x_rows=x_rows)
+            yd = ops.gather_qmm_sorted_tiles(h, self.down_tiles, tiles)
+            ys = self._shared_mlp(x2)
+        else:
+            x_rows, inv, tiles = ops.route_block(idx, self.num_experts, shared=True)
+            h = ops.gather_qmm_sorted_tiles_shared(x2, self.gu_tiles, gu_t, tiles, x_rows=x_rows)
+            yd = ops.gather_qmm_sorted_tiles_shared(h, self.down_tiles, dn_t, tiles)
+            ys = yd[T * k:]
+        return ops.moe_weighted_sum_shared(yd, inv, scores, ys, self.wsum_mode)
+
+    def _shared_mlp(self, x2: torch.Tensor) -> torch.Tensor:
+        """The shared expert's SwiGLU MLP of up to 16 tokens, ungated."""
+        T = x2.shape[0]
+        zeros, ones = self._zeros[:T], self._ones[:T]
+        if self._shared_decode_tiles:
+            gu_t, dn_t = self._shared_tiles
+            return ops.down_wsum_tiles(ops.gate_up_silu_tiles(x2, gu_t, zeros), dn_t, zeros, ones)
+        sh = self.shared
+        h = ops.gate_up_silu(x2, *sh.gate_up, zeros, self.group_size, self.bits)
+        return ops.down_wsum(h, *sh.down, zeros, ones, self.group_size, self.bits)
 
     def shared_expert(self, x2: torch.Tensor) -> torch.Tensor:
         """sigmoid(x w_gate) * SwiGLU-MLP(x) (language.py:81-89)."""
@@ -241,7 +286,10 @@ class SparseMoeBlock:
             h, idx, scores = ops.gate_up_silu_tiles_topk_shared(x2, self.gu_tiles, self.route_logits(x2), self.top_k,
                                                                 gu_t, self.shared.gate_weight, self.norm)
             return ops.down_wsum_tiles_shared(h, self.down_tiles, idx, scores, dn_t).reshape(x.shape)
-        if self.decodes_with_topk(x2.shape[0]):
+        T = x2.shape[0]
+        if self._shared_expert_rows and not (T * self.top_k < self.sort_min_pairs and T <= 16):
+            return self._sorted_with_shared(x2).reshape(x.shape)
+        if self.decodes_with_topk(T):
             h, idx, scores = ops.gate_up_silu_tiles_topk(x2, self.gu_tiles, self.route_logits(x2), self.top_k,
                                                          self.norm)
             y = ops.down_wsum_tiles(h, self.down_tiles, idx, scores)

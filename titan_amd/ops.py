@@ -199,6 +199,29 @@ def route(ids: torch.Tensor, num_experts: int, tile_rows_: int | None = None) ->
     return Routing(order, inv, srt, tiles, ws[:1])
 
 
+def route_block(idx: torch.Tensor, num_experts: int, shared: bool = False):
+    """The routing step of a whole block over expert ids ``idx`` [T, k]
+    (qmoe_route_block): (x_rows, inv_order, tiles), x_rows [T*k (+ T)] the token
+    of each sorted row.  ``shared`` adds a shared expert as expert
+    ``num_experts``, whose T rows (one per token) follow the sorted pairs."""
+    _dev(idx, "idx")
+    dev = idx.device
+    T, k = idx.shape
+    ids = _i32(idx, "idx", dev)
+    n, extra, tr = T * k, T if shared else 0, tile_rows()
+    E = num_experts + (1 if shared else 0)
+    mt = max_tiles(n, num_experts, tr) + (extra + tr - 1) // tr
+    ws = int(_lib.load().qmoe_route_workspace_size(n, num_experts)) // 4
+    # one allocation, cut into the tables, each from a 256-byte boundary
+    sizes = [m for size in (n + extra, n, E + 1, mt, mt, 1, ws) for m in (size, -size % 64)]
+    x_rows, _, inv, _, offsets, _, trow, _, texp, _, nt, _, wsp, _ = torch.empty(
+        sum(sizes), dtype=torch.int32, device=dev).split(sizes)
+    _lib.call("qmoe_route_block", ids.data_ptr(), n, k, num_experts, extra, tr, x_rows.data_ptr(), inv.data_ptr(),
+              offsets.data_ptr(), trow.data_ptr(), texp.data_ptr(), nt.data_ptr(), mt, wsp.data_ptr(),
+              wsp.numel() * 4, _stream(ids))
+    return x_rows, inv, TileTable(offsets, trow, texp, nt, mt, tr, E, n + extra)
+
+
 # ------------------------------------------------------------- gather_qmm
 
 
@@ -682,6 +705,65 @@ def gather_qmm_swiglu_sorted_tiles(x: torch.Tensor, tw: TileWeights, tiles: Tile
     return h
 
 
+def gather_qmm_sorted_tiles_shared(x: torch.Tensor, tw: TileWeights, shared: TileWeights, tiles: TileTable,
+                                   x_rows: torch.Tensor | None = None) -> torch.Tensor:
+    """:func:`gather_qmm_sorted_tiles` (:func:`gather_qmm_swiglu_sorted_tiles`
+    for gate/up-paired weights) over ``route_block``'s tables with a shared
+    expert, whose weights are ``shared``."""
+    x = _bf16(x, "x")
+    K = x.shape[-1]
+    if K != tw.K:
+        raise ValueError(f"x has K={K}, the weights K={tw.K}")
+    if (shared.num_experts, shared.N, shared.K, shared.swiglu_pairs) != (1, tw.N, tw.K, tw.swiglu_pairs):
+        raise ValueError("the shared expert must have the routed experts' shape and layout")
+    if tiles.num_experts != tw.num_experts + 1 or tiles.tile_rows != tile_rows():
+        raise ValueError("tile table does not match this call")
+    x2 = x.reshape(-1, K)
+    xr = None if x_rows is None else _i32(x_rows.reshape(-1), "x_rows", x.device)
+    out = torch.empty(tiles.rows, tw.N // 2 if tw.swiglu_pairs else tw.N, dtype=torch.bfloat16, device=x.device)
+    _lib.call("qmoe_gather_qmm_sorted_tiles_shared", x2.data_ptr(), _ptr(xr), tiles.rows, K, tw.wp.data_ptr(),
+              tw.sb.data_ptr(), shared.wp.data_ptr(), shared.sb.data_ptr(), tw.num_experts, tw.N,
+              int(tw.swiglu_pairs), tiles.offsets.data_ptr(), tiles.tile_row.data_ptr(), tiles.tile_exp.data_ptr(),
+              tiles.ntiles.data_ptr(), tiles.maxt, out.data_ptr(), _stream(x))
+    return out
+
+
+def moe_weighted_sum_shared(xs: torch.Tensor, inv_order: torch.Tensor, scores: torch.Tensor, shared: torch.Tensor,
+                            mode: str = "fast") -> torch.Tensor:
+    """:func:`moe_weighted_sum` over the first rows*k of ``xs`` plus
+    ``scores[r, k] * shared[r]``: scores [rows, k + 1], shared [rows, D]."""
+    if mode not in _lib.WSUM_MODES:
+        raise QmoeUnsupported(_lib.ERR_UNSUPPORTED, f"mode={mode!r}")
+    xs, shared = _bf16(xs, "xs"), _bf16(shared, "shared")
+    rows, dim = shared.shape
+    k = scores.shape[-1] - 1
+    if xs.shape[-1] != dim or xs.shape[0] < rows * k or inv_order.numel() < rows * k or scores.shape[0] != rows:
+        raise ValueError("xs, inv_order, scores and shared disagree on rows, k or D")
+    sc = _f32(scores, "scores", xs.device)
+    inv = _i32(inv_order, "inv_order", xs.device)
+    out = torch.empty(rows, dim, dtype=torch.bfloat16, device=xs.device)
+    _lib.call("qmoe_weighted_sum_shared", xs.data_ptr(), inv.data_ptr(), sc.data_ptr(), rows, k, dim,
+              _lib.WSUM_MODES[mode], shared.data_ptr(), out.data_ptr(), _stream(xs))
+    return out
+
+
+def router_topk_shared(logits: torch.Tensor, k: int, x: torch.Tensor, gate: torch.Tensor, norm: bool = True):
+    """:func:`router_topk` with the shared expert's weight sigmoid(x . gate) as
+    one more score: (idx int32 [T, k], scores float32 [T, k + 1])."""
+    _dev(logits, "logits")
+    x, gate = _bf16(x, "x"), _bf16(gate, "gate")
+    T, E = logits.shape
+    lg = _logits(logits, T, E, x.device)
+    K = x.shape[-1]
+    if x.shape[0] != T or gate.numel() != K:
+        raise ValueError("x, logits and gate disagree")
+    idx = torch.empty(T, k, dtype=torch.int32, device=x.device)
+    scores = torch.empty(T, k + 1, dtype=torch.float32, device=x.device)
+    _lib.call("qmoe_router_topk_shared", lg.data_ptr(), T, E, k, int(bool(norm)), x.data_ptr(), gate.data_ptr(), K,
+              idx.data_ptr(), scores.data_ptr(), _stream(x))
+    return idx, scores
+
+
 def router_topk(logits: torch.Tensor, k: int, norm: bool = True):
     """Top-k experts per token from router logits, (idx int32 [T, k], scores
     float32 [T, k]); descending, ties to the lower expert index.  norm: the
@@ -728,6 +810,7 @@ __all__ = [
     "GROUP", "BITS", "QmoeError", "QmoeUnsupported", "TileTable", "TileWeights", "Routing", "build_tiles", "route",
     "repack_tiles", "gather_qmm_sorted_tiles", "gather_qmm_int8_sorted_tiles", "router_topk", "router_logits", "gather_qmm_swiglu_sorted_tiles", "swiglu_pair_order", "gather_qmv_tiles", "gate_up_silu_tiles",
     "down_wsum_tiles", "gate_up_silu_tiles_topk", "gate_up_silu_tiles_topk_shared", "down_wsum_tiles_shared",
+    "route_block", "gather_qmm_sorted_tiles_shared", "moe_weighted_sum_shared", "router_topk_shared",
     "max_tiles", "tile_rows", "unpack", "dequantize", "gather_qmv", "gather_qmm_sorted", "gather_qmm",
     "gemm_supported", "quantized_matmul", "gate_up_silu", "down_wsum", "moe_weighted_sum",
     "quantize_act_int8", "gather_qmm_int8_sorted",
