@@ -1,0 +1,44 @@
+"""The grouped GEMM's kernel for few rows per expert against its tile kernel:
+the same rows and weights through a table of many experts (few rows per expert)
+and through one of only the used experts give the same bits."""
+
+import pytest
+import torch
+
+from titan_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _quant(g, lead, K, dev):
+    w = torch.randint(-2 ** 31, 2 ** 31, (*lead, K // 8), dtype=torch.int32, device=dev, generator=g)
+    s = (0.004 + 0.004 * torch.rand(*lead, K // 64, device=dev, generator=g)).to(torch.bfloat16)
+    return w, s, (-7.5 * s.float()).to(torch.bfloat16)
+
+
+# rows of the used experts: one row, the 32-row subtile's and the 128-row
+# tile's edges, several tiles; K of 1, 2, 3, 4 and 8 groups (the unrolled cycle
+# is three)
+@pytest.mark.parametrize("rows", [(1,), (31, 32, 33), (127, 128, 129), (64, 1, 300)])
+@pytest.mark.parametrize("N,K", [(256, 64), (512, 128), (256, 192), (768, 256), (256, 512)])
+@pytest.mark.parametrize("gathered", [False, True])
+def test_rows_kernel_is_the_tile_kernel(dev, rows, N, K, gathered):
+    print(f"[case] few rows {rows} N={N} K={K} gathered={gathered}", flush=True)
+    R, n = sum(rows), len(rows)
+    E = (R + 5) // 6 + n            # at most six rows per expert
+    g = torch.Generator(device=dev).manual_seed(R + N + K)
+    used = torch.randperm(E, device=dev, generator=g)[:n].sort()[0]
+    few = torch.repeat_interleave(torch.arange(n, device=dev), torch.tensor(rows, device=dev))
+    more = 7 * (n + 1)              # rows of one more expert, which put the second table past the limit
+    T = R + more
+    x = torch.randn(T, K, device=dev, generator=g).to(torch.bfloat16)
+    x_rows = torch.randint(0, T, (T,), dtype=torch.int32, device=dev, generator=g) if gathered else None
+    w = _quant(g, (E, N), K, dev)
+    sub = tuple(t[torch.cat([used, used[:1]])].contiguous() for t in w)
+    many_t = ops.build_tiles(used[few].to(torch.int32), E)
+    few_t = ops.build_tiles(torch.cat([few, torch.full((more,), n, device=dev)]).to(torch.int32), n + 1)
+    for pairs in (False, True):
+        gemm = ops.gather_qmm_swiglu_sorted_tiles if pairs else ops.gather_qmm_sorted_tiles
+        y = gemm(x, ops.repack_tiles(*w, swiglu_pairs=pairs), many_t, x_rows=None if x_rows is None else x_rows[:R])
+        ref = gemm(x, ops.repack_tiles(*sub, swiglu_pairs=pairs), few_t, x_rows=x_rows)
+        assert torch.equal(y, ref[:R])

@@ -632,15 +632,176 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmA
 #endif
 }
 
+// ---- few rows per expert -------------------------------------------------
+//
+// The same products for tiles of few rows, where a call streams its experts'
+// weights for a handful of rows each.  A wave owns one 64-column block of up
+// to kRowsPerUnit rows of one tile, alone: no LDS, no barrier.  In the tile
+// layout a lane's share of a group's codes (two 16-byte units) and of its
+// scale|bias words (two) needs no exchange, so they go straight to registers,
+// kRowsDepth groups ahead, and so do the lane's 64 contiguous bytes of its
+// activation row (the rows past the tile repeat its last valid row: the same
+// lines).  Dequantisation, MFMAs, their order and the epilogue's arithmetic
+// are the tile kernel's, so the results are bit-identical to it.
+//
+// Where the tile kernel has one 256-column unit per workgroup, each with its
+// own latency to fill and drain a ring, here 4 to 16 times as many waves run
+// independently.  Per call in a graph (256 experts, top-10, 2048 x 1024
+// gate_up + SwiGLU / 512 x 2048 down; floor: the used experts' bytes at a 2 GiB
+// copy's 4.86 TB/s):
+//   tokens   tile kernel    this kernel    floor
+//        7   32.9 / 14.3    17.7 / 10.4    13.6 /  6.8 us
+//       16   33.0 / 22.3    27.4 / 15.1    21.6 / 10.8
+//       32   37.3 / 23.1    31.8 / 19.6    29.9 / 14.9
+//       96   60.2 / 34.6    52.0 / 29.3    45.9 / 22.9
+//      200   64.1 / 42.2    68.6 / 40.0    50.7 / 25.4
+//      400   71.0 / 44.2    90.8 / 54.1    55.8 / 27.9
+// Beyond about six rows per expert the activation reads, a row's line per lane
+// and wave where the tile kernel copies each row once per workgroup, are what
+// bounds it (few_rows draws the line there).  Two or four groups ahead, and two
+// or four waves per SIMD, measured within 5% of three and three; a 32-column
+// unit twice as often (half the dequantisation per wave, all of its activation
+// reads) is slower from 7 tokens on, up to 1.9x at the down shape.
+constexpr int kRowsPerUnit = 32;
+constexpr int kRowsDepth = 3;
+constexpr int kRowsMaxPerExpert = 6;
+
+struct RowsGroup {
+  i32x4_t a[4];    // activation bytes 64h .. 64h + 63 of the group
+  i32x4_t c[2];    // the lane's codes of columns l32 and 32 + l32
+  uint32_t sb[2];  // their scale|bias words
+};
+
+template <bool SWIGLU>
+__global__ __launch_bounds__(kThreads, 3) void gemm_rows_kernel(GemmArgs a, int max_tiles) {
+  constexpr int D = kRowsDepth;
+  const int lane = threadIdx.x % 64, l32 = lane % 32, h = lane / 32;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+  const int NB = a.N / kBN;
+  // blocks: row subtile slowest (most tiles have only the first), then tile
+  // from the last (a shared expert's full tiles) to the first, then columns
+  const int per_sub = max_tiles * NB;
+  const int sub = blockIdx.x / per_sub;
+  const int rem = blockIdx.x - sub * per_sub;
+  const int back = rem / NB;
+  const int nblk = rem - back * NB;
+  const int tile = a.ntiles[0] - 1 - back;
+  if (tile < 0) return;
+  const TileRows tr = tile_rows_of(Tiles{a.offsets, a.tile_row, a.tile_exp, a.ntiles, a.n_rows, a.num_experts}, tile);
+  const int valid = tr.valid - sub * kRowsPerUnit;
+  if (valid <= 0) return;
+  const int64_t row0 = tr.row0 + sub * kRowsPerUnit;
+  const int K = a.K, G = K / 64;
+  const bool last = a.last_w && tr.e == a.num_experts - 1;
+  const int64_t chunk0 = uniform64(((int64_t)(last ? 0 : tr.e) * (a.N / 64) + nblk * kWaves + wave) * G);
+  const char* wb = reinterpret_cast<const char*>(last ? a.last_w : a.w) + chunk0 * 2048;
+  const char* sbb = reinterpret_cast<const char*>(last ? a.last_sb : a.sb) + chunk0 * 256;
+  int64_t src = row0 + min(l32, valid - 1);
+  if (a.x_rows) src = a.x_rows[src];
+  const char* xa = reinterpret_cast<const char*>(a.x + src * K) + 64 * h;
+
+  // the activations first: loads return in order, and a wait for them would
+  // otherwise be a wait for the same group's weights, D groups ahead
+  auto load = [&](RowsGroup& r, int g) {
+    const char* ag = xa + (size_t)g * 128;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r.a[q] = *reinterpret_cast<const i32x4_t*>(ag + 16 * q);
+    const char* wg = wb + (size_t)g * 2048;
+    const char* sg = sbb + (size_t)g * 256;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      r.sb[j] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(sg + j * 128 + l32 * 4));
+      r.c[j] = __builtin_nontemporal_load(reinterpret_cast<const i32x4_t*>(wg + j * 1024 + lane * 16));
+    }
+  };
+
+  f32x16_t acc[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+  auto group = [&](const RowsGroup& r) {
+    WState ws;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) ws.w[j][t] = (uint32_t)r.c[j][t];
+      set_scale(ws, j, r.sb[j], r.sb[j], 0, 16);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      i32x4_t b[2];
+#pragma unroll
+      for (int pr = 0; pr < 4; ++pr) dequant_pair(b, ws, kk, pr);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, b[j]),
+                                                         __builtin_bit_cast(bf16x8_t, r.a[kk]), acc[j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);  // else the scheduler spreads dequantised fragments past the registers
+    }
+  };
+  RowsGroup rg[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(rg[d], min(d, G - 1));
+  int g0 = 0;
+  for (; g0 + D <= G; g0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      group(rg[d]);
+      load(rg[d], min(g0 + d + D, G - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d + 1 < D; ++d)
+    if (g0 + d < G) group(rg[d]);  // uniform
+
+  // lane l32 is row l32; register 4q + t is MFMA row 8q + 4h + t
+  if (l32 >= valid) return;
+  const int unit = nblk * kWaves + wave;
+  uint16_t* orow = a.out + (row0 + l32) * (int64_t)(SWIGLU ? a.N / 2 : a.N) + unit * (SWIGLU ? 32 : 64) + 4 * h;
+  if constexpr (SWIGLU) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float hv[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float g = acc[0][4 * q + t], u = acc[1][4 * q + t];
+        hv[t] = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
+      }
+      *reinterpret_cast<uint2*>(orow + 8 * q) = make_uint2(cvt_pk_bf16(hv[0], hv[1]), cvt_pk_bf16(hv[2], hv[3]));
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<uint2*>(orow + 32 * j + 8 * q) =
+            make_uint2(cvt_pk_bf16(acc[j][4 * q], acc[j][4 * q + 1]), cvt_pk_bf16(acc[j][4 * q + 2], acc[j][4 * q + 3]));
+  }
+}
+
 }  // namespace
 
 extern "C" int qmoe_gemm_tile_rows(void) { return kBM; }
 
 namespace {
 
+// Few rows per expert: gemm_rows_kernel (its comment has both sides measured).
+bool few_rows(const GemmArgs& a, int64_t max_tiles) {
+  const int64_t blocks = max_tiles * (a.N / kBN) * (kTileRows / kRowsPerUnit);
+  return a.n_rows <= (int64_t)kRowsMaxPerExpert * a.num_experts && blocks <= 0x7FFFFFFF;
+}
+
 int launch_gemm(const GemmArgs& a, int64_t max_tiles, bool tiled, void* stream, bool swiglu = false) {
   const dim3 grid((unsigned)grid_blocks(max_tiles * (a.N / kBN)));
   hipStream_t st = qmoe::as_stream(stream);
+  if (tiled && few_rows(a, max_tiles)) {
+    const dim3 g((unsigned)(max_tiles * (a.N / kBN) * (kTileRows / kRowsPerUnit)));
+    if (swiglu) gemm_rows_kernel<true><<<g, dim3(kThreads), 0, st>>>(a, (int)max_tiles);
+    else gemm_rows_kernel<false><<<g, dim3(kThreads), 0, st>>>(a, (int)max_tiles);
+    return qmoe::launch_status("gemm_rows_kernel");
+  }
   if (swiglu) gemm_bf16_kernel<true, true><<<grid, dim3(kThreads), 0, st>>>(a);
   else if (tiled) gemm_bf16_kernel<true, false><<<grid, dim3(kThreads), 0, st>>>(a);
   else gemm_bf16_kernel<false, false><<<grid, dim3(kThreads), 0, st>>>(a);
