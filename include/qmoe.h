@@ -150,7 +150,9 @@ int qmoe_gather_qmv(const uint16_t* x, const int32_t* x_rows,
 /* mx.quantized_matmul(x, w, scales, biases, transpose=True, group_size, bits)
  * for x [M, K] (titan/adapters/mlx/compiled.py:209-218; small-M drop-in
  * engine/patches/smallm/kernel.py:333-391): out [M, N].  Same bit widths and
- * group sizes as qmoe_gather_qmv. */
+ * group sizes as qmoe_gather_qmv: its kernels for a row or few, a kernel that
+ * reads the weights once per up to 64 rows for more; the same exact affine
+ * weights and fp32 accumulation in both. */
 int qmoe_quantized_matmul(const uint16_t* x, int64_t M, int64_t K,
                           const uint32_t* w, const uint16_t* scales,
                           const uint16_t* biases, int64_t N, int group_size,

@@ -20,6 +20,7 @@
 #include <stdlib.h>
 
 #include "common.h"
+#include "qmm.h"
 #include "topk.h"
 
 namespace {
@@ -1663,6 +1664,8 @@ extern "C" int qmoe_quantized_matmul(const uint16_t* x, int64_t M, int64_t K, co
   if (rc) return rc;
   if (!qmoe::aligned16(x) || !qmoe::aligned16(w)) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "x and w must be 16-byte aligned");
   if (N > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "N too large");
+  if (qmoe_qmm::takes(M, N, K, group_size, bits))
+    return qmoe_qmm::launch(x, M, K, w, scales, biases, N, group_size, bits, out, qmoe::as_stream(stream));
   QmvArgs a{x, K, nullptr, 1, nullptr, M, (int)K, group_size, w, scales, biases, 1, (int)N, (int)N, out};
   return launch_qmv<0>(a, lpr, nv, qmoe::as_stream(stream), bits);
 }
