@@ -44,12 +44,11 @@ struct XChunk {
   float sum;
 };
 
-__device__ __forceinline__ void load_x_chunk(const uint16_t* __restrict__ src, XChunk& c) {
-  const uint4* q = reinterpret_cast<const uint4*>(src);
+__device__ __forceinline__ void pair_x_chunk(const uint4 (&q)[4], XChunk& c) {
   float s = 0.f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    uint4 a = q[j];
+    const uint4 a = q[j];
     c.p[4 * j + 0] = (a.x & 0xFFFFu) | (a.z << 16);
     c.p[4 * j + 1] = (a.x >> 16) | (a.z & 0xFFFF0000u);
     c.p[4 * j + 2] = (a.y & 0xFFFFu) | (a.w << 16);
@@ -58,6 +57,15 @@ __device__ __forceinline__ void load_x_chunk(const uint16_t* __restrict__ src, X
          ((bf16lo(a.z) + bf16hi(a.z)) + (bf16lo(a.w) + bf16hi(a.w)));
   }
   c.sum = s;
+}
+__device__ __forceinline__ void load_x_raw(const uint16_t* __restrict__ src, uint4 (&q)[4]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) q[j] = reinterpret_cast<const uint4*>(src)[j];
+}
+__device__ __forceinline__ void load_x_chunk(const uint16_t* __restrict__ src, XChunk& c) {
+  uint4 q[4];
+  load_x_raw(src, q);
+  pair_x_chunk(q, c);
 }
 
 // (a & m) | c in one v_and_or_b32.  A gfx950 VOP3 instruction encodes no
@@ -1205,54 +1213,80 @@ __global__ __launch_bounds__(1024) void down_wsum_kernel(DownArgs a) {
   if (l == 0 && valid) a.y[(int64_t)t * a.D + d] = (uint16_t)f32_to_bf16(acc);
 }
 
-// Fused down + weighted sum for I = 512, pair-parallel: one block per
-// (token t, R output rows), one wave per expert slot j of the token (k waves).
-// Lane (rg = lane/16, l = lane%16) owns 32-code chunk l of rows d0 + 4i + rg
-// (i < R/4), so each 16-byte load instruction reads four consecutive 256-byte
-// rows.  A wave streams only its own expert's R rows (R * 288 bytes), which
-// puts k waves per row block in flight: at one token, 2560 waves where a wave
-// per (token, row block) walking all k experts gives 256 and is latency-bound.
-// The pair's h chunk is loaded before the expert id (it does not depend on
-// it); the slots' score-weighted row values meet in LDS and are summed in
+// Fused down + weighted sum, pair-parallel: one block per (token t, R output
+// rows), one wave per expert slot j of the token (k waves).  Lane (rg =
+// lane / LPR, l = lane % LPR) owns 32-code chunks l, l + LPR, .. (NV of them)
+// of rows d0 + GPW*i + rg (GPW = 64 / LPR rows per pass, i < R / GPW), so each
+// 16-byte load instruction reads LPR * 16 contiguous bytes of GPW rows.  A wave
+// streams only its own expert's R rows, which puts k waves per row block in
+// flight: at one token and I = 512, 2560 waves where a wave per (token, row
+// block) walking all k experts gives 256 and is latency-bound (and so at other
+// widths: I = 768, three tokens x top-8 of 128 experts, 2048 rows, 18.1 against
+// 8.0 us with such waves; 10.9 against 6.3 us at I = 256 and eight tokens, 39.5
+// against 24.6 us at I = 1536, top-4 and sixteen).
+// The expert id is requested first and the pair's h chunks, which do not wait
+// for it, next (paired up before the id's use, they cost 4.8 -> 5.6 us at I = 512
+// and two tokens); the slots' score-weighted row values meet in LDS and are summed in
 // slot order, so the result is deterministic (fused_kernels.py:93-169
 // arithmetic: fp32 throughout, one bf16 rounding).  Tokens that share an
 // expert read its rows from L2 or the Infinity Cache.
 constexpr int kPairMaxK = 16;
+constexpr int kPairMaxNV = 3;  // 17 registers per chunk of h and four per row's: 128 hold no more
 
-template <int R>
+template <int R, int NV, int LPR>
 __global__ __launch_bounds__(64 * kPairMaxK) void down_pair_kernel(DownArgs a) {
-  constexpr int NI = R / 4;
+  constexpr int GPW = 64 / LPR;
+  constexpr int NI = R / GPW;
+  constexpr int I = 32 * LPR * NV;
+  static_assert(R % GPW == 0, "whole passes");
   __shared__ float red[kPairMaxK][R];
   const int t = blockIdx.y;
   const int j = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const int rg = lane >> 4, l = lane & 15;
+  const int rg = lane / LPR, l = lane % LPR;
   const int d0 = blockIdx.x * R;
   const int D = a.D;
-  const int G = 512 / a.group_size;
-  const int gi = (l * 32) / a.group_size;
+  const int G = I / a.group_size;
   const int64_t p = (int64_t)t * a.k + j;
-  // the pair's h chunk first: it does not wait for the expert id
-  XChunk hc;
-  load_x_chunk(a.h + p * 512 + l * 32, hc);
+  // the expert id, then the pair's h chunks, which do not wait for it; they
+  // are paired up only once the rows it selects have been asked for
   int e = a.idx[p];
+  uint4 hr[NV][4];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) load_x_raw(a.h + p * I + v * 32 * LPR + l * 32, hr[v]);
+  __builtin_amdgcn_sched_barrier(0);
   e = min(max(e, 0), a.num_experts - 1);
   const float sc = a.scores[p];
-  uint4 wq[NI];
-  uint16_t sv[NI], bv[NI];
+  uint4 wq[NI][NV];
+  uint16_t sv[NI][NV], bv[NI][NV];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int64_t row = (int64_t)e * D + min(d0 + 4 * i + rg, D - 1);
-    wq[i] = load_nt(reinterpret_cast<const uint4*>(a.w + row * 64) + l);
-    sv[i] = a.s[row * G + gi];
-    bv[i] = a.b[row * G + gi];
+    const int64_t row = (int64_t)e * D + min(d0 + GPW * i + rg, D - 1);
+    const uint4* pw = reinterpret_cast<const uint4*>(a.w + row * (I / 8)) + l;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int gi = (v * 32 * LPR + l * 32) / a.group_size;
+      wq[i][v] = load_nt(pw + v * LPR);
+      sv[i][v] = a.s[row * G + gi];
+      bv[i][v] = a.b[row * G + gi];
+    }
   }
+  __builtin_amdgcn_sched_barrier(0);
+  XChunk hc[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) pair_x_chunk(hr[v], hc[v]);
   const uint32_t mv = magic_vgpr();
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const float v = group_sum<16>(affine_chunk(dot_chunk(wq[i], hc, mv), hc.sum, bf16_to_f32(sv[i]),
-                                               bf16_to_f32(bv[i])));
-    if (l == 0) red[j][4 * i + rg] = sc * v;
+    float part = 0.f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const float c = affine_chunk(dot_chunk(wq[i][v], hc[v], mv), hc[v].sum, bf16_to_f32(sv[i][v]),
+                                   bf16_to_f32(bv[i][v]));
+      part = v == 0 ? c : part + c;
+    }
+    const float s = group_sum<LPR>(part);
+    if (l == 0) red[j][GPW * i + rg] = sc * s;
   }
   __syncthreads();
   if (threadIdx.x < R) {
@@ -1261,6 +1295,22 @@ __global__ __launch_bounds__(64 * kPairMaxK) void down_pair_kernel(DownArgs a) {
     const int d = d0 + threadIdx.x;
     if (d < D) a.y[(int64_t)t * D + d] = (uint16_t)f32_to_bf16(y);
   }
+}
+
+// Rows per wave.  One token: the fewest whole passes of at least eight rows
+// (more waves in flight); from two tokens on 16 (measured at I = 512: 3.6 vs
+// 4.5 us at T = 1, 11.6 vs 14.9 us at T = 8, R = 8 vs 16), or 8 where two passes
+// of a wide row fill the registers.
+template <int NV, int LPR>
+int launch_down_pair(const DownArgs& a, hipStream_t st) {
+  constexpr int GPW = 64 / LPR;
+  constexpr int R1 = GPW > 8 ? GPW : 8;
+  constexpr int R2 = LPR == 16 && NV > 2 ? 8 : 16;
+  const int R = a.T == 1 ? R1 : R2;
+  const dim3 grid((unsigned)((a.D + R - 1) / R), (unsigned)a.T), block((unsigned)(64 * a.k));
+  if (a.T == 1) down_pair_kernel<R1, NV, LPR><<<grid, block, 0, st>>>(a);
+  else down_pair_kernel<R2, NV, LPR><<<grid, block, 0, st>>>(a);
+  return qmoe::launch_status("down_pair_kernel");
 }
 
 // down_pair_kernel over tile-layout down weights [E, D, I = 512] (group 64,
@@ -1723,14 +1773,12 @@ extern "C" int qmoe_moe_down_wsum(const uint16_t* h, const int32_t* idx, const f
   DownArgs a{h, idx, scores, (int)T, (int)top_k, (int)I, group_size, w, scales, biases,
              num_experts, (int)D, y};
   hipStream_t st = qmoe::as_stream(stream);
-  if (I == 512 && top_k <= kPairMaxK) {
-    // rows per wave: 8 for one token (more waves in flight), 16 from two on
-    // (measured: 3.6 vs 4.5 us at T = 1, 11.6 vs 14.9 us at T = 8)
-    const int R = T == 1 ? 8 : 16;
-    dim3 grid2((unsigned)((D + R - 1) / R), (unsigned)T), block2((unsigned)(64 * top_k));
-    if (R == 8) down_pair_kernel<8><<<grid2, block2, 0, st>>>(a);
-    else down_pair_kernel<16><<<grid2, block2, 0, st>>>(a);
-    return qmoe::launch_status("down_pair_kernel");
+  if (top_k <= kPairMaxK && nv <= kPairMaxNV) {
+#define DP_CASE(NV_, L_) \
+  if (nv == NV_ && lpr == L_) return launch_down_pair<NV_, L_>(a, st);
+    // (pick_split gives eight or four lanes per row odd counts of chunks only)
+    DP_CASE(1, 16) DP_CASE(2, 16) DP_CASE(3, 16) DP_CASE(1, 8) DP_CASE(3, 8) DP_CASE(1, 4) DP_CASE(3, 4)
+#undef DP_CASE
   }
   const int gpw = 64 / lpr;
   dim3 grid((unsigned)((D + gpw - 1) / gpw)), block((unsigned)(64 * T));
