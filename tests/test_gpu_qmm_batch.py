@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 # than a batch of four units, a ragged last batch, one batch per wave and more
 @pytest.mark.parametrize("bits,gs", [(4, 32), (4, 64), (4, 128), (8, 32), (8, 64), (8, 128)])
 @pytest.mark.parametrize("M,N,K", [(3, 4096, 2048), (5, 4099, 1024), (16, 1000, 2048), (17, 999, 2048), (33, 600, 2560),
-                                   (49, 700, 896), (64, 520, 768), (130, 257, 640), (1400, 100, 128), (4, 2048, 6144)])
+                                   (49, 700, 896), (64, 520, 768), (130, 257, 640), (1400, 100, 128), (8, 2048, 6144)])
 def test_quantized_matmul_batch(dev, bits, gs, M, N, K):
     if bits == 8 and K > 4096 and K % 2048:
         pytest.skip("no 8-bit kernel for this K")

@@ -303,13 +303,18 @@ int launch_gs(const QmmArgs& a, int group_size, hipStream_t st) {
 namespace qmoe_qmm {
 
 bool takes(int64_t M, int64_t N, int64_t K, int group_size, int bits) {
-  (void)group_size;
   if (K % 64 || K > (1 << 24) || M > 65535LL * 32 || (bits != 4 && bits != 8)) return false;
   // The GEMV re-reads the weights for every row, at about 7 TB/s from the
-  // caches: below 8 MB of such reads its shorter chain wins (the table above:
-  // 1000 x 2048 at 8 rows, 8.2 MB, is where they meet), and so it does for two
-  // rows of 4-bit codes at any size (9216 x 2048: 6.2 against 7.3 us).
-  return (M >= 3 || (M == 2 && bits == 8)) && M * (N * K * bits / 8) >= (8 << 20);
+  // caches; this kernel's time hardly depends on the rows up to 16 but starts
+  // from a longer chain.  Over 1000 x 2048 to 9216 x 2048 and 2048 x 4096 they
+  // meet between two and five rows of 4-bit codes (at four rows 5.2/4.5 us for
+  // 4096 x 2048 but 5.2/5.6 for 2048 x 4096) and between two and three of 8-bit
+  // ones (at three 7.1/4.9 and 7.5/6.1); group 32, whose units cost it twice
+  // the matrix work, at up to eight (4.1/4.2 at 1000 x 2048) and five rows.
+  // Below a few MB of weight reads both are launch-bound and the GEMV's chain
+  // is the shorter one.
+  const int64_t min_rows = bits == 4 ? (group_size == 32 ? 8 : 5) : (group_size == 32 ? 5 : 3);
+  return M >= min_rows && M * (N * K * bits / 8) >= (4 << 20);
 }
 
 int launch(const uint16_t* x, int64_t M, int64_t K, const uint32_t* w, const uint16_t* scales, const uint16_t* biases,
