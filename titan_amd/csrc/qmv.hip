@@ -44,19 +44,32 @@ struct XChunk {
   float sum;
 };
 
+// Eight elements (a quarter of a chunk): their pairs in p, their sum returned.
+__device__ __forceinline__ float pair_x_quarter(const uint4& a, uint4& p) {
+  p.x = (a.x & 0xFFFFu) | (a.z << 16);
+  p.y = (a.x >> 16) | (a.z & 0xFFFF0000u);
+  p.z = (a.y & 0xFFFFu) | (a.w << 16);
+  p.w = (a.y >> 16) | (a.w & 0xFFFF0000u);
+  return ((bf16lo(a.x) + bf16hi(a.x)) + (bf16lo(a.y) + bf16hi(a.y))) +
+         ((bf16lo(a.z) + bf16hi(a.z)) + (bf16lo(a.w) + bf16hi(a.w)));
+}
 __device__ __forceinline__ void pair_x_chunk(const uint4 (&q)[4], XChunk& c) {
   float s = 0.f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const uint4 a = q[j];
-    c.p[4 * j + 0] = (a.x & 0xFFFFu) | (a.z << 16);
-    c.p[4 * j + 1] = (a.x >> 16) | (a.z & 0xFFFF0000u);
-    c.p[4 * j + 2] = (a.y & 0xFFFFu) | (a.w << 16);
-    c.p[4 * j + 3] = (a.y >> 16) | (a.w & 0xFFFF0000u);
-    s += ((bf16lo(a.x) + bf16hi(a.x)) + (bf16lo(a.y) + bf16hi(a.y))) +
-         ((bf16lo(a.z) + bf16hi(a.z)) + (bf16lo(a.w) + bf16hi(a.w)));
+    uint4 p;
+    s += pair_x_quarter(q[j], p);
+    c.p[4 * j + 0] = p.x;
+    c.p[4 * j + 1] = p.y;
+    c.p[4 * j + 2] = p.z;
+    c.p[4 * j + 3] = p.w;
   }
   c.sum = s;
+}
+// v of one lane of the quad (quad_perm broadcast, SEL = 0x55 * lane)
+template <int SEL>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), SEL, 0xf, 0xf, false));
 }
 __device__ __forceinline__ void load_x_raw(const uint16_t* __restrict__ src, uint4 (&q)[4]) {
 #pragma unroll
@@ -263,24 +276,21 @@ __device__ __forceinline__ void pair_topk_store(const QmvArgs& a, uint32_t t, co
 }
 
 // The shared expert's score of token t (language.py:81-89): sigmoid(x . gate)
-// in fp32, from the x row the wave holds (lane l: elements v*2048 + 32l ..),
-// written to the token's last slot with id num_experts (the routed experts end
-// below it; the down kernel goes by the slot).
+// in fp32, by one wave, written to the token's last slot with id num_experts
+// (the routed experts end below it; the down kernel goes by the slot).
 template <int NV>
-__device__ __forceinline__ void shared_score_store(const QmvArgs& a, uint32_t t, const uint4 (&xa)[NV][4]) {
+__device__ __forceinline__ void shared_score_store(const QmvArgs& a, uint32_t t, const uint16_t* xrow) {
   const int lane = threadIdx.x & 63;
+  const uint4* xp = reinterpret_cast<const uint4*>(xrow);
+  const uint4* gp = reinterpret_cast<const uint4*>(a.sh_gate);
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const uint4* gp = reinterpret_cast<const uint4*>(a.sh_gate + v * 2048 + lane * 32);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint4 gq = gp[q];
-      acc[q] = dot2_bf16(xa[v][q].x, gq.x, acc[q]);
-      acc[q] = dot2_bf16(xa[v][q].y, gq.y, acc[q]);
-      acc[q] = dot2_bf16(xa[v][q].z, gq.z, acc[q]);
-      acc[q] = dot2_bf16(xa[v][q].w, gq.w, acc[q]);
-    }
+  for (int u = 0; u < 4 * NV; ++u) {
+    const uint4 xq = xp[u * 64 + lane], gq = gp[u * 64 + lane];
+    acc[u % 4] = dot2_bf16(xq.x, gq.x, acc[u % 4]);
+    acc[u % 4] = dot2_bf16(xq.y, gq.y, acc[u % 4]);
+    acc[u % 4] = dot2_bf16(xq.z, gq.z, acc[u % 4]);
+    acc[u % 4] = dot2_bf16(xq.w, gq.w, acc[u % 4]);
   }
   const float z = qmoe_topk::wave_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
   if (lane == 0) {
@@ -404,6 +414,14 @@ __device__ __forceinline__ float sum8(float v) {
   v += as_f(__builtin_amdgcn_update_dpp(0, as_u(v), 0x4E, 0xf, 0xf, false));   // quad_perm 2,3,0,1
   v += as_f(__builtin_amdgcn_update_dpp(0, as_u(v), 0x141, 0xf, 0xf, false));  // row_half_mirror
   return v;
+}
+// sum over the eight lanes l, l ^ 8, l ^ 16, ..: in every lane, period 8
+__device__ __forceinline__ float sum_slots(float v) {
+  v += as_f(__builtin_amdgcn_update_dpp(0, as_u(v), 0x128, 0xf, 0xf, false));  // row_ror:8
+  const auto r16 = __builtin_amdgcn_permlane16_swap(as_u(v), as_u(v), false, false);
+  v = as_f(r16[0]) + as_f(r16[1]);
+  const auto r32 = __builtin_amdgcn_permlane32_swap(as_u(v), as_u(v), false, false);
+  return as_f(r32[0]) + as_f(r32[1]);
 }
 // eight per-lane partials -> 64-lane sums; lanes 8q..8q+7 hold sum q
 __device__ __forceinline__ float reduce8(const float (&v)[8], int lane) {
@@ -960,7 +978,7 @@ __global__ __launch_bounds__(64) void qmv64_paired_kernel(QmvArgs a) {
       wu[q][v] = load_nt(units + 64);  // half j = 1: up, two 32-unit halves further
     }
   pair_topk_store<PER, SH>(a, xr, ts);  // while the weights are in flight
-  if (SH && shared && i0 == 0) shared_score_store<NV>(a, xr, xa);
+  if (SH && shared && i0 == 0) shared_score_store<NV>(a, xr, xrow);
   XChunk xc[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
@@ -1009,43 +1027,53 @@ __global__ __launch_bounds__(64) void qmv64_paired_kernel(QmvArgs a) {
 
 // Fused gate_up + SwiGLU over the gate/up-paired tile layout with line reads:
 // a wave computes RG indices i0 .. (gate rows l0 .. l0 + RG - 1 of half j = 0
-// of column block c = i0 / 32, up rows in half j = 1).  Lane 8r + s holds row
+// of column block c = i0 / 32, up rows in half j = 1).  Lane 8 s + r holds row
 // slot r and group slot s; its load (p, h) reads the 16-byte unit
-// (g = 8p + s, j, h, l0 + rr) of its row, so the lanes of one group slot read
+// (g = 8p + s, j, h, l0 + rr) of its row, so eight neighbouring lanes read
 // consecutive rows of one (g, j, h): RG = 8 gives each slot two whole 128-byte
 // lines (rows of gate and of up, r = 0..7 each), RG = 4 one 64-byte half-line
 // of gate rows (r < 4) and one of up rows (r >= 4), whose other halves the
-// XCD-adjacent item reads.  x changes with the group, so the wave stages its x
-// row in LDS once (per 32-element chunk: the 16 bf16 pairs matched to the
-// nibble pairs, and the chunk's sum) and each lane reads the chunk of its
-// (g, h) per step.  Per lane the affine chunk arithmetic is qmv64_kernel's;
-// the row sums close over the eight group slots with three DPP steps.
-template <int NV, int RG, int PER = 0, bool SH = false>
-__global__ __launch_bounds__(64) void qmv64_paired_lines_kernel(QmvArgs a) {
+// XCD-adjacent item reads.  x changes with the group, so the block's W waves
+// (of one pair) stage its x row in LDS once (per 32-element chunk: the 16 bf16
+// pairs matched to the nibble pairs, and the chunk's sum) and each lane reads
+// the chunk of its (g, h) per step.  Per lane the affine chunk arithmetic is
+// qmv64_kernel's; the row sums close over the eight group slots with one DPP
+// step and two lane swaps.
+template <int NV, int RG, int W, int PER = 0, bool SH = false>
+__global__ __launch_bounds__(64 * W) void qmv64_paired_lines_kernel(QmvArgs a) {
   static_assert(RG == 4 || RG == 8, "four or eight indices per wave");
   constexpr int NCH = 64 * NV;   // 32-element chunks of x
   constexpr int NP = 4 * NV;     // group steps per lane: g = 8p + s
   constexpr int NJ = RG / 4;     // row halves a lane reads: both (RG = 8) or its own (RG = 4)
   __shared__ uint4 xl[4][NCH];   // quarter q of chunk c at xl[q][c]: 16-byte reads of 8 chunks hit distinct banks
   __shared__ float xsum[NCH];
-  const int lane = threadIdx.x;
-  const int r = lane >> 3, sl = lane & 7;
+  const int lane = threadIdx.x % 64;
+  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+  const int r = lane & 7, sl = lane >> 3;  // rows fastest: eight neighbouring lanes read one line
   const int jr = RG == 8 ? 0 : r >> 2;        // RG = 4: the lane's half (gate or up)
   const int rr = RG == 8 ? r : (r & 3);       // row within the wave's RG rows
   const uint32_t item = xcd_item(blockIdx.x, gridDim.x);
   const uint32_t pr = fast_div(item, a.blk_div);
-  const int i0 = (int)(item - pr * a.blk_div.d) * RG;
+  const int i0 = ((int)(item - pr * a.blk_div.d) * W + wave) * RG;
   const uint32_t xr = fast_div(pr, a.x_divf);
   // the expert id is requested before x; a top-k selection goes after x's loads
   PairTopk<PER> ts;
   int e = 0;
   if constexpr (PER == 0) e = pair_expert<PER>(a, pr, xr, false, ts);
   const uint16_t* xrow = a.x + (int64_t)xr * a.x_stride;
-  uint4 xa[NV][4];
+  // x: a whole chunk per lane (W = 1), or the block's threads one 16-byte piece
+  // (quarter threadIdx.x % 4 of a chunk) at a time
+  constexpr int NX = W == 1 ? NV : 4 * NCH / (64 * W);
+  uint4 xa[NX][W == 1 ? 4 : 1];
 #pragma unroll
-  for (int v = 0; v < NV; ++v)
+  for (int v = 0; v < NX; ++v) {
+    if constexpr (W == 1) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) xa[v][q] = reinterpret_cast<const uint4*>(xrow + v * 2048 + lane * 32)[q];
+      for (int q = 0; q < 4; ++q) xa[v][q] = reinterpret_cast<const uint4*>(xrow + v * 2048 + lane * 32)[q];
+    } else {
+      xa[v][0] = reinterpret_cast<const uint4*>(xrow)[v * 64 * W + threadIdx.x];
+    }
+  }
   if constexpr (PER > 0) e = pair_expert<PER, SH>(a, pr, xr, i0 == 0, ts);
   const bool shared = SH && e == kSharedSlot;  // wave-uniform
   const uint32_t* wbase = shared ? a.sh_w : a.w;
@@ -1074,28 +1102,33 @@ __global__ __launch_bounds__(64) void qmv64_paired_lines_kernel(QmvArgs a) {
         wv[pp][h][jj] = load_nt(reinterpret_cast<const uint4*>(wbase) + ((chunk * 2 + jr + jj) * 2 + h) * 32 + l0 + rr);
       }
   pair_topk_store<PER, SH>(a, xr, ts);  // while the weights are in flight
-  if (SH && shared && i0 == 0) shared_score_store<NV>(a, xr, xa);
-  // stage x: lane l writes chunk v*64 + l (elements v*2048 + 32l ..)
+  if (SH && shared && i0 == 0) shared_score_store<NV>(a, xr, xrow);
+  // stage x: chunk c's quarter q at xl[q][c], its pairs matched to the nibble pairs
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    uint32_t pw[16];
-    float sum = 0.f;
+  for (int v = 0; v < NX; ++v) {
+    if constexpr (W == 1) {
+      XChunk xc;
+      pair_x_chunk(xa[v], xc);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint4 t = xa[v][q];
-      pw[4 * q + 0] = (t.x & 0xFFFFu) | (t.z << 16);
-      pw[4 * q + 1] = (t.x >> 16) | (t.z & 0xFFFF0000u);
-      pw[4 * q + 2] = (t.y & 0xFFFFu) | (t.w << 16);
-      pw[4 * q + 3] = (t.y >> 16) | (t.w & 0xFFFF0000u);
-      sum += ((bf16lo(t.x) + bf16hi(t.x)) + (bf16lo(t.y) + bf16hi(t.y))) +
-             ((bf16lo(t.z) + bf16hi(t.z)) + (bf16lo(t.w) + bf16hi(t.w)));
+      for (int q = 0; q < 4; ++q)
+        xl[q][v * 64 + lane] = make_uint4(xc.p[4 * q], xc.p[4 * q + 1], xc.p[4 * q + 2], xc.p[4 * q + 3]);
+      xsum[v * 64 + lane] = xc.sum;
+    } else {
+      const int u = v * 64 * W + threadIdx.x, c = u / 4, q = u % 4;
+      uint4 pw;
+      const float sq = pair_x_quarter(xa[v][0], pw);
+      xl[q][c] = pw;
+      // the chunk's sum over its four lanes, in quarter order
+      const float sum = ((quad_lane<0x00>(sq) + quad_lane<0x55>(sq)) + quad_lane<0xAA>(sq)) + quad_lane<0xFF>(sq);
+      if (q == 0) xsum[c] = sum;
     }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) xl[q][v * 64 + lane] = make_uint4(pw[4 * q], pw[4 * q + 1], pw[4 * q + 2], pw[4 * q + 3]);
-    xsum[v * 64 + lane] = sum;
   }
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the staged x is visible to the wave
-  __builtin_amdgcn_wave_barrier();
+  if constexpr (W == 1) {
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the staged x is visible to the wave
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
   const uint32_t mv = magic_vgpr();
   float acc[NJ];
 #pragma unroll
@@ -1123,14 +1156,12 @@ __global__ __launch_bounds__(64) void qmv64_paired_lines_kernel(QmvArgs a) {
   }
   float gate, up;
   if constexpr (RG == 8) {
-    gate = sum8(acc[0]);
-    up = sum8(acc[1]);
+    gate = sum_slots(acc[0]);
+    up = sum_slots(acc[1]);
   } else {
-    // lanes 8r, r < 4: gate row r; r >= 4: up row r - 4, 32 lanes above
-    const float t = sum8(acc[0]);
-    auto sw = __builtin_amdgcn_permlane32_swap(as_u(t), as_u(t), false, false);
-    gate = t;
-    up = as_f(sw[1]);
+    // r < 4: gate row r; r >= 4: up row r - 4, four lanes above (row_ror:4 of a value of period 8)
+    gate = sum_slots(acc[0]);
+    up = as_f(__builtin_amdgcn_update_dpp(0, as_u(gate), 0x124, 0xf, 0xf, false));
   }
   if (sl == 0 && r < RG)
     a.out[(int64_t)pr * a.n_out + i0 + r] = (uint16_t)f32_to_bf16(swiglu_f32(gate, up));
@@ -1627,30 +1658,39 @@ int launch_qmv_paired_rg(QmvArgs a, hipStream_t st) {
 
 // K = 2048 n: RG indices per wave for n <= 2, four above (16 rows x n 16-byte
 // code loads per lane would pass 256 registers)
-// Indices per wave of the line-read paired kernel.
-// (four measured faster than eight at the decode shapes: 5.7 against 6.1 us at
-// one token x top-10 of 256 experts, hidden 2048; twice the waves in flight)
-#ifndef QMOE_PAIRED_LINES_RG
+// Indices per wave of the line-read paired kernel for one token.
 #define QMOE_PAIRED_LINES_RG 4
-#endif
+
+template <int RG, int W, int PER, bool SH>
+int launch_qmv_lines(const QmvArgs& a, hipStream_t st) {
+  QmvArgs b = a;
+  const int64_t nblk = a.n_out / (RG * W);
+  const int64_t blocks = a.n_pairs * nblk;
+  if (blocks <= 0) return QMOE_OK;
+  if (blocks > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "grid too large");
+  b.blk_div = make_fastdiv((uint32_t)nblk);
+  b.x_divf = make_fastdiv((uint32_t)a.x_div);
+  const dim3 grid((unsigned)blocks), block(64 * W);
+  if (a.K == 2048) qmv64_paired_lines_kernel<1, RG, W, PER, SH><<<grid, block, 0, st>>>(b);
+  else qmv64_paired_lines_kernel<2, RG, W, PER, SH><<<grid, block, 0, st>>>(b);
+  return qmoe::launch_status("qmv64_paired_lines_kernel");
+}
 
 template <int PER = 0, bool SH = false>
 int launch_qmv_paired(const QmvArgs& a, hipStream_t st) {
   if (a.K <= 4096) {
     // line reads with x staged in LDS (K = 2048 or 4096)
-    constexpr int RG = QMOE_PAIRED_LINES_RG;
-    QmvArgs b = a;
-    const int64_t nblk = a.n_out / RG;
-    const int64_t blocks = a.n_pairs * nblk;
-    if (blocks <= 0) return QMOE_OK;
-    if (blocks > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "grid too large");
     if (a.x_div < 1 || a.x_div > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_INVALID, "top_k out of range");
-    b.blk_div = make_fastdiv((uint32_t)nblk);
-    b.x_divf = make_fastdiv((uint32_t)a.x_div);
-    dim3 grid((unsigned)blocks), block(64);
-    if (a.K == 2048) qmv64_paired_lines_kernel<1, RG, PER, SH><<<grid, block, 0, st>>>(b);
-    else qmv64_paired_lines_kernel<2, RG, PER, SH><<<grid, block, 0, st>>>(b);
-    return qmoe::launch_status("qmv64_paired_lines_kernel");
+    // One token: four indices per wave (twice the waves in flight).  More:
+    // eight, whose x staging and selection are half as much work per weight
+    // byte, four waves to a block (they share the staged x) once the blocks
+    // fill the CUs one and a half times.  gate_up with top-k, 256 experts x
+    // top-10, hidden 2048, us per call at 1 / 2 / 3 / 4 / 6 tokens: four indices
+    // 6.2 / 8.9 / 11.8 / 15.0 / 20.6, eight 6.7 / 8.1 / 10.3 / 12.2 / 16.0, eight in
+    // four-wave blocks - / 8.8 / 10.0 / 11.9 / 15.0 (floor at four: 9).
+    if (a.n_pairs <= a.x_div) return launch_qmv_lines<QMOE_PAIRED_LINES_RG, 1, PER, SH>(a, st);
+    if (8 * (a.n_pairs * (a.n_out / 32)) < 3 * (int64_t)simd_count()) return launch_qmv_lines<8, 1, PER, SH>(a, st);
+    return launch_qmv_lines<8, 4, PER, SH>(a, st);
   }
   return launch_qmv_paired_rg<4, PER, SH>(a, st);
 }
