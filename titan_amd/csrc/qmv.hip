@@ -1658,7 +1658,7 @@ int launch_qmv_paired_rg(QmvArgs a, hipStream_t st) {
 
 // K = 2048 n: RG indices per wave for n <= 2, four above (16 rows x n 16-byte
 // code loads per lane would pass 256 registers)
-// Indices per wave of the line-read paired kernel for one token.
+// Indices per wave of the line-read paired kernel where waves in flight are few.
 #define QMOE_PAIRED_LINES_RG 4
 
 template <int RG, int W, int PER, bool SH>
@@ -1681,14 +1681,17 @@ int launch_qmv_paired(const QmvArgs& a, hipStream_t st) {
   if (a.K <= 4096) {
     // line reads with x staged in LDS (K = 2048 or 4096)
     if (a.x_div < 1 || a.x_div > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_INVALID, "top_k out of range");
-    // One token: four indices per wave (twice the waves in flight).  More:
+    // Four indices per wave while eight would leave SIMDs without a wave (one
+    // token; one expert of few tokens): twice the waves in flight.  Beyond,
     // eight, whose x staging and selection are half as much work per weight
     // byte, four waves to a block (they share the staged x) once the blocks
     // fill the CUs one and a half times.  gate_up with top-k, 256 experts x
     // top-10, hidden 2048, us per call at 1 / 2 / 3 / 4 / 6 tokens: four indices
     // 6.2 / 8.9 / 11.8 / 15.0 / 20.6, eight 6.7 / 8.1 / 10.3 / 12.2 / 16.0, eight in
-    // four-wave blocks - / 8.8 / 10.0 / 11.9 / 15.0 (floor at four: 9).
-    if (a.n_pairs <= a.x_div) return launch_qmv_lines<QMOE_PAIRED_LINES_RG, 1, PER, SH>(a, st);
+    // four-wave blocks - / 8.8 / 10.0 / 11.9 / 15.0 (floor at four: 9); hidden
+    // 4096, 128 experts x top-8, 2 / 4 / 16 tokens 13.3 / 22.7 / 78.5 against 12.0 /
+    // 17.1 / 52.8; one expert, 2 / 6 / 16 tokens 3.4 / 4.6 / 8.9 against 4.3 / 5.3 / 6.8.
+    if (a.n_pairs * (a.n_out / 8) < simd_count()) return launch_qmv_lines<QMOE_PAIRED_LINES_RG, 1, PER, SH>(a, st);
     if (8 * (a.n_pairs * (a.n_out / 32)) < 3 * (int64_t)simd_count()) return launch_qmv_lines<8, 1, PER, SH>(a, st);
     return launch_qmv_lines<8, 4, PER, SH>(a, st);
   }
