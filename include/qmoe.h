@@ -64,6 +64,18 @@ int qmoe_dequantize(const uint32_t* w, const uint16_t* scales,
                     const uint16_t* biases, int64_t rows, int64_t K,
                     int group_size, int bits, uint16_t* out, void* stream);
 
+/* out[i] = src[rows[i] / div] over rows of row_bytes bytes (a multiple of 16):
+ * the sorted rows of a layer's tokens (div = top_k) and their un-sort (div = 1),
+ * switch_layers.py:13-25.  Indices are clamped to [0, n_src). */
+int qmoe_gather_rows(const void* src, int64_t n_src, const int32_t* rows,
+                     int64_t n, int32_t div, int64_t row_bytes, void* out,
+                     void* stream);
+
+/* h [rows, I] = silu(gate) * up of gate_up [rows, 2I] (gate first), fp32, one
+ * rounding (activations.py:9-11).  I % 8 == 0. */
+int qmoe_swiglu(const uint16_t* gate_up, int64_t rows, int64_t I, uint16_t* h,
+                void* stream);
+
 /* --------------------------------------------------------------- routing --
  * Replaces _gather_sort (titan/adapters/mlx/vendor/mlx_lm/models/
  * switch_layers.py:13-18) together with build_tiles

@@ -74,6 +74,8 @@ SIGNATURES: dict[str, tuple] = {
     "qmoe_gather_qmm_sorted_tiles_shared": (INT, [P, P, I64, I64, P, P, P, P, I32, I64, INT, P, P, P, P, I64, P, P]),
     "qmoe_weighted_sum_shared": (INT, [P, P, P, I64, I64, I64, INT, P, P, P]),
     "qmoe_router_topk_shared": (INT, [P, I64, I64, I64, INT, P, P, I64, P, P, P]),
+    "qmoe_gather_rows": (INT, [P, I64, P, I64, I32, I64, P, P]),
+    "qmoe_swiglu": (INT, [P, I64, I64, P, P]),
     "qmoe_quantize_act_int8": (INT, [P, I64, I64, P, P, P]),
     "qmoe_gather_qmm_int8_sorted": (INT, [P, P, P, I64, I64, P, P, P, I32, I64, INT, INT, P, P, P, P,
                                           I64, P, P]),

@@ -159,3 +159,68 @@ extern "C" int qmoe_repack_tiles(const uint32_t* w, const uint16_t* scales, cons
   repack_sb_kernel<<<dim3((unsigned)bw), dim3(256), 0, st>>>(scales, biases, sb, words, N, (int)NC, (int)G);
   return qmoe::launch_status("repack_sb_kernel");
 }
+
+namespace {
+
+// out[i] = src[rows[i] / div], 16 bytes per thread.  Bound by memory: each row
+// written once and (div > 1) read div times, from the caches after the first.
+__global__ __launch_bounds__(256) void gather_rows_kernel(const i32x4_t* __restrict__ src, int64_t n_src,
+                                                          const int32_t* __restrict__ rows, int64_t n, uint32_t div,
+                                                          int64_t units, i32x4_t* __restrict__ out) {
+  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (u >= n * units) return;
+  const int64_t i = u / units, c = u - i * units;
+  const int64_t r = min((int64_t)((uint32_t)max(rows[i], 0) / div), n_src - 1);
+  __builtin_nontemporal_store(src[r * units + c], out + u);
+}
+
+// h[r, i] = silu(gu[r, i]) * gu[r, I + i] in fp32 with one rounding
+// (activations.py:9-11), eight elements per thread.
+__global__ __launch_bounds__(256) void swiglu_kernel(const uint4* __restrict__ gu, int64_t n, int units,
+                                                     uint4* __restrict__ h) {
+  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (u >= n) return;
+  const int64_t r = u / units, c = u - r * units;
+  const uint4 g = gu[r * 2 * units + c], v = gu[(r * 2 + 1) * units + c];
+  const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, vw[4] = {v.x, v.y, v.z, v.w};
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float g0 = bf16lo(gw[i]), g1 = bf16hi(gw[i]);
+    o[i] = pack_bf16x2(g0 * (1.0f / (1.0f + expf(-g0))) * bf16lo(vw[i]),
+                       g1 * (1.0f / (1.0f + expf(-g1))) * bf16hi(vw[i]));
+  }
+  h[u] = make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+}  // namespace
+
+extern "C" int qmoe_gather_rows(const void* src, int64_t n_src, const int32_t* rows, int64_t n, int32_t div,
+                                int64_t row_bytes, void* out, void* stream) {
+  if (n_src < 0 || n < 0 || div <= 0 || row_bytes < 0) return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
+  if (n == 0 || row_bytes == 0) return QMOE_OK;
+  if (n_src == 0) return qmoe::fail(QMOE_ERR_INVALID, "no source rows");
+  if (!src || !rows || !out) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+  if (row_bytes % 16 || !qmoe::aligned16(src) || !qmoe::aligned16(out))
+    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "rows must be multiples of 16 bytes, 16-byte aligned");
+  const int64_t units = row_bytes / 16;
+  const int64_t blocks = n > 0x7FFFFFFF / units * 256 ? -1 : (n * units + 255) / 256;
+  if (blocks < 0 || blocks > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "too many rows");
+  gather_rows_kernel<<<dim3((unsigned)blocks), dim3(256), 0, qmoe::as_stream(stream)>>>(
+      static_cast<const i32x4_t*>(src), n_src, rows, n, (uint32_t)div, units, static_cast<i32x4_t*>(out));
+  return qmoe::launch_status("gather_rows_kernel");
+}
+
+extern "C" int qmoe_swiglu(const uint16_t* gate_up, int64_t rows, int64_t I, uint16_t* h, void* stream) {
+  if (rows < 0 || I < 0) return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
+  if (rows == 0 || I == 0) return QMOE_OK;
+  if (!gate_up || !h) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+  if (I % 8 || I > 0x7FFFFFFF || !qmoe::aligned16(gate_up) || !qmoe::aligned16(h))
+    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "I=%lld: must be a multiple of 8, the tensors 16-byte aligned", (long long)I);
+  const int64_t units = I / 8;
+  const int64_t blocks = rows > 0x7FFFFFFF / units * 256 ? -1 : (rows * units + 255) / 256;
+  if (blocks < 0 || blocks > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "too many rows");
+  swiglu_kernel<<<dim3((unsigned)blocks), dim3(256), 0, qmoe::as_stream(stream)>>>(
+      reinterpret_cast<const uint4*>(gate_up), rows * units, (int)units, reinterpret_cast<uint4*>(h));
+  return qmoe::launch_status("swiglu_kernel");
+}

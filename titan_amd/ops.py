@@ -222,6 +222,29 @@ def route_block(idx: torch.Tensor, num_experts: int, shared: bool = False):
     return x_rows, inv, TileTable(offsets, trow, texp, nt, mt, tr, E, n + extra)
 
 
+def gather_rows(x: torch.Tensor, rows: torch.Tensor, div: int = 1) -> torch.Tensor:
+    """x[rows // div] for contiguous x [R, D] and int32 ``rows`` [n]."""
+    _dev(x, "x")
+    x = _ready(x)
+    if x.dim() != 2:
+        raise ValueError(f"x must be [R, D], got {tuple(x.shape)}")
+    rows = _i32(rows, "rows", x.device)
+    n = rows.numel()
+    out = torch.empty(n, x.shape[1], dtype=x.dtype, device=x.device)
+    _lib.call("qmoe_gather_rows", x.data_ptr(), x.shape[0], rows.data_ptr(), n, div, x.shape[1] * x.element_size(),
+              out.data_ptr(), _stream(x))
+    return out
+
+
+def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up of a fused [.., 2I] projection, gate first: fp32, one rounding."""
+    gate_up = _bf16(gate_up, "gate_up")
+    I = gate_up.shape[-1] // 2
+    h = torch.empty(*gate_up.shape[:-1], I, dtype=torch.bfloat16, device=gate_up.device)
+    _lib.call("qmoe_swiglu", gate_up.data_ptr(), h.numel() // I if I else 0, I, h.data_ptr(), _stream(gate_up))
+    return h
+
+
 # ------------------------------------------------------------- gather_qmm
 
 
@@ -811,7 +834,7 @@ __all__ = [
     "repack_tiles", "gather_qmm_sorted_tiles", "gather_qmm_int8_sorted_tiles", "router_topk", "router_logits", "gather_qmm_swiglu_sorted_tiles", "swiglu_pair_order", "gather_qmv_tiles", "gate_up_silu_tiles",
     "down_wsum_tiles", "gate_up_silu_tiles_topk", "gate_up_silu_tiles_topk_shared", "down_wsum_tiles_shared",
     "route_block", "gather_qmm_sorted_tiles_shared", "moe_weighted_sum_shared", "router_topk_shared",
-    "max_tiles", "tile_rows", "unpack", "dequantize", "gather_qmv", "gather_qmm_sorted", "gather_qmm",
+    "gather_rows", "swiglu", "max_tiles", "tile_rows", "unpack", "dequantize", "gather_qmv", "gather_qmm_sorted", "gather_qmm",
     "gemm_supported", "quantized_matmul", "gate_up_silu", "down_wsum", "moe_weighted_sum",
     "quantize_act_int8", "gather_qmm_int8_sorted",
 ]
