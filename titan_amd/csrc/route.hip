@@ -457,9 +457,24 @@ __global__ __launch_bounds__(kScanThreads) void tiles_from_sorted_kernel(const i
                                                                          int32_t* __restrict__ tile_exp,
                                                                          int32_t* __restrict__ ntiles,
                                                                          int64_t max_tiles) {
+  // first row whose id >= e, in two levels: a search over every stride-th id,
+  // read by the block at once, then one inside a stride.  (Each step of a
+  // search in memory is a dependent read, 15 of them at 20,480 rows: 4.8 -> 4.5
+  // us per call in a graph, where the ids are in the caches.)
   __shared__ int lds[kScanThreads];
+  const int64_t stride = (n + kScanThreads - 1) / kScanThreads;
+  const int ns = n > 0 ? (int)((n + stride - 1) / stride) : 0;  // samples
+  if ((int)threadIdx.x < ns) lds[threadIdx.x] = sorted_ids[threadIdx.x * stride];
+  __syncthreads();
   for (int e = threadIdx.x; e <= E; e += kScanThreads) {
-    int64_t lo = 0, hi = n;  // first row whose id >= e
+    int a = 0, b = ns;
+    while (a < b) {
+      const int mid = (a + b) >> 1;
+      if (lds[mid] < e) a = mid + 1;
+      else b = mid;
+    }
+    // sample a is the first with id >= e: the row lies past sample a - 1
+    int64_t lo = a > 0 ? (a - 1) * stride + 1 : 0, hi = min(a * stride, n);
     while (lo < hi) {
       const int64_t mid = (lo + hi) >> 1;
       if (sorted_ids[mid] < e) lo = mid + 1;
