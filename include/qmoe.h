@@ -304,7 +304,20 @@ int qmoe_moe_gate_up_swiglu_tiles_topk(const uint16_t* x, const float* logits,
                                        int64_t I, uint16_t* h, int32_t* idx,
                                        float* scores, void* stream);
 
-/* The same two decode launches with the layer's sigmoid-gated shared expert
+/* qmoe_moe_gate_up_swiglu with the router's top-k folded in the same way, over
+ * MLX-layout weights: h, idx and scores equal qmoe_router_topk followed by
+ * qmoe_moe_gate_up_swiglu (its four-index kernel).  Requires K = 2048 or 4096,
+ * 4-bit codes, group 64, 16-byte aligned scales and biases, top_k <= 64 and
+ * num_experts <= 1024. */
+int qmoe_moe_gate_up_swiglu_topk(const uint16_t* x, const float* logits,
+                                 int norm, int64_t T, int64_t top_k, int64_t K,
+                                 const uint32_t* w, const uint16_t* scales,
+                                 const uint16_t* biases, int32_t num_experts,
+                                 int64_t I, int group_size, int bits,
+                                 uint16_t* h, int32_t* idx, float* scores,
+                                 void* stream);
+
+/* The two tile-layout decode launches with the layer's sigmoid-gated shared expert
  * (qwen3_5_moe/language.py:81-89: sigmoid(x . sh_gate) * SwiGLU-MLP(x)) as one
  * more slot per token: h [T, top_k + 1, I], idx and scores [T, top_k + 1], the
  * last slot the shared expert's (id num_experts, score sigmoid(x . sh_gate) in
@@ -420,6 +433,13 @@ int qmoe_router_topk_shared(const float* logits, int64_t T, int64_t E,
                             int64_t k, int norm, const uint16_t* x,
                             const uint16_t* gate, int64_t K, int32_t* idx,
                             float* scores, void* stream);
+
+/* out[t, :] = y[t, :] + sigmoid(x[t] . gate) * ys[t, :] in fp32, one bf16
+ * rounding: the shared expert's part of a block whose shared expert runs apart
+ * (qwen3_5_moe/language.py:81-89).  x [T, K], gate [K], the rest [T, D]. */
+int qmoe_shared_combine(const uint16_t* y, const uint16_t* ys,
+                        const uint16_t* x, const uint16_t* gate, int64_t T,
+                        int64_t K, int64_t D, uint16_t* out, void* stream);
 
 /* Router logits in fp32 from an affine-quantized router weight [E, K*bits/32]
  * (replaces the fused router's quantized matvec,

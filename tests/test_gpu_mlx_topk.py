@@ -1,0 +1,55 @@
+"""The MLX-layout decode gate_up that selects its experts, against the router
+top-k and the kernel that takes ids."""
+
+import pytest
+import torch
+
+from titan_amd import ops
+from titan_amd.moe_block import SharedExpert, SparseMoeBlock
+
+pytestmark = pytest.mark.gpu
+
+
+def _quant(g, lead, K, dev):
+    w = torch.randint(-2 ** 31, 2 ** 31, (*lead, K // 8), dtype=torch.int32, device=dev, generator=g)
+    s = (0.004 + 0.004 * torch.rand(*lead, K // 64, device=dev, generator=g)).to(torch.bfloat16)
+    return w, s, (-7.5 * s.float()).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("T,k,E,K,I", [(1, 8, 128, 2048, 768), (3, 1, 1, 2048, 6), (16, 64, 64, 2048, 33),
+                                       (2, 10, 600, 4096, 64), (5, 20, 256, 4096, 12)])
+def test_gate_up_topk_over_mlx_weights(dev, T, k, E, K, I, norm):
+    print(f"[case] MLX gate_up with top-k T={T} k={k} E={E} K={K} I={I} norm={norm}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T + k + E)
+    w = _quant(g, (E, 2 * I), K, dev)
+    x = torch.randn(T, K, device=dev, generator=g).to(torch.bfloat16)
+    lg = torch.randn(T, E, device=dev, generator=g)
+    lg[:, ::3] = lg[:, ::3].round()  # ties among them
+    h, idx, sc = ops.gate_up_silu_topk(x, *w, lg, k, norm)
+    idx0, sc0 = ops.router_topk(lg, k, norm)
+    assert torch.equal(idx, idx0) and torch.equal(sc, sc0)
+    assert torch.equal(h, ops.gate_up_silu(x, *w, idx0))
+
+
+@pytest.mark.parametrize("T", [1, 3, 7])
+@pytest.mark.parametrize("resident,I,shared", [("tiles", 768, False), ("both", 512, False), ("tiles", 768, True),
+                                               ("both", 512, True)])
+def test_block_decode_over_mlx_weights(dev, T, resident, I, shared):
+    print(f"[case] MLX-layout block decode T={T} {resident} I={I} shared={shared}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T + I)
+    E, H, k = 24, 2048, 8
+    gu, dn = _quant(g, (E, 2 * I), H, dev), _quant(g, (E, H), I, dev)
+    sgu, sdn = _quant(g, (1, 2 * I), H, dev), _quant(g, (1, H), I, dev)
+    gate = (torch.randn(1, H, device=dev, generator=g) * H ** -0.5).to(torch.bfloat16)
+    router = (torch.randn(E, H, device=dev, generator=g) * H ** -0.5).to(torch.bfloat16)
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    block = SparseMoeBlock(router, gu, dn, k, resident=resident, shared=SharedExpert(sgu, sdn, gate) if shared else None)
+    y = block(x)
+    idx, sc = block.route(x)
+    ref = block.experts(x, idx, sc)
+    if not shared:
+        assert torch.equal(y, ref)
+    else:  # one rounding of the sum where the parts' sum has two
+        both = ref.double() + block.shared_expert(x).double()
+        assert bool(((y.double() - both).abs() <= 2.0 ** -7 * both.abs().max()).all())

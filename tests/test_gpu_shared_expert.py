@@ -180,3 +180,35 @@ def test_topk_with_shared_score(dev, T, E, K):
         z = x.double() @ gate.double().t()
         bound = 0.25 * K * 2.0 ** -24 * (x.double().abs() @ gate.double().abs().t()) + 4 * 2.0 ** -24
         assert bool(((sc[:, k:].double() - torch.sigmoid(z)).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("T,K,D", [(1, 8, 8), (5, 2048, 2048), (300, 520, 4104)])
+def test_shared_combine(dev, T, K, D):
+    print(f"[case] shared combine T={T} K={K} D={D}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T + K)
+    x, y, ys = (torch.randn(T, n, device=dev, generator=g).to(torch.bfloat16) for n in (K, D, D))
+    gate = (torch.randn(1, K, device=dev, generator=g) * K ** -0.5).to(torch.bfloat16)
+    out = ops.shared_combine(y, ys, x, gate).double()
+    s = torch.sigmoid(x.double() @ gate.double().t())
+    ref = y.double() + s * ys.double()
+    # one bf16 rounding; the score's fp32 sum is within K * 2^-24 of sum |x w|, its sigmoid's slope at most 1/4
+    off = 0.25 * K * 2.0 ** -24 * (x.double().abs() @ gate.double().abs().t()) + 4 * 2.0 ** -24
+    assert bool(((out - ref).abs() <= 2.0 ** -8 * ref.abs() + off * ys.double().abs() + 2.0 ** -23 * y.double().abs()).all())
+
+
+@pytest.mark.parametrize("n", [1, 5, 1023, 1024, 1025, 2047, 20480, 70001])
+@pytest.mark.parametrize("E", [1, 7, 256, 1500])
+def test_tiles_of_sorted_ids(dev, n, E):
+    """Offsets and tiles over sorted ids at the edges of the sampled search."""
+    print(f"[case] tiles of sorted ids n={n} E={E}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(n + E)
+    for ids in (torch.randint(0, E, (n,), device=dev, generator=g), torch.full((n,), E - 1, device=dev),
+                torch.zeros(n, dtype=torch.int64, device=dev)):
+        ids = ids.sort()[0].to(torch.int32)
+        t = ops.build_tiles(ids, E)
+        edges = torch.searchsorted(ids.long(), torch.arange(E + 1, device=dev))
+        assert torch.equal(t.offsets.long(), edges)
+        per = (edges[1:] - edges[:-1] + 127) // 128
+        assert int(t.ntiles) == int(per.sum())
+        exp = torch.repeat_interleave(torch.arange(E, device=dev), per)
+        assert torch.equal(t.tile_exp[:exp.numel()].long(), exp)

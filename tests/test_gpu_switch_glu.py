@@ -69,5 +69,6 @@ def test_layer_over_its_kernels_and_without(dev, T, how, monkeypatch):
     monkeypatch.setattr(switch_layers, "_plain", lambda t, width: False)
     ref = layer(x, idx)
     assert y.shape == ref.shape == (T, k, K)
+    y, ref = y.detach(), ref.detach()
     err = (y.double() - ref.double()).norm() / ref.double().norm()
     assert float(err) < 2.0 ** -9  # single ULPs of h, seldom

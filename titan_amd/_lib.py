@@ -76,6 +76,8 @@ SIGNATURES: dict[str, tuple] = {
     "qmoe_router_topk_shared": (INT, [P, I64, I64, I64, INT, P, P, I64, P, P, P]),
     "qmoe_gather_rows": (INT, [P, I64, P, I64, I32, I64, P, P]),
     "qmoe_swiglu": (INT, [P, I64, I64, P, P]),
+    "qmoe_shared_combine": (INT, [P, P, P, P, I64, I64, I64, P, P]),
+    "qmoe_moe_gate_up_swiglu_topk": (INT, [P, P, INT, I64, I64, I64, P, P, P, I32, I64, INT, INT, P, P, P, P]),
     "qmoe_quantize_act_int8": (INT, [P, I64, I64, P, P, P]),
     "qmoe_gather_qmm_int8_sorted": (INT, [P, P, P, I64, I64, P, P, P, I32, I64, INT, INT, P, P, P, P,
                                           I64, P, P]),

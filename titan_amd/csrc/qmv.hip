@@ -470,7 +470,10 @@ namespace {
 #define QMV_AFTER(v)
 #endif
 
-template <int NV, int TL, int MODE, int RG, int GS, bool GATHER, bool XROWS, int BITS>
+//
+// PER > 0 (MODE 1): the expert is chosen here from the token's router logits
+// (pair_expert), once x has been asked for.
+template <int NV, int TL, int MODE, int RG, int GS, bool GATHER, bool XROWS, int BITS, int PER = 0>
 __device__ __forceinline__ void qmv64_rows(const QmvArgs& a) {
   QMV_STAMP(ts_entry);
   // K = 2048 * NV + 512 * TL: NV whole chunks of 64 lanes x 32 elements and,
@@ -494,9 +497,10 @@ __device__ __forceinline__ void qmv64_rows(const QmvArgs& a) {
   const int n0 = (int)(bid - r * a.blk_div.d) * OUTS;
   QMV_AFTER_S(r);
   QMV_STAMP(ts_args);
-  int e = GATHER ? a.experts[r] : 0;
+  int e = GATHER && PER == 0 ? a.experts[r] : 0;
   const uint32_t xr = XROWS ? (uint32_t)a.x_rows[r] : fast_div(r, a.x_divf);
   const uint16_t* xrow = a.x + (int64_t)xr * a.x_stride;
+  PairTopk<PER> ts;
   const bool tail_lane = lane < 16 * TL;  // holds data in the tail chunk
   uint4 xa[NC][4];
 #pragma unroll
@@ -506,6 +510,7 @@ __device__ __forceinline__ void qmv64_rows(const QmvArgs& a) {
       xa[v][q] = (v < NV || tail_lane) ? reinterpret_cast<const uint4*>(xrow + v * 2048 + lane * 32)[q]
                                        : make_uint4(0u, 0u, 0u, 0u);
 
+  if constexpr (PER > 0) e = pair_expert<PER>(a, r, xr, n0 == 0, ts);
   e = min(max(e, 0), a.num_experts - 1);
   QMV_AFTER_S(e);
   QMV_STAMP(ts_id);
@@ -541,6 +546,7 @@ __device__ __forceinline__ void qmv64_rows(const QmvArgs& a) {
         for (int c = 0; c < WPC; ++c)
           wv[g][i][v][c] = (v < NV || tail_lane) ? load_nt(p + WPC * v * 64 + c) : make_uint4(0u, 0u, 0u, 0u);
     }
+  pair_topk_store<PER>(a, xr, ts);  // while the weights are in flight
   XChunk xc[NC];
 #pragma unroll
   for (int v = 0; v < NC; ++v) {
@@ -635,6 +641,11 @@ __device__ __forceinline__ void qmv64_rows(const QmvArgs& a) {
 template <int NV, int TL, int MODE, int RG, int GS, bool GATHER, bool XROWS>
 __global__ __launch_bounds__(64) void qmv64_kernel(QmvArgs a) {
   qmv64_rows<NV, TL, MODE, RG, GS, GATHER, XROWS, 4>(a);
+}
+// the fused gate_up form that selects its experts (group 64)
+template <int NV, int RG, int PER>
+__global__ __launch_bounds__(64) void qmv64_topk_kernel(QmvArgs a) {
+  qmv64_rows<NV, 0, 1, RG, 64, true, false, 4, PER>(a);
 }
 template <int NV, int RG, int GS, bool GATHER, bool XROWS>
 __global__ __launch_bounds__(64) void qmv64_kernel8(QmvArgs a) {
@@ -1978,6 +1989,45 @@ extern "C" int qmoe_moe_gate_up_swiglu_tiles_topk_shared(const uint16_t* x, cons
                                                          float* scores, void* stream) {
   return gate_up_tiles_topk<true>(x, logits, norm, T, top_k, K, wp, sb, num_experts, I, sh_wp, sh_sb, sh_gate, h, idx,
                                   scores, stream);
+}
+
+extern "C" int qmoe_moe_gate_up_swiglu_topk(const uint16_t* x, const float* logits, int norm, int64_t T,
+                                            int64_t top_k, int64_t K, const uint32_t* w, const uint16_t* scales,
+                                            const uint16_t* biases, int32_t num_experts, int64_t I, int group_size,
+                                            int bits, uint16_t* h, int32_t* idx, float* scores, void* stream) {
+  if (T < 0 || top_k <= 0 || I <= 0 || num_experts <= 0) return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
+  if (T == 0) return QMOE_OK;
+  if (!x || !w || !scales || !biases || !h || !idx || !scores) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+  int per = 0;
+  const int rc = check_topk(logits, top_k, num_experts, &per);
+  if (rc) return rc;
+  if (bits != 4 || group_size != 64 || (K != 2048 && K != 4096))
+    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "K=%lld, group %d, %d bits: takes K = 2048 or 4096, group 64, 4 bits",
+                      (long long)K, group_size, bits);
+  if (!qmoe::aligned16(x) || !qmoe::aligned16(w) || !qmoe::aligned16(scales) || !qmoe::aligned16(biases))
+    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "x and the weights must be 16-byte aligned");
+  if (I > 0x3FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "I too large");
+  constexpr int RG = QMOE_QMV_RG_GU;
+  const int64_t nblk = (I + RG - 1) / RG, blocks = T * top_k * nblk;
+  if (blocks > 0x7FFFFFFF) return qmoe::fail(QMOE_ERR_UNSUPPORTED, "grid too large");
+  QmvArgs a{x, K, nullptr, top_k, nullptr, T * top_k, (int)K, 64, w, scales, biases, num_experts, (int)I,
+            (int)(2 * I), h};
+  a.logits = logits;
+  a.topk_idx = idx;
+  a.topk_scores = scores;
+  a.topk_norm = norm ? 1 : 0;
+  a.blk_div = make_fastdiv((uint32_t)nblk);
+  a.x_divf = make_fastdiv((uint32_t)top_k);
+  const dim3 grid((unsigned)blocks), block(64);
+  hipStream_t st = qmoe::as_stream(stream);
+  if (K == 2048) {
+    if (per == 4) qmv64_topk_kernel<1, RG, 4><<<grid, block, 0, st>>>(a);
+    else qmv64_topk_kernel<1, RG, 16><<<grid, block, 0, st>>>(a);
+  } else {
+    if (per == 4) qmv64_topk_kernel<2, RG, 4><<<grid, block, 0, st>>>(a);
+    else qmv64_topk_kernel<2, RG, 16><<<grid, block, 0, st>>>(a);
+  }
+  return qmoe::launch_status("qmv64_topk_kernel");
 }
 
 #ifdef QMOE_QMV_STAMPS

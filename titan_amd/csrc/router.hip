@@ -318,3 +318,55 @@ extern "C" int qmoe_router_topk_shared(const float* logits, int64_t T, int64_t E
                                        float* scores, void* stream) {
   return launch_router_topk<true>(logits, T, E, k, norm, x, gate, K, idx, scores, stream);
 }
+
+namespace {
+
+// out[t] = y[t] + sigmoid(x[t] . gate) * ys[t] in fp32, one rounding: a shared
+// expert that has launches of its own (language.py:81-89).  One block per token.
+__global__ __launch_bounds__(256) void shared_combine_kernel(const uint16_t* __restrict__ y,
+                                                             const uint16_t* __restrict__ ys,
+                                                             const uint16_t* __restrict__ x,
+                                                             const uint16_t* __restrict__ gate, int K, int D,
+                                                             uint16_t* __restrict__ out) {
+  __shared__ float part[4];
+  const int64_t t = blockIdx.x;
+  const int tid = threadIdx.x;
+  const uint4* xp = reinterpret_cast<const uint4*>(x + t * K);
+  const uint4* gp = reinterpret_cast<const uint4*>(gate);
+  float z[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int u = tid; u < K / 8; u += 256) {
+    const uint4 xv = xp[u], gv = gp[u];
+    z[0] = dot2_bf16(xv.x, gv.x, z[0]);
+    z[1] = dot2_bf16(xv.y, gv.y, z[1]);
+    z[2] = dot2_bf16(xv.z, gv.z, z[2]);
+    z[3] = dot2_bf16(xv.w, gv.w, z[3]);
+  }
+  const float w = wave_sum((z[0] + z[1]) + (z[2] + z[3]));
+  if (tid % 64 == 0) part[tid / 64] = w;
+  __syncthreads();
+  const float s = 1.0f / (1.0f + expf(-((part[0] + part[1]) + (part[2] + part[3]))));
+  for (int u = tid; u < D / 8; u += 256) {
+    const uint4 a = reinterpret_cast<const uint4*>(y + t * D)[u], b = reinterpret_cast<const uint4*>(ys + t * D)[u];
+    const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      o[i] = pack_bf16x2(fmaf(s, bf16lo(bw[i]), bf16lo(aw[i])), fmaf(s, bf16hi(bw[i]), bf16hi(aw[i])));
+    reinterpret_cast<uint4*>(out + t * D)[u] = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
+}  // namespace
+
+extern "C" int qmoe_shared_combine(const uint16_t* y, const uint16_t* ys, const uint16_t* x, const uint16_t* gate,
+                                   int64_t T, int64_t K, int64_t D, uint16_t* out, void* stream) {
+  if (T < 0 || K <= 0 || D <= 0) return qmoe::fail(QMOE_ERR_INVALID, "bad sizes");
+  if (T == 0) return QMOE_OK;
+  if (!y || !ys || !x || !gate || !out) return qmoe::fail(QMOE_ERR_INVALID, "null pointer");
+  if (K % 8 || D % 8 || K > 0x7FFFFFFF || D > 0x7FFFFFFF || T > 0x7FFFFFFF)
+    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "K=%lld, D=%lld: must be multiples of 8", (long long)K, (long long)D);
+  if (!qmoe::aligned16(y) || !qmoe::aligned16(ys) || !qmoe::aligned16(x) || !qmoe::aligned16(gate) || !qmoe::aligned16(out))
+    return qmoe::fail(QMOE_ERR_UNSUPPORTED, "the tensors must be 16-byte aligned");
+  shared_combine_kernel<<<dim3((unsigned)T), dim3(256), 0, qmoe::as_stream(stream)>>>(y, ys, x, gate, (int)K, (int)D, out);
+  return qmoe::launch_status("shared_combine_kernel");
+}

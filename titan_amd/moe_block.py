@@ -9,6 +9,7 @@ engine/patches/decode-fusion/fused_kernels.py:232-371).
     decode  (T * k < 64, switch_layers.py:218):
         h   = silu(x W_gate^T) * (x W_up^T)          qmoe_moe_gate_up_swiglu_tiles[_topk]
         y   = sum_j sc_j * W_down[idx_j] h_j          qmoe_moe_down_wsum_tiles
+        (over the MLX tensors where those stay: qmoe_moe_gate_up_swiglu[_topk], qmoe_moe_down_wsum)
         (the _topk form selects idx and sc from the logits in-kernel, by the
         top-k's own code, and writes them for the down kernel, so the decode
         block is three launches)
@@ -145,6 +146,9 @@ class SparseMoeBlock:
                                                                                group_size, bits, self.top_k)
         self.gate_up = None if self.decode_tiles else tuple(gate_up)
         self.down = None if self.decode_tiles else tuple(down)
+        # MLX-layout decode whose gate_up kernel picks the experts itself
+        self._mlx_topk = self.gate_up is not None and ops.gate_up_topk_supported(
+            self.hidden, self.num_experts, self.top_k, group_size, bits)
         # the sorted (grouped GEMM) path from this many (token, expert) pairs
         # on; below it the decode kernels (which take at most 16 tokens)
         self.sort_min_pairs = int(sort_min_pairs)
@@ -167,8 +171,8 @@ class SparseMoeBlock:
         self._shared_expert_rows = (self._shared_tiles is not None and self._shared_tiles[0].N == self.gu_tiles.N
                                     and shared.gate_weight.numel() == self.hidden
                                     and self.num_experts <= ROUTE_BLOCK_MAX_E)
-        if self._shared_expert_rows:  # constant ids and scores of the shared expert's decode kernels
-            dev = self.gu_tiles.wp.device
+        if shared is not None:  # constant ids and scores of the shared expert's decode kernels
+            dev = shared.gate_weight.device
             self._zeros = torch.zeros(16, 1, dtype=torch.int32, device=dev)
             self._ones = torch.ones(16, 1, dtype=torch.float32, device=dev)
 
@@ -226,21 +230,24 @@ class SparseMoeBlock:
         gu_t, dn_t = self._shared_tiles
         gate = self.shared.gate_weight
         idx, scores = ops.router_topk_shared(self.route_logits(x2), k, x2, gate, self.norm)
+        x_rows, inv, tiles = ops.route_block(idx, self.num_experts, shared=T > 16)
         if T <= 16:
-            x_rows, inv, tiles = ops.route_block(idx, self.num_experts)
             h = ops.gather_qmm_swiglu_sorted_tiles(x2, self.gu_tiles, tiles, x_rows=x_rows)
             yd = ops.gather_qmm_sorted_tiles(h, self.down_tiles, tiles)
             ys = self._shared_mlp(x2)
         else:
-            x_rows, inv, tiles = ops.route_block(idx, self.num_experts, shared=True)
             h = ops.gather_qmm_sorted_tiles_shared(x2, self.gu_tiles, gu_t, tiles, x_rows=x_rows)
             yd = ops.gather_qmm_sorted_tiles_shared(h, self.down_tiles, dn_t, tiles)
             ys = yd[T * k:]
         return ops.moe_weighted_sum_shared(yd, inv, scores, ys, self.wsum_mode)
 
     def _shared_mlp(self, x2: torch.Tensor) -> torch.Tensor:
-        """The shared expert's SwiGLU MLP of up to 16 tokens, ungated."""
+        """The shared expert's SwiGLU MLP, ungated."""
         T = x2.shape[0]
+        if T > 16 and self._shared_tiles is not None:
+            gu_t, dn_t = self._shared_tiles
+            tiles = ops.build_tiles(torch.zeros(T, dtype=torch.int32, device=x2.device), 1)
+            return ops.gather_qmm_sorted_tiles(ops.gather_qmm_swiglu_sorted_tiles(x2, gu_t, tiles), dn_t, tiles)
         zeros, ones = self._zeros[:T], self._ones[:T]
         if self._shared_decode_tiles:
             gu_t, dn_t = self._shared_tiles
@@ -293,9 +300,16 @@ class SparseMoeBlock:
             h, idx, scores = ops.gate_up_silu_tiles_topk(x2, self.gu_tiles, self.route_logits(x2), self.top_k,
                                                          self.norm)
             y = ops.down_wsum_tiles(h, self.down_tiles, idx, scores)
+        elif self._mlx_topk and T <= 16 and T * self.top_k < self.sort_min_pairs:
+            h, idx, scores = ops.gate_up_silu_topk(x2, *self.gate_up, self.route_logits(x2), self.top_k, self.norm)
+            y = ops.down_wsum(h, *self.down, idx, scores, self.group_size, self.bits)
         else:
             idx, scores = self.route(x2)
             y = self.experts(x2, idx, scores)
         if self.shared is not None:
-            y = (y.float() + self.shared_expert(x2).float()).to(torch.bfloat16)
+            gate = self.shared.gate_weight
+            if gate.numel() == self.hidden and self.hidden % 8 == 0:
+                y = ops.shared_combine(y, self._shared_mlp(x2), x2, gate)
+            else:
+                y = (y.float() + self.shared_expert(x2).float()).to(torch.bfloat16)
         return y.reshape(x.shape)

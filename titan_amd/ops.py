@@ -604,6 +604,33 @@ def gate_up_silu(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases:
     return h
 
 
+def gate_up_topk_supported(K: int, num_experts: int, top_k: int, group_size: int, bits: int) -> bool:
+    """Does :func:`gate_up_silu_topk` take a layer of this shape?"""
+    return (K in (2048, 4096) and (group_size, bits) == (GROUP, BITS) and num_experts <= 1024
+            and 1 <= top_k <= min(64, num_experts))
+
+
+def gate_up_silu_topk(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
+                      logits: torch.Tensor, top_k: int, norm: bool = True, group_size: int = GROUP,
+                      bits: int = BITS):
+    """:func:`gate_up_silu` with each token's experts chosen in the kernel from
+    its fp32 router logits [T, E], as :func:`gate_up_silu_tiles_topk`:
+    (h [T, k, I], idx, scores [T, k])."""
+    x = _bf16(x, "x")
+    w, scales, biases = _words(w, "w"), _bf16(scales, "scales"), _bf16(biases, "biases")
+    T, K = x.shape
+    _check_quant(w, scales, group_size, bits, K)
+    E, I = w.shape[0], w.shape[1] // 2
+    lg = _logits(logits, T, E, x.device)
+    h = torch.empty(T, top_k, I, dtype=torch.bfloat16, device=x.device)
+    idx = torch.empty(T, top_k, dtype=torch.int32, device=x.device)
+    scores_ = torch.empty(T, top_k, dtype=torch.float32, device=x.device)
+    _lib.call("qmoe_moe_gate_up_swiglu_topk", x.data_ptr(), lg.data_ptr(), int(bool(norm)), T, top_k, K, w.data_ptr(),
+              scales.data_ptr(), biases.data_ptr(), E, I, group_size, bits, h.data_ptr(), idx.data_ptr(),
+              scores_.data_ptr(), _stream(x))
+    return h, idx, scores_
+
+
 def down_wsum(h: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
               idx: torch.Tensor, scores: torch.Tensor, group_size: int = GROUP,
               bits: int = BITS) -> torch.Tensor:
@@ -770,6 +797,19 @@ def moe_weighted_sum_shared(xs: torch.Tensor, inv_order: torch.Tensor, scores: t
     return out
 
 
+def shared_combine(y: torch.Tensor, ys: torch.Tensor, x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
+    """y + sigmoid(x . gate) * ys in fp32, one rounding; y and ys [T, D], x [T, K]."""
+    y, ys, x, gate = _bf16(y, "y"), _bf16(ys, "ys"), _bf16(x, "x"), _bf16(gate, "gate")
+    T, D = y.shape
+    K = x.shape[-1]
+    if ys.shape != y.shape or x.shape[0] != T or gate.numel() != K:
+        raise ValueError("y, ys, x and gate disagree")
+    out = torch.empty_like(y)
+    _lib.call("qmoe_shared_combine", y.data_ptr(), ys.data_ptr(), x.data_ptr(), gate.data_ptr(), T, K, D,
+              out.data_ptr(), _stream(y))
+    return out
+
+
 def router_topk_shared(logits: torch.Tensor, k: int, x: torch.Tensor, gate: torch.Tensor, norm: bool = True):
     """:func:`router_topk` with the shared expert's weight sigmoid(x . gate) as
     one more score: (idx int32 [T, k], scores float32 [T, k + 1])."""
@@ -834,7 +874,7 @@ __all__ = [
     "repack_tiles", "gather_qmm_sorted_tiles", "gather_qmm_int8_sorted_tiles", "router_topk", "router_logits", "gather_qmm_swiglu_sorted_tiles", "swiglu_pair_order", "gather_qmv_tiles", "gate_up_silu_tiles",
     "down_wsum_tiles", "gate_up_silu_tiles_topk", "gate_up_silu_tiles_topk_shared", "down_wsum_tiles_shared",
     "route_block", "gather_qmm_sorted_tiles_shared", "moe_weighted_sum_shared", "router_topk_shared",
-    "gather_rows", "swiglu", "max_tiles", "tile_rows", "unpack", "dequantize", "gather_qmv", "gather_qmm_sorted", "gather_qmm",
+    "gate_up_silu_topk", "gate_up_topk_supported", "gather_rows", "swiglu", "shared_combine", "max_tiles", "tile_rows", "unpack", "dequantize", "gather_qmv", "gather_qmm_sorted", "gather_qmm",
     "gemm_supported", "quantized_matmul", "gate_up_silu", "down_wsum", "moe_weighted_sum",
     "quantize_act_int8", "gather_qmm_int8_sorted",
 ]
