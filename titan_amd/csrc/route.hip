@@ -494,6 +494,12 @@ __global__ __launch_bounds__(kScanThreads) void tiles_from_sorted_kernel(const i
 // expert, and the wave then walks its segment in order ranking equal ids with
 // ballots, as route_scatter_kernel does per chunk -- stable, no global round
 // trips between the phases.
+// Few pairs take half the waves: the histograms to clear and scan halve, and a
+// wave still has at most two steps of 64 rows.  Per call in a graph at 256
+// experts (two / four / eight / sixteen waves): 70 pairs 4.8 / 4.9 / 4.9 / 5.7 us,
+// 510 pairs 6.7 / 5.4 / 4.9 / 5.7, 1020 pairs - / 6.8 / 5.5 / 5.7, 2000 - / - / 7.0 / 6.6.
+constexpr int kSmallWaves = 8;
+constexpr int64_t kSmallMaxN = 1024;
 constexpr int kFusedWaves = kScanThreads / 64;
 constexpr int kFusedMaxE = 512;
 constexpr int kFusedSteps = 4;
@@ -502,17 +508,18 @@ constexpr int kFusedSteps = 4;
 // the block's serial walk has grown with n to about the launches' cost
 constexpr int64_t kFusedMaxN = (int64_t)kFusedWaves * 64 * kFusedSteps;
 
-__global__ __launch_bounds__(kScanThreads) void route_fused_kernel(
+template <int W>
+__global__ __launch_bounds__(64 * W) void route_fused_kernel(
     const int32_t* __restrict__ ids, int64_t n, int E, int nbits, int tile_rows, int32_t* __restrict__ order,
     int32_t* __restrict__ inv_order, int32_t* __restrict__ sorted_ids, int32_t* __restrict__ offsets,
     int32_t* __restrict__ tile_row, int32_t* __restrict__ tile_exp, int32_t* __restrict__ ntiles,
     int64_t max_tiles, int32_t* __restrict__ bad, BlockRows br) {
   extern __shared__ int sm[];
-  int* hist = sm;                          // [kFusedWaves][E + 1]; slot E counts out-of-range ids
-  int* off = sm + kFusedWaves * (E + 1);   // [E + 2]
-  __shared__ int lds[kScanThreads];
+  int* hist = sm;                          // [W][E + 1]; slot E counts out-of-range ids
+  int* off = sm + W * (E + 1);   // [E + 2]
+  __shared__ int lds[(64 * W)];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int64_t seg = (n + kFusedWaves - 1) / kFusedWaves;
+  const int64_t seg = (n + W - 1) / W;
   const int64_t lo = min((int64_t)w * seg, n), hi = min(lo + seg, n);
   int* my = hist + w * (E + 1);
   int idv[kFusedSteps];  // the segment's ids (seg <= 64 * kFusedSteps)
@@ -520,7 +527,7 @@ __global__ __launch_bounds__(kScanThreads) void route_fused_kernel(
 #pragma unroll
     for (int q = 0; q < kFusedSteps; ++q) idv[q] = load_id(ids, lo + 64 * q + lane, hi);
   }
-  for (int i = tid; i < kFusedWaves * (E + 1); i += kScanThreads) hist[i] = 0;
+  for (int i = tid; i < W * (E + 1); i += (64 * W)) hist[i] = 0;
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < kFusedSteps; ++q) {
@@ -532,26 +539,26 @@ __global__ __launch_bounds__(kScanThreads) void route_fused_kernel(
   __syncthreads();
   if (tid == 0) {
     int nb = 0;
-    for (int q = 0; q < kFusedWaves; ++q) nb += hist[q * (E + 1) + E];
+    for (int q = 0; q < W; ++q) nb += hist[q * (E + 1) + E];
     bad[0] = nb;
   }
-  // exclusive scan, in place, over f = e * kFusedWaves + w (expert-major): a
+  // exclusive scan, in place, over f = e * W + w (expert-major): a
   // wave's rows of one expert come after every lower wave's rows of it
-  const int L = E * kFusedWaves;
-  const int per = (L + kScanThreads - 1) / kScanThreads;
+  const int L = E * W;
+  const int per = (L + (64 * W) - 1) / (64 * W);
   const int f0 = min(tid * per, L), f1 = min(f0 + per, L);
   int local = 0;
-  for (int f = f0; f < f1; ++f) local += hist[(f % kFusedWaves) * (E + 1) + f / kFusedWaves];
+  for (int f = f0; f < f1; ++f) local += hist[(f % W) * (E + 1) + f / W];
   int total;
-  int run = block_exclusive_scan(local, lds, &total);  // its barriers order every read above before the writes
+  int run = block_exclusive_scan<64 * W>(local, lds, &total);  // its barriers order every read above before the writes
   for (int f = f0; f < f1; ++f) {
-    int* h = &hist[(f % kFusedWaves) * (E + 1) + f / kFusedWaves];
+    int* h = &hist[(f % W) * (E + 1) + f / W];
     const int c = *h;
     *h = run;
     run += c;
   }
   __syncthreads();
-  for (int e = tid; e < E; e += kScanThreads) {
+  for (int e = tid; e < E; e += (64 * W)) {
     off[e] = hist[e];  // wave 0's first slot = the expert's offset
     offsets[e] = hist[e];
   }
@@ -562,7 +569,7 @@ __global__ __launch_bounds__(kScanThreads) void route_fused_kernel(
     if (br.rows > 0) offsets[E + 1] = (int32_t)(n + br.rows);
   }
   if (br.x_rows)
-    for (int i = tid; i < br.rows; i += kScanThreads) br.x_rows[n + i] = i;
+    for (int i = tid; i < br.rows; i += (64 * W)) br.x_rows[n + i] = i;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
   for (int q = 0; q < kFusedSteps; ++q) {
@@ -590,7 +597,7 @@ __global__ __launch_bounds__(kScanThreads) void route_fused_kernel(
     __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
-  emit_tiles(off, E + (br.rows > 0 ? 1 : 0), tile_rows, tile_row, tile_exp, ntiles, max_tiles, lds);
+  emit_tiles<64 * W>(off, E + (br.rows > 0 ? 1 : 0), tile_rows, tile_row, tile_exp, ntiles, max_tiles, lds);
 }
 
 int64_t n_chunks(int64_t n) { return (n + kChunk - 1) / kChunk; }
@@ -639,10 +646,15 @@ int route_launch(const int32_t* ids, int64_t n_pairs, int32_t num_experts, int32
   if (n_pairs <= kFusedMaxN && num_experts <= kFusedMaxE) {
     int nbits = 1;
     while ((1 << nbits) <= num_experts) ++nbits;  // ids in [0, E] (E is the sentinel)
-    const size_t shm = ((size_t)(kFusedWaves + 1) * (num_experts + 1) + 1) * sizeof(int);
-    route_fused_kernel<<<dim3(1), dim3(kScanThreads), shm, st>>>(ids, n_pairs, num_experts, nbits, tile_rows,
-                                                                order, inv_order, sorted_ids, offsets, tile_row,
-                                                                tile_exp, ntiles, max_tiles, bad, br);
+    const int W = n_pairs <= kSmallMaxN ? kSmallWaves : kFusedWaves;
+    const size_t shm = ((size_t)(W + 1) * (num_experts + 1) + 1) * sizeof(int);
+#define ROUTE_FUSED(W_) \
+  route_fused_kernel<W_><<<dim3(1), dim3(64 * W_), shm, st>>>(ids, n_pairs, num_experts, nbits, tile_rows, order, \
+                                                              inv_order, sorted_ids, offsets, tile_row, tile_exp, \
+                                                              ntiles, max_tiles, bad, br)
+    if (W == kSmallWaves) ROUTE_FUSED(kSmallWaves);
+    else ROUTE_FUSED(kFusedWaves);
+#undef ROUTE_FUSED
     return qmoe::launch_status("route_fused_kernel");
   }
   int nbits = 1;
