@@ -96,6 +96,24 @@ def test_block_with_shared_expert_matches_its_parts(dev, T, k, S):
     assert bool(((y.double() - ref).abs() <= 2.0 ** -7 * ref.abs().max()).all())
 
 
+@pytest.mark.parametrize("sort_min_pairs", [0, 64])
+@pytest.mark.parametrize("S", [None, 512, 768])
+def test_block_of_no_tokens(dev, S, sort_min_pairs):
+    print(f"[case] block of no tokens S={S} sort_min_pairs={sort_min_pairs}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(3)
+    H, I, E = 2048, 512, 16
+    shared = None
+    if S:
+        gate = torch.randn(1, H, device=dev, generator=g).to(torch.bfloat16)
+        shared = SharedExpert(_quant(g, (1, 2 * S), H, dev), _quant(g, (1, H), S, dev), gate)
+    rw = torch.randn(E, H, device=dev, generator=g).to(torch.bfloat16)
+    blk = SparseMoeBlock(rw, _quant(g, (E, 2 * I), H, dev), _quant(g, (E, H), I, dev), 4, shared=shared,
+                         sort_min_pairs=sort_min_pairs)
+    x = torch.empty(0, H, dtype=torch.bfloat16, device=dev)
+    assert blk(x).shape == (0, H)
+    assert blk.experts(x, *blk.route(x)).shape == (0, H)
+
+
 @pytest.mark.parametrize("T,k,E", [(1, 1, 1), (7, 10, 256), (64, 64, 100), (409, 10, 512), (410, 10, 256),
                                    (129, 3, 2048), (5, 4, 513), (3000, 10, 64)])
 def test_route_block_matches_route(dev, T, k, E):

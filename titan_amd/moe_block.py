@@ -215,7 +215,7 @@ class SparseMoeBlock:
                 return ops.down_wsum_tiles(h, self.down_tiles, idx, scores)
             h = ops.gate_up_silu(x2, *self.gate_up, idx, self.group_size, self.bits)
             return ops.down_wsum(h, *self.down, idx, scores, self.group_size, self.bits)
-        if self.num_experts > ROUTE_BLOCK_MAX_E:
+        if T == 0 or self.num_experts > ROUTE_BLOCK_MAX_E:
             r = ops.route(idx, self.num_experts)
             x_rows, inv, tiles = torch.div(r.order, k, rounding_mode="floor").to(torch.int32), r.inv_order, r.tiles
         else:
@@ -294,7 +294,7 @@ class SparseMoeBlock:
                                                                 gu_t, self.shared.gate_weight, self.norm)
             return ops.down_wsum_tiles_shared(h, self.down_tiles, idx, scores, dn_t).reshape(x.shape)
         T = x2.shape[0]
-        if self._shared_expert_rows and not (T * self.top_k < self.sort_min_pairs and T <= 16):
+        if T and self._shared_expert_rows and not (T * self.top_k < self.sort_min_pairs and T <= 16):
             return self._sorted_with_shared(x2).reshape(x.shape)
         if self.decodes_with_topk(T):
             h, idx, scores = ops.gate_up_silu_tiles_topk(x2, self.gu_tiles, self.route_logits(x2), self.top_k,
