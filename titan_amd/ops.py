@@ -489,6 +489,9 @@ def down_wsum_tiles_shared(h: torch.Tensor, tw: TileWeights, idx: torch.Tensor, 
     T, slots, I = h.shape
     if (shared.num_experts, shared.N, shared.K) != (1, tw.N, tw.K) or I != tw.K:
         raise ValueError("h and the shared expert must have the routed experts' shape")
+    if idx.numel() != T * slots or scores.numel() != T * slots:
+        raise ValueError(f"idx and scores must be [T, slots] = [{T}, {slots}], got {tuple(idx.shape)} and "
+                         f"{tuple(scores.shape)}")
     idx = _i32(idx, "idx", h.device)
     sc = _f32(scores, "scores", h.device)
     y = torch.empty(T, tw.N, dtype=torch.bfloat16, device=h.device)
