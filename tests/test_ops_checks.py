@@ -35,3 +35,23 @@ def test_down_wsum_shared_needs_every_slot(ids, scores):
     with pytest.raises(AssertionError, match="launched"):  # the right ones reach the kernel
         ops.down_wsum_tiles_shared(h, _tiles(5, D, I), torch.zeros(T, slots, dtype=torch.int32),
                                    torch.zeros(T, slots), _tiles(1, D, I))
+
+
+# the rows of the routed pairs alone, as a routing without shared rows gives them
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("pairs", [False, True])
+def test_gemm_with_shared_expert_needs_every_row(gathered, pairs):
+    T, k, E, K, N = 6, 3, 5, 128, 256
+    i32 = torch.zeros(E + 2, dtype=torch.int32)
+    table = ops.TileTable(i32, i32, i32, i32[:1], E + 2, 128, E + 1, T * k + T)
+
+    def gemm(rows):
+        x = torch.zeros(T if gathered else rows, K, dtype=torch.bfloat16)
+        ops.gather_qmm_sorted_tiles_shared(x, _tiles(E, N, K, pairs), _tiles(1, N, K, pairs), table,
+                                           x_rows=torch.zeros(rows, dtype=torch.int32) if gathered else None)
+
+    for rows in (0, T * k, T * k + T - 1):
+        with pytest.raises(ValueError, match="rows"):
+            gemm(rows)
+    with pytest.raises(AssertionError, match="launched"):
+        gemm(T * k + T)

@@ -773,6 +773,9 @@ def gather_qmm_sorted_tiles_shared(x: torch.Tensor, tw: TileWeights, shared: Til
         raise ValueError("tile table does not match this call")
     x2 = x.reshape(-1, K)
     xr = None if x_rows is None else _i32(x_rows.reshape(-1), "x_rows", x.device)
+    have = x2.shape[0] if xr is None else xr.numel()
+    if have < tiles.rows:
+        raise ValueError(f"{'x' if xr is None else 'x_rows'} has {have} rows, the tile table {tiles.rows}")
     out = torch.empty(tiles.rows, tw.N // 2 if tw.swiglu_pairs else tw.N, dtype=torch.bfloat16, device=x.device)
     _lib.call("qmoe_gather_qmm_sorted_tiles_shared", x2.data_ptr(), _ptr(xr), tiles.rows, K, tw.wp.data_ptr(),
               tw.sb.data_ptr(), shared.wp.data_ptr(), shared.sb.data_ptr(), tw.num_experts, tw.N,
