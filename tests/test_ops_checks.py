@@ -55,3 +55,11 @@ def test_gemm_with_shared_expert_needs_every_row(gathered, pairs):
             gemm(rows)
     with pytest.raises(AssertionError, match="launched"):
         gemm(T * k + T)
+
+
+@pytest.mark.parametrize("width", [1, 17, 1025])
+def test_swiglu_needs_both_halves(width):
+    with pytest.raises(ValueError, match="2I"):
+        ops.swiglu(torch.zeros(3, width, dtype=torch.bfloat16))
+    with pytest.raises(AssertionError, match="launched"):
+        ops.swiglu(torch.zeros(3, width + 15 + (width + 15) % 2, dtype=torch.bfloat16))

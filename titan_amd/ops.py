@@ -239,6 +239,8 @@ def gather_rows(x: torch.Tensor, rows: torch.Tensor, div: int = 1) -> torch.Tens
 def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
     """silu(gate) * up of a fused [.., 2I] projection, gate first: fp32, one rounding."""
     gate_up = _bf16(gate_up, "gate_up")
+    if gate_up.shape[-1] % 2:
+        raise ValueError(f"gate_up must be [.., 2I], got {tuple(gate_up.shape)}")
     I = gate_up.shape[-1] // 2
     h = torch.empty(*gate_up.shape[:-1], I, dtype=torch.bfloat16, device=gate_up.device)
     _lib.call("qmoe_swiglu", gate_up.data_ptr(), h.numel() // I if I else 0, I, h.data_ptr(), _stream(gate_up))
