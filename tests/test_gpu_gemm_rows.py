@@ -42,3 +42,35 @@ def test_rows_kernel_is_the_tile_kernel(dev, rows, N, K, gathered):
         y = gemm(x, ops.repack_tiles(*w, swiglu_pairs=pairs), many_t, x_rows=None if x_rows is None else x_rows[:R])
         ref = gemm(x, ops.repack_tiles(*sub, swiglu_pairs=pairs), few_t, x_rows=x_rows)
         assert torch.equal(y, ref[:R])
+
+
+# What decides between the two kernels, and the rows kernel's grid, on either
+# side: the rows of a call (320 | more), the rows per tile (16 | more), more
+# tiles and more 33-row tiles than a round of the grid has blocks for, and a
+# table past the limit of rows per expert.  (rows per used expert, experts, N)
+@pytest.mark.parametrize("rows,E,N", [
+    ((32,) * 10, 100, 512), ((33,) + (32,) * 9, 100, 512),   # 320 and 321 rows
+    ((97, 65, 33, 1, 125), 60, 768),                         # 321 rows: every subtile, tile kernel
+    ((16,) * 30, 100, 256), ((17,) + (16,) * 29, 100, 256),  # 16 rows per tile and a little more
+    ((1,) * 40 + (100, 300, 33), 80, 512),                   # few rows per tile, several large tiles
+    ((1,) * 2300, 2400, 256),                                # more tiles than 2048 blocks of one column block
+    ((33, 1, 1) * 150, 900, 4096),                           # more large tiles than the 128 of a round
+])
+def test_either_kernel_is_the_tile_kernel(dev, rows, E, N):
+    print(f"[case] rows {len(rows)} x {max(rows)} of {E} experts, N={N}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(sum(rows) + E)
+    n, R, K = len(rows), sum(rows), 64
+    assert R <= 6 * E
+    used = torch.randperm(E, device=dev, generator=g)[:n].sort()[0]
+    ids = torch.repeat_interleave(torch.arange(n, device=dev), torch.tensor(rows, device=dev))
+    more = 6 * (n + 1) + 1  # rows of one more expert, which put the second table past the limit
+    x = torch.randn(R + more, K, device=dev, generator=g).to(torch.bfloat16)
+    w = _quant(g, (E, N), K, dev)
+    sub = tuple(t[torch.cat([used, used[:1]])].contiguous() for t in w)
+    many_t = ops.build_tiles(used[ids].to(torch.int32), E)
+    past_t = ops.build_tiles(torch.cat([ids, torch.full((more,), n, device=dev)]).to(torch.int32), n + 1)
+    for pairs in (False, True):
+        gemm = ops.gather_qmm_swiglu_sorted_tiles if pairs else ops.gather_qmm_sorted_tiles
+        y = gemm(x[:R], ops.repack_tiles(*w, swiglu_pairs=pairs), many_t)
+        ref = gemm(x, ops.repack_tiles(*sub, swiglu_pairs=pairs), past_t)
+        assert torch.equal(y, ref[:R])

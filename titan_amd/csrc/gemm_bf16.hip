@@ -51,6 +51,7 @@
 // K order inside a group is free as long as A and B agree: lane half h
 // supplies group elements 32h + 8kk .. +7 at k-step kk -- word kk of the
 // lane's 16-byte code chunk and 16-byte unit 4h + kk of the activation row.
+#include <algorithm>
 #include <type_traits>
 
 #include "gemm_common.h"
@@ -117,6 +118,8 @@ struct Cfg {
   // at most 63 vector-memory operations outstanding per wave
   static_assert((kStages - 1) * kCopies <= 63, "vmcnt range");
 };
+
+constexpr int kRowsPerUnit = 32;  // rows of gemm_rows_kernel's unit
 
 struct GemmArgs {
   const uint16_t* x;
@@ -579,10 +582,10 @@ __device__ __forceinline__ void run_unit(const GemmArgs& a, char* smem, int tile
   else store_tile<TILED>(a, smem, c, acc, row0, valid, msub, nblk);
 }
 
-// Persistent grid (kBlocksPerCU blocks per CU), each block walking its
+// One block of a persistent grid of `blocks` (kBlocksPerCU per CU), walking its
 // slot's units of the ranked tile order.
 template <bool TILED, bool SWIGLU>
-__global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmArgs a) {
+__device__ __forceinline__ void tile_block(const GemmArgs& a, int blocks) {
   using C = Cfg<TILED>;
   __shared__ __attribute__((aligned(1024))) char smem[C::kLdsBytes];
   __shared__ int order[kMaxOrder];
@@ -590,7 +593,7 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmA
   const Tiles tt{a.offsets, a.tile_row, a.tile_exp, a.ntiles, a.n_rows, a.num_experts};
   const int NB = a.N / kBN;
   const int ntiles = a.ntiles[0];
-  const Snake sn((int64_t)ntiles * NB);
+  const Snake sn((int64_t)ntiles * NB, blocks);
   if (sn.unit(0) < 0) return;
   const bool sorted = ntiles <= kMaxOrder;
   if (sorted) rank_tiles(tt, ntiles, order, reinterpret_cast<int*>(smem));  // the ring is free until the first unit
@@ -609,7 +612,7 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmA
       // us on the 4096-token gate_up, 415.5 -> 407.9 us on the MoE block; the
       // MLX-layout form measured slower with it (246 -> 255 us) and keeps
       // the hardware's order.
-      if (((uint32_t)k ^ (blockIdx.x >= gridDim.x / 2 ? 1u : 0u)) & 1u) __builtin_amdgcn_s_setprio(1);
+      if (((uint32_t)k ^ ((int)blockIdx.x >= blocks / 2 ? 1u : 0u)) & 1u) __builtin_amdgcn_s_setprio(1);
       else __builtin_amdgcn_s_setprio(0);
     }
 #ifdef QMOE_GEMM_STAMPS
@@ -632,6 +635,11 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmA
 #endif
 }
 
+template <bool TILED, bool SWIGLU>
+__global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmArgs a) {
+  tile_block<TILED, SWIGLU>(a, gridDim.x);
+}
+
 // ---- few rows per expert -------------------------------------------------
 //
 // The same products for tiles of few rows, where a call streams its experts'
@@ -646,25 +654,51 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmA
 //
 // Where the tile kernel has one 256-column unit per workgroup, each with its
 // own latency to fill and drain a ring, here 4 to 16 times as many waves run
-// independently.  Per call in a graph (256 experts, top-10, 2048 x 1024
-// gate_up + SwiGLU / 512 x 2048 down; floor: the used experts' bytes at a 2 GiB
-// copy's 4.86 TB/s):
+// independently.  Per call in a graph (256 experts, top-10 of uneven
+// popularity, 2048 x 1024 gate_up + SwiGLU / 512 x 2048 down; floor: the used
+// experts' bytes at a 2 GiB copy's 4.86 TB/s):
 //   tokens   tile kernel    this kernel    floor
-//        7   32.9 / 14.3    17.7 / 10.4    13.6 /  6.8 us
-//       16   33.0 / 22.3    27.4 / 15.1    21.6 / 10.8
-//       32   37.3 / 23.1    31.8 / 19.6    29.9 / 14.9
-//       96   60.2 / 34.6    52.0 / 29.3    45.9 / 22.9
-//      200   64.1 / 42.2    68.6 / 40.0    50.7 / 25.4
-//      400   71.0 / 44.2    90.8 / 54.1    55.8 / 27.9
-// Beyond about six rows per expert the activation reads, a row's line per lane
-// and wave where the tile kernel copies each row once per workgroup, are what
-// bounds it (few_rows draws the line there).  Two or four groups ahead, and two
-// or four waves per SIMD, measured within 5% of three and three; a 32-column
-// unit twice as often (half the dequantisation per wave, all of its activation
-// reads) is slower from 7 tokens on, up to 1.9x at the down shape.
-constexpr int kRowsPerUnit = 32;
+//        7   32.6 / 14.4    17.9 / 10.8    13.6 /  6.8 us
+//       16   33.1 / 22.6    27.6 / 14.2    21.6 / 10.8
+//       32   38.3 / 23.7    31.1 / 19.3    29.9 / 14.9
+//       96   61.2 / 35.1    51.3 / 29.5    45.9 / 22.9
+//      200   65.3 / 44.7    64.9 / 39.7    50.7 / 25.4
+//      400   70.0 / 48.0    87.3 / 55.4    55.8 / 27.9
+// and with a shared expert's rows in the table (its tile has several subtiles)
+//       32   48.3 / 28.3    40.3 / 21.5
+//       96   61.8 / 35.1    53.0 / 30.8
+//      140   64.0 / 42.3    57.3 / 35.1
+// Beyond about six rows per expert (kRowsMaxPerExpert) the activation reads, a
+// row's line per lane and wave where the tile kernel copies each row once per
+// workgroup, are what bounds it.  They do so at fewer rows when these go to few
+// experts: 150 tokens that all choose the same 10 of 512 experts take 107 / 43
+// us (hidden 4096) against the tile kernel's 86 / 21.  Up to kRowsAlways rows
+// even the most uneven routing leaves this kernel ahead (320 rows of 10 to 64
+// experts: at most 0.85 of the tile kernel's time); past them only the device
+// knows, and gemm_either_kernel holds both and goes by the rows per tile: up to
+// 16 the rows kernel (24 to 30 rows per tile: 1.1 to 1.6 times the tile
+// kernel's time at the 4096-column down shape, 0.6 to 1.0 at the others), more
+// the tile kernel.  Against the tile kernel alone over 370 routings (8 to 150
+// tokens, 10 to all experts used, the three layer shapes 256 x 512 x 2048, 128
+// x 768 x 2048 and 512 x 512 x 4096) the geometric mean is 0.78 and the
+// largest ratio 1.07 (64 experts of 15 rows at that down shape).
+// The two share the tile kernel's registers and LDS, which leaves the rows
+// kernel two waves per SIMD instead of three: within 6% at those sizes.
+//
+// The grid has blocks for the rows there can be (RowsGrid), not for every
+// subtile of max_tiles tiles: 2^15 blocks that return at once cost the
+// 512-expert down launch 9 us of 17.  Past kRowsAlways it is kept at
+// kRowsMaxBlocks a subtile, and blocks take further tiles in turn.
+//
+// Two or four groups ahead, and two or four waves per SIMD, measured within 5%
+// of three and three; a 32-column unit twice as often (half the dequantisation
+// per wave, all of its activation reads) is slower from 7 tokens on, up to
+// 1.9x at the down shape.
 constexpr int kRowsDepth = 3;
 constexpr int kRowsMaxPerExpert = 6;
+constexpr int kRowsAlways = 320;
+constexpr int kRowsMaxPerTile = 16;
+constexpr int kRowsMaxBlocks = 2048;
 
 struct RowsGroup {
   i32x4_t a[4];    // activation bytes 64h .. 64h + 63 of the group
@@ -672,21 +706,49 @@ struct RowsGroup {
   uint32_t sb[2];  // their scale|bias words
 };
 
+// Tiles a launch has blocks for, per subtile: every tile holds a row, so there
+// are no more tiles than rows, and no more with a row past 32 s than n / (32 s + 1).
+constexpr int kRowsSubs = kTileRows / kRowsPerUnit;
+struct RowsGrid {
+  int tiles[kRowsSubs];
+};
+
+// The j-th tile, from the last, of more than `rows` rows (-1: fewer than j + 1).
+// Called by the whole block.
+__device__ int large_tile(const Tiles& t, int ntiles, int rows, int j) {
+  constexpr int W = kThreads / 64;
+  __shared__ int cnt[W];
+  __shared__ int found;
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const uint64_t below = (1ull << lane) - 1;
+  for (int base = 0; base < ntiles; base += kThreads) {
+    const int i = ntiles - 1 - base - (int)threadIdx.x;
+    const bool f = i >= 0 && tile_rows_of(t, i).valid > rows;
+    const uint64_t m = __ballot(f);
+    __syncthreads();  // every wave is done with the last round's counts and result
+    if (lane == 0) cnt[wave] = __popcll(m);
+    __syncthreads();
+    int before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      before += w < wave ? cnt[w] : 0;
+      total += cnt[w];
+    }
+    if (j < total) {  // block-uniform
+      if (f && before + __popcll(m & below) == j) found = i;
+      __syncthreads();
+      return __builtin_amdgcn_readfirstlane(found);
+    }
+    j -= total;
+  }
+  return -1;
+}
+
 template <bool SWIGLU>
-__global__ __launch_bounds__(kThreads, 3) void gemm_rows_kernel(GemmArgs a, int max_tiles) {
+__device__ __forceinline__ void rows_unit(const GemmArgs& a, int tile, int sub, int nblk) {
   constexpr int D = kRowsDepth;
   const int lane = threadIdx.x % 64, l32 = lane % 32, h = lane / 32;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
-  const int NB = a.N / kBN;
-  // blocks: row subtile slowest (most tiles have only the first), then tile
-  // from the last (a shared expert's full tiles) to the first, then columns
-  const int per_sub = max_tiles * NB;
-  const int sub = blockIdx.x / per_sub;
-  const int rem = blockIdx.x - sub * per_sub;
-  const int back = rem / NB;
-  const int nblk = rem - back * NB;
-  const int tile = a.ntiles[0] - 1 - back;
-  if (tile < 0) return;
   const TileRows tr = tile_rows_of(Tiles{a.offsets, a.tile_row, a.tile_exp, a.ntiles, a.n_rows, a.num_experts}, tile);
   const int valid = tr.valid - sub * kRowsPerUnit;
   if (valid <= 0) return;
@@ -781,26 +843,78 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_rows_kernel(GemmArgs a, int 
   }
 }
 
+template <bool SWIGLU>
+__device__ __forceinline__ void rows_block(const GemmArgs& a, const RowsGrid& grid) {
+  const int NB = a.N / kBN;
+  // blocks: the further subtiles of the tiles that have them (these look for
+  // their tile first, so they start first), then the tiles' first subtiles;
+  // from the last tile (a shared expert's full tiles) to the first, columns
+  // fastest
+  int sub = kRowsSubs - 1, back = blockIdx.x / NB, step = grid.tiles[sub];
+  const int nblk = blockIdx.x - back * NB;
+#pragma unroll
+  for (int s = kRowsSubs - 2; s >= 0; --s)
+    if (sub == s + 1 && back >= step) {
+      back -= step;
+      step = grid.tiles[s];
+      sub = s;
+    }
+  if (back >= step) return;  // a grid rounded up
+  const int ntiles = a.ntiles[0];
+  // one round, unless a caller's own table holds empty or overlapping tiles
+  for (;; back += step) {
+    const int tile = sub == 0 ? ntiles - 1 - back
+                              : large_tile(Tiles{a.offsets, a.tile_row, a.tile_exp, a.ntiles, a.n_rows, a.num_experts},
+                                           ntiles, sub * kRowsPerUnit, back);
+    if (tile < 0) return;  // block-uniform
+    rows_unit<SWIGLU>(a, tile, sub, nblk);
+  }
+}
+
+template <bool SWIGLU>
+__global__ __launch_bounds__(kThreads, 3) void gemm_rows_kernel(GemmArgs a, RowsGrid grid) {
+  rows_block<SWIGLU>(a, grid);
+}
+
+// Either way, as the table says: only the device knows how many experts the
+// rows are spread over.
+template <bool SWIGLU>
+__global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_either_kernel(GemmArgs a, RowsGrid grid, int tile_blocks) {
+  if (a.n_rows <= (int64_t)kRowsMaxPerTile * a.ntiles[0]) rows_block<SWIGLU>(a, grid);
+  else if ((int)blockIdx.x < tile_blocks) tile_block<true, SWIGLU>(a, tile_blocks);
+}
+
 }  // namespace
 
 extern "C" int qmoe_gemm_tile_rows(void) { return kBM; }
 
 namespace {
 
-// Few rows per expert: gemm_rows_kernel (its comment has both sides measured).
-bool few_rows(const GemmArgs& a, int64_t max_tiles) {
-  const int64_t blocks = max_tiles * (a.N / kBN) * (kTileRows / kRowsPerUnit);
-  return a.n_rows <= (int64_t)kRowsMaxPerExpert * a.num_experts && blocks <= 0x7FFFFFFF;
-}
-
 int launch_gemm(const GemmArgs& a, int64_t max_tiles, bool tiled, void* stream, bool swiglu = false) {
   const dim3 grid((unsigned)grid_blocks(max_tiles * (a.N / kBN)));
   hipStream_t st = qmoe::as_stream(stream);
-  if (tiled && few_rows(a, max_tiles)) {
-    const dim3 g((unsigned)(max_tiles * (a.N / kBN) * (kTileRows / kRowsPerUnit)));
-    if (swiglu) gemm_rows_kernel<true><<<g, dim3(kThreads), 0, st>>>(a, (int)max_tiles);
-    else gemm_rows_kernel<false><<<g, dim3(kThreads), 0, st>>>(a, (int)max_tiles);
-    return qmoe::launch_status("gemm_rows_kernel");
+  // few rows per expert: gemm_rows_kernel's comment has both sides measured
+  if (tiled && a.n_rows <= (int64_t)kRowsMaxPerExpert * a.num_experts) {
+    const int64_t NB = a.N / kBN;
+    const bool always = a.n_rows <= kRowsAlways;
+    RowsGrid rg;
+    int64_t blocks = 0;
+    for (int s = 0; s < kRowsSubs; ++s) {
+      int64_t t = std::min<int64_t>(max_tiles, a.n_rows / (s * kRowsPerUnit + 1));
+      if (!always) t = std::min(t, std::max<int64_t>(1, kRowsMaxBlocks / NB));
+      rg.tiles[s] = (int)t;
+      blocks += t * NB;
+    }
+    if (always) {  // at most 320 + 9 + 4 + 3 tiles and 2^16 column blocks
+      const dim3 g((unsigned)blocks);
+      if (swiglu) gemm_rows_kernel<true><<<g, dim3(kThreads), 0, st>>>(a, rg);
+      else gemm_rows_kernel<false><<<g, dim3(kThreads), 0, st>>>(a, rg);
+      return qmoe::launch_status("gemm_rows_kernel");
+    }
+    const dim3 g(std::max((unsigned)blocks, grid.x));
+    if (swiglu) gemm_either_kernel<true><<<g, dim3(kThreads), 0, st>>>(a, rg, (int)grid.x);
+    else gemm_either_kernel<false><<<g, dim3(kThreads), 0, st>>>(a, rg, (int)grid.x);
+    return qmoe::launch_status("gemm_either_kernel");
   }
   if (swiglu) gemm_bf16_kernel<true, true><<<grid, dim3(kThreads), 0, st>>>(a);
   else if (tiled) gemm_bf16_kernel<true, false><<<grid, dim3(kThreads), 0, st>>>(a);

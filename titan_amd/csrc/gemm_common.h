@@ -200,8 +200,7 @@ __device__ inline void rank_tiles(const Tiles& t, int ntiles, int* order, int* c
 struct Snake {
   int64_t units;
   int P, q;
-  __device__ __forceinline__ Snake(int64_t units_) : units(units_) {
-    P = gridDim.x;
+  __device__ __forceinline__ Snake(int64_t units_, int blocks = gridDim.x) : units(units_), P(blocks) {
     const int b = blockIdx.x;
     q = (b % 8) * (P / 8) + b / 8;
   }
