@@ -1038,9 +1038,9 @@ __global__ __launch_bounds__(64) void qmv64_paired_kernel(QmvArgs a) {
 
 // Fused gate_up + SwiGLU over the gate/up-paired tile layout with line reads:
 // a wave computes RG indices i0 .. (gate rows l0 .. l0 + RG - 1 of half j = 0
-// of column block c = i0 / 32, up rows in half j = 1).  Lane 8 s + r holds row
-// slot r and group slot s; its load (p, h) reads the 16-byte unit
-// (g = 8p + s, j, h, l0 + rr) of its row, so eight neighbouring lanes read
+// of column block c = i0 / 32, up rows in half j = 1).  Lane 8 s + r (8 r + s
+// without kRowsFast) holds row slot r and group slot s; its load (p, h) reads
+// the 16-byte unit (g = 8p + s, j, h, l0 + rr) of its row, so eight lanes read
 // consecutive rows of one (g, j, h): RG = 8 gives each slot two whole 128-byte
 // lines (rows of gate and of up, r = 0..7 each), RG = 4 one 64-byte half-line
 // of gate rows (r < 4) and one of up rows (r >= 4), whose other halves the
@@ -1048,8 +1048,8 @@ __global__ __launch_bounds__(64) void qmv64_paired_kernel(QmvArgs a) {
 // (of one pair) stage its x row in LDS once (per 32-element chunk: the 16 bf16
 // pairs matched to the nibble pairs, and the chunk's sum) and each lane reads
 // the chunk of its (g, h) per step.  Per lane the affine chunk arithmetic is
-// qmv64_kernel's; the row sums close over the eight group slots with one DPP
-// step and two lane swaps.
+// qmv64_kernel's; the row sums close over the eight group slots (s ^ 1, s ^ 2,
+// s ^ 4: the same bits from either lane order).
 template <int NV, int RG, int W, int PER = 0, bool SH = false>
 __global__ __launch_bounds__(64 * W) void qmv64_paired_lines_kernel(QmvArgs a) {
   static_assert(RG == 4 || RG == 8, "four or eight indices per wave");
@@ -1060,7 +1060,12 @@ __global__ __launch_bounds__(64 * W) void qmv64_paired_lines_kernel(QmvArgs a) {
   __shared__ float xsum[NCH];
   const int lane = threadIdx.x % 64;
   const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
-  const int r = lane & 7, sl = lane >> 3;  // rows fastest: eight neighbouring lanes read one line
+  // Rows fastest: eight neighbouring lanes read one line.  Four indices of
+  // given ids at K = 4096 are faster with the group slots fastest (one to four
+  // pairs of 128 experts: 4.8 to 5.4 us against 4.9 to 5.7; the same launch with
+  // the top-k in it 5.1 to 6.4 against 5.1 to 6.1, so that keeps the rows).
+  constexpr bool kRowsFast = RG == 8 || NV == 1 || PER > 0;
+  const int r = kRowsFast ? lane & 7 : lane >> 3, sl = kRowsFast ? lane >> 3 : lane & 7;
   const int jr = RG == 8 ? 0 : r >> 2;        // RG = 4: the lane's half (gate or up)
   const int rr = RG == 8 ? r : (r & 3);       // row within the wave's RG rows
   const uint32_t item = xcd_item(blockIdx.x, gridDim.x);
@@ -1169,6 +1174,11 @@ __global__ __launch_bounds__(64 * W) void qmv64_paired_lines_kernel(QmvArgs a) {
   if constexpr (RG == 8) {
     gate = sum_slots(acc[0]);
     up = sum_slots(acc[1]);
+  } else if constexpr (!kRowsFast) {
+    // lanes 8r, r < 4: gate row r; r >= 4: up row r - 4, 32 lanes above
+    gate = sum8(acc[0]);
+    const auto sw = __builtin_amdgcn_permlane32_swap(as_u(gate), as_u(gate), false, false);
+    up = as_f(sw[1]);
   } else {
     // r < 4: gate row r; r >= 4: up row r - 4, four lanes above (row_ror:4 of a value of period 8)
     gate = sum_slots(acc[0]);
