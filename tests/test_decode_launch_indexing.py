@@ -192,13 +192,12 @@ def test_single_wave_indexing_overruns_in_wider_workgroups(W):
 PAIRED_RG = int(re.search(r"#define QMOE_PAIRED_LINES_RG (\d+)", SRC.read_text()).group(1))
 
 
-def paired_lines_accesses(E, T, k, n_out, NV, W=1, RG=None):
+def paired_lines_accesses(E, T, k, n_out, NV, RG=None, W=1):
     """Byte ranges each buffer sees from one launch of qmv64_paired_lines_kernel
-    (tile-layout gate_up + SwiGLU, the form that takes expert ids): one 64-lane
-    wave per workgroup, item = xcd_item(block, grid), as launch_qmv_paired
-    sizes the grid.  (W > 1 models W waves per workgroup, item =
-    xcd_item(block) * W + wave, with per-wave LDS staging and waves past the
-    last item leaving.)"""
+    (tile-layout gate_up + SwiGLU, the form that takes expert ids): W waves of
+    one pair per workgroup, item = xcd_item(block, grid), the waves' indices
+    consecutive, as launch_qmv_lines sizes the grid.  One wave stages x a chunk
+    per lane, more a 16-byte piece per thread and step."""
     RG = RG or PAIRED_RG
     NCH, NP, NJ = 64 * NV, 4 * NV, RG // 4
     K = 2048 * NV
@@ -206,32 +205,35 @@ def paired_lines_accesses(E, T, k, n_out, NV, W=1, RG=None):
     n_w = 2 * n_out
     NC = n_w // 64
     n_pairs = T * k
-    nblk = n_out // RG
-    nitems = n_pairs * nblk
-    blocks = (nitems + W - 1) // W
+    nblk = n_out // (RG * W)
+    blocks = n_pairs * nblk
     threads = 64 * W
     b = np.repeat(np.arange(blocks, dtype=np.int64), threads)
     t = np.tile(np.arange(threads, dtype=np.int64), blocks)
     lane, wave = t % 64, t // 64
-    item = xcd_item(b, blocks) * W + wave if W > 1 else xcd_item(b, blocks)
-    live = item < nitems
-    lane, wave, item = lane[live], wave[live], item[live]
-    r, sl = lane >> 3, lane & 7
+    item = xcd_item(b, blocks)
+    # rows fastest, but for four indices of given ids at K = 4096
+    r, sl = (lane & 7, lane >> 3) if RG == 8 or NV == 1 else (lane >> 3, lane & 7)
     jr = np.zeros_like(r) if RG == 8 else r >> 2
     rr = r if RG == 8 else r & 3
     pr = item // nblk
-    i0 = (item - pr * nblk) * RG
+    i0 = ((item - pr * nblk) * W + wave) * RG
     xr = pr // k
     ids = (E - 1 - 7 * np.arange(n_pairs, dtype=np.int64)) % E
     e = ids[pr]
     c, l0 = i0 >> 5, i0 & 31
     cbase = (e * NC + c) * G
     acc = {"experts": [(pr * 4, pr * 4 + 4)], "x": [], "w": [], "sb": [], "lds": [], "out": []}
-    for v in range(NV):
-        lo = (xr * K + v * 2048 + lane * 32) * 2
-        acc["x"].append((lo, lo + 64))
-        for q in range(4):
-            lds = ((wave * 4 + q) * NCH + v * 64 + lane) * 16
+    for v in range(NV if W == 1 else 4 * NCH // threads):
+        if W == 1:
+            chunk, quarters = v * 64 + lane, range(4)
+        else:
+            u = v * threads + t
+            chunk, quarters = u // 4, [u % 4]
+        for q in quarters:
+            lo = xr * K * 2 + chunk * 64 + q * 16
+            acc["x"].append((lo, lo + 16))
+            lds = (q * NCH + chunk) * 16
             acc["lds"].append((lds, lds + 16))
     for pp in range(NP):
         chunk = cbase + 8 * pp + sl
@@ -245,13 +247,13 @@ def paired_lines_accesses(E, T, k, n_out, NV, W=1, RG=None):
     o = pr[m] * n_out + i0[m] + r[m]
     acc["out"].append((o * 2, o * 2 + 2))
     ext = {"experts": n_pairs * 4, "x": T * K * 2, "w": E * n_w * K // 2, "sb": E * NC * G * 64 * 4,
-           "lds": W * 4 * NCH * 16, "out": n_pairs * n_out * 2}
+           "lds": 4 * NCH * 16, "out": n_pairs * n_out * 2}
     return acc, ext
 
 
 PAIRED_SHAPES = [
     # E, tokens, top_k, I, NV: workload 1's block shape, two tokens, K = 4096,
-    # an item count that is not a multiple of W, and few experts
+    # an item count that is not a multiple of the XCDs, and few experts
     (256, 1, 10, 512, 1),
     (256, 2, 10, 512, 1),
     (256, 1, 8, 512, 2),
@@ -260,16 +262,22 @@ PAIRED_SHAPES = [
 ]
 
 
+# indices per wave and waves per workgroup, as launch_qmv_paired picks them
+PAIRED_FORMS = [(PAIRED_RG, 1), (8, 1), (8, 4)]
+
+
+@pytest.mark.parametrize("RG,W", PAIRED_FORMS)
 @pytest.mark.parametrize("E,T,k,n_out,NV", PAIRED_SHAPES)
-def test_paired_lines_kernel_accesses_in_bounds(E, T, k, n_out, NV):
-    acc, ext = paired_lines_accesses(E, T, k, n_out, NV)
+def test_paired_lines_kernel_accesses_in_bounds(E, T, k, n_out, NV, RG, W):
+    acc, ext = paired_lines_accesses(E, T, k, n_out, NV, RG, W)
     for name, (lo, over) in overruns(acc, ext).items():
         assert lo >= 0, (name, lo)
         assert over <= 0, (name, over)
 
 
+@pytest.mark.parametrize("RG,W", PAIRED_FORMS)
 @pytest.mark.parametrize("E,T,k,n_out,NV", PAIRED_SHAPES)
-def test_paired_lines_kernel_covers_every_output_once(E, T, k, n_out, NV):
-    acc, _ = paired_lines_accesses(E, T, k, n_out, NV)
+def test_paired_lines_kernel_covers_every_output_once(E, T, k, n_out, NV, RG, W):
+    acc, _ = paired_lines_accesses(E, T, k, n_out, NV, RG, W)
     stores = np.concatenate([r[0] for r in acc["out"]]) // 2
     assert np.array_equal(np.sort(stores), np.arange(T * k * n_out))

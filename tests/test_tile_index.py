@@ -231,9 +231,10 @@ def test_tiled_down_reads_the_mlx_words(R):
 
 @pytest.mark.parametrize("K,I,E,RG", [(2048, 512, 3, 8), (4096, 64, 2, 8), (2048, 96, 2, 4), (4096, 32, 2, 4)])
 def test_paired_lines_kernel_reads_the_mlx_words(K, I, E, RG):
-    """qmv64_paired_lines_kernel: lane 8r + s, step p, half h, j: unit
-    (g = 8p + s, j, h, l0 + r) -- the row's 32 codes of group g, half h -- and
-    the matching x chunk 2g + h and scale|bias word 32j + l0 + r."""
+    """qmv64_paired_lines_kernel: lane 8s + r (8r + s for four indices of K = 4096),
+    step p, half h, j: unit (g = 8p + s, j, h, l0 + r) -- the row's 32 codes of
+    group g, half h -- and the matching x chunk 2g + h and scale|bias word
+    32j + l0 + r."""
     rng = np.random.default_rng(K * 3 + I)
     w, s, b = synth.quant_weights(rng, (E, 2 * I), K)
     perm = pair_rows(I)
@@ -251,7 +252,7 @@ def test_paired_lines_kernel_reads_the_mlx_words(K, I, E, RG):
         c, l0 = i0 >> 5, i0 & 31
         cbase = (e * NC + c) * G
         for lane in range(64):
-            r, sl = lane >> 3, lane & 7
+            r, sl = (lane & 7, lane >> 3) if RG == 8 or NV == 1 else (lane >> 3, lane & 7)
             jr, rr = (0, r) if RG == 8 else (r >> 2, r & 3)
             halves = (0, 1) if RG == 8 else (jr,)
             for pp in range(4 * NV):
