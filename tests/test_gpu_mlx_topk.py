@@ -53,3 +53,25 @@ def test_block_decode_over_mlx_weights(dev, T, resident, I, shared):
     else:  # one rounding of the sum where the parts' sum has two
         both = ref.double() + block.shared_expert(x).double()
         assert bool(((y.double() - both).abs() <= 2.0 ** -7 * both.abs().max()).all())
+
+
+# both sides of the lines between the selecting gate_up and a top-k launch: 256 |
+# 257 experts, top-16 | 17 and 64 pairs below, top-4 | 5 and 16 pairs above
+@pytest.mark.parametrize("E,k,T,selects", [
+    (256, 10, 6, True), (256, 16, 3, True), (256, 17, 1, False), (64, 8, 8, False), (64, 63, 1, False),
+    (257, 4, 4, True), (257, 4, 5, False), (512, 5, 1, False), (512, 10, 1, False), (1024, 1, 16, True)])
+def test_block_decode_over_mlx_weights_selects_where_it_pays(dev, E, k, T, selects, monkeypatch):
+    print(f"[case] MLX-layout block decode E={E} k={k} T={T}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(E + k + T)
+    H, I = 2048, 128
+    gu, dn = _quant(g, (E, 2 * I), H, dev), _quant(g, (E, H), I, dev)
+    router = (torch.randn(E, H, device=dev, generator=g) * H ** -0.5).to(torch.bfloat16)
+    block = SparseMoeBlock(router, gu, dn, k, resident="both", sort_min_pairs=1 << 20)
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    calls = []
+    fused, plain = ops.gate_up_silu_topk, ops.router_topk
+    monkeypatch.setattr(ops, "gate_up_silu_topk", lambda *a, **kw: calls.append(True) or fused(*a, **kw))
+    monkeypatch.setattr(ops, "router_topk", lambda *a, **kw: calls.append(False) or plain(*a, **kw))
+    y = block(x)
+    assert calls == [selects]
+    assert torch.equal(y, block.experts(x, *block.route(x)))

@@ -146,7 +146,7 @@ class SparseMoeBlock:
                                                                                group_size, bits, self.top_k)
         self.gate_up = None if self.decode_tiles else tuple(gate_up)
         self.down = None if self.decode_tiles else tuple(down)
-        # MLX-layout decode whose gate_up kernel picks the experts itself
+        # MLX-layout decode whose gate_up kernel can pick the experts itself
         self._mlx_topk = self.gate_up is not None and ops.gate_up_topk_supported(
             self.hidden, self.num_experts, self.top_k, group_size, bits)
         # the sorted (grouped GEMM) path from this many (token, expert) pairs
@@ -285,6 +285,20 @@ class SparseMoeBlock:
         return (self.decode_tiles and T <= 16 and T * self.top_k < self.sort_min_pairs
                 and self.num_experts <= 1024)
 
+    def _mlx_selects(self, T: int) -> bool:
+        """Does a decode call over the MLX tensors let the gate_up kernel pick the
+        experts?  Each wave of slot j walks j + 1 rounds of the selection, over 4
+        logits per lane up to 256 experts and 16 above, against one launch of
+        router_topk.  The launches' time with / without it, hidden 2048 and 4096,
+        widths 512 to 1536, below 64 pairs: up to 256 experts 0.72-1.00 to top-10,
+        0.75-1.02 at top-16, 0.80-1.07 at top-32, 0.93-1.23 at top-64 (from 64 pairs on
+        0.88-1.11 to top-16); 512 experts 0.76-0.94 up to 16 pairs of top-4 at most,
+        0.86-1.07 beyond these, 0.94-1.27 at top-8 and top-10."""
+        pairs = T * self.top_k
+        if self.num_experts <= 256:
+            return self.top_k <= 16 and pairs < 64
+        return self.top_k <= 4 and pairs <= 16
+
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         H = x.shape[-1]
         x2 = x.reshape(-1, H).to(torch.bfloat16).contiguous()
@@ -300,7 +314,7 @@ class SparseMoeBlock:
             h, idx, scores = ops.gate_up_silu_tiles_topk(x2, self.gu_tiles, self.route_logits(x2), self.top_k,
                                                          self.norm)
             y = ops.down_wsum_tiles(h, self.down_tiles, idx, scores)
-        elif self._mlx_topk and T <= 16 and T * self.top_k < self.sort_min_pairs:
+        elif self._mlx_topk and T <= 16 and T * self.top_k < self.sort_min_pairs and self._mlx_selects(T):
             h, idx, scores = ops.gate_up_silu_topk(x2, *self.gate_up, self.route_logits(x2), self.top_k, self.norm)
             y = ops.down_wsum(h, *self.down, idx, scores, self.group_size, self.bits)
         else:
