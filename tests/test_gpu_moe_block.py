@@ -455,3 +455,23 @@ def test_moe_block_graph_replays(dev, T, with_shared):
         assert torch.equal(static_y, want[i]), (T, with_shared, rep)
         blk(xs[(i + 1) % len(xs)])  # eager work between replays
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("shape", [(6, 50), (300,), (1, 3, 100)])
+def test_experts_take_ids_of_several_token_dimensions(dev, shape):
+    """The sorted path flattens its ids and scores, whatever their token dimensions."""
+    say(f"experts with ids over tokens {shape}")
+    g = torch.Generator(device=dev).manual_seed(5)
+    E, H, I, T = 16, 512, 256, 300
+
+    def quant(N, K):
+        w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K // 8), dtype=torch.int32, device=dev, generator=g)
+        s = (0.004 + 0.004 * torch.rand(E, N, K // 64, device=dev, generator=g)).to(torch.bfloat16)
+        return w, s, (-7.5 * s.float()).to(torch.bfloat16)
+
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    block = moe_block.SparseMoeBlock(torch.randn(E, H, device=dev, generator=g).to(torch.bfloat16), quant(2 * I, H),
+                                     quant(H, I), 4)
+    idx, sc = block.route(x)
+    y = block.experts(x, idx, sc)
+    assert torch.equal(block.experts(x, idx.reshape(*shape, 4), sc.reshape(*shape, 4)), y)

@@ -201,7 +201,8 @@ class SparseMoeBlock:
 
     # ------------------------------------------------------------- experts
     def experts(self, x2: torch.Tensor, idx: torch.Tensor, scores: torch.Tensor) -> torch.Tensor:
-        """sum_j scores[t, j] * expert_{idx[t, j]}(x2[t]) for x2 [T, H]."""
+        """sum_j scores[t, j] * expert_{idx[t, j]}(x2[t]) for x2 [T, H]; idx and
+        scores [T, k], or with T in several dimensions."""
         T = x2.shape[0]
         k = idx.shape[-1]
         decode = T * k < self.sort_min_pairs and T <= 16
@@ -219,7 +220,7 @@ class SparseMoeBlock:
             r = ops.route(idx, self.num_experts)
             x_rows, inv, tiles = torch.div(r.order, k, rounding_mode="floor").to(torch.int32), r.inv_order, r.tiles
         else:
-            x_rows, inv, tiles = ops.route_block(idx, self.num_experts)
+            x_rows, inv, tiles = ops.route_block(idx.reshape(-1, k), self.num_experts)
         h = ops.gather_qmm_swiglu_sorted_tiles(x2, self.gu_tiles, tiles, x_rows=x_rows)
         yd = ops.gather_qmm_sorted_tiles(h, self.down_tiles, tiles)
         return ops.moe_weighted_sum(yd, inv, scores, (T, self.hidden), self.wsum_mode)
