@@ -230,3 +230,40 @@ def test_tiles_of_sorted_ids(dev, n, E):
         assert int(t.ntiles) == int(per.sum())
         exp = torch.repeat_interleave(torch.arange(E, device=dev), per)
         assert torch.equal(t.tile_exp[:exp.numel()].long(), exp)
+
+
+def _block_weights(g, dev, E, H, I):
+    return ((torch.randn(E, H, device=dev, generator=g) * H ** -0.5).to(torch.bfloat16), _quant(g, (E, 2 * I), H, dev),
+            _quant(g, (E, H), I, dev))
+
+
+def _shared64(x, sgu, sdn, z):
+    """sigmoid(z) * SwiGLU-MLP(x) in 64 bits, over the exact affine weights up to
+    16 tokens and bf16-materialised ones above, as the block takes them."""
+    wgu, wdn = (_deq64(q)[0] if x.shape[0] <= 16 else _deq64(q)[0].to(torch.bfloat16).double() for q in (sgu, sdn))
+    a, u = (x.double() @ wgu.t()).chunk(2, dim=-1)
+    return torch.sigmoid(z) * ((torch.nn.functional.silu(a) * u) @ wdn.t())
+
+
+@pytest.mark.parametrize("T", [1, 16, 17, 100])
+@pytest.mark.parametrize("S,resident", [(512, "tiles"), (512, "both"), (256, "tiles")])
+def test_shared_expert_with_a_quantized_gate(dev, T, S, resident):
+    """A gate of codes, which router_logits takes, over every dispatch."""
+    print(f"[case] quantized gate T={T} S={S} {resident}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T + S)
+    E, H, I, k = 32, 2048, 512, 4
+    router, gu, dn = _block_weights(g, dev, E, H, I)
+    sgu, sdn = _quant(g, (1, 2 * S), H, dev), _quant(g, (1, H), S, dev)
+    gate = _quant(g, (1,), H, dev)
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    block = SparseMoeBlock(router, gu, dn, k, resident=resident, shared=SharedExpert(sgu, sdn, gate))
+    y = block(x)
+    idx, sc = block.route(x)
+    routed, shared = block.experts(x, idx, sc).double(), _shared64(x, sgu, sdn, x.double() @ _deq64(gate).t())
+    # bf16 roundings, 2^-9 of a value each: of h (the down product of errors of
+    # independent signs grows no faster than that of h itself), of the shared
+    # expert's rows before and after the gate, and of the sum
+    err = (y.double() - routed - shared).norm()
+    bound = 2.0 ** -9 * (3 * shared.norm() + (routed + shared).norm())
+    print(f"[parity] err/bound {float(err / bound):.3g}", flush=True)
+    assert float(err) <= float(bound)

@@ -84,11 +84,12 @@ def tile_decode_supported(hidden: int, inter: int, group_size: int = ops.GROUP, 
 class SharedExpert:
     """Dense quantized SwiGLU MLP and its scalar gate (language.py:51-53, 81-89):
     gate_up (w, s, b) [1, 2S, H*bits/32] gate rows first, down (w, s, b)
-    [1, H, S*bits/32], gate weight bf16 [1, H]."""
+    [1, H, S*bits/32], gate weight bf16 [1, H] or, as router_logits takes it, a
+    4-bit group-64 (w, s, b) of one row."""
 
     gate_up: tuple
     down: tuple
-    gate_weight: torch.Tensor
+    gate_weight: torch.Tensor | tuple
 
 
 class SparseMoeBlock:
@@ -162,17 +163,19 @@ class SparseMoeBlock:
             if self.resident == "tiles" and tile_decode_supported(self.hidden, S, group_size, bits):
                 self._shared_decode_tiles = True
                 self.shared = SharedExpert(None, None, shared.gate_weight)
+        # a dense gate row is read by the kernels that score the shared expert;
+        # any other gate goes through router_logits
+        self._gate_row = (shared is not None and isinstance(shared.gate_weight, torch.Tensor)
+                          and shared.gate_weight.numel() == self.hidden)
         # a shared expert of the routed experts' shape is one more slot of the
         # decode kernels (qmoe_moe_*_shared)
         self._shared_slot = (self.decode_tiles and self._shared_decode_tiles and self.top_k < TILE_DECODE_MAX_K
-                             and self._shared_tiles[0].N == self.gu_tiles.N
-                             and shared.gate_weight.numel() == self.hidden)
+                             and self._shared_tiles[0].N == self.gu_tiles.N and self._gate_row)
         # and one more expert of the sorted path's GEMMs
         self._shared_expert_rows = (self._shared_tiles is not None and self._shared_tiles[0].N == self.gu_tiles.N
-                                    and shared.gate_weight.numel() == self.hidden
-                                    and self.num_experts <= ROUTE_BLOCK_MAX_E)
+                                    and self._gate_row and self.num_experts <= ROUTE_BLOCK_MAX_E)
         if shared is not None:  # constant ids and scores of the shared expert's decode kernels
-            dev = shared.gate_weight.device
+            dev = gate_up[0].device
             self._zeros = torch.zeros(16, 1, dtype=torch.int32, device=dev)
             self._ones = torch.ones(16, 1, dtype=torch.float32, device=dev)
 
@@ -322,9 +325,8 @@ class SparseMoeBlock:
             idx, scores = self.route(x2)
             y = self.experts(x2, idx, scores)
         if self.shared is not None:
-            gate = self.shared.gate_weight
-            if gate.numel() == self.hidden and self.hidden % 8 == 0:
-                y = ops.shared_combine(y, self._shared_mlp(x2), x2, gate)
+            if self._gate_row:
+                y = ops.shared_combine(y, self._shared_mlp(x2), x2, self.shared.gate_weight)
             else:
                 y = (y.float() + self.shared_expert(x2).float()).to(torch.bfloat16)
         return y.reshape(x.shape)
