@@ -16,6 +16,13 @@ def _quant(g, lead, K, dev):
     return w, s, (-7.5 * s.float()).to(torch.bfloat16)
 
 
+def _deq64(q):
+    w, s, b = q
+    shifts = torch.arange(0, 32, 4, device=w.device, dtype=torch.int32)
+    c = ((w.unsqueeze(-1) >> shifts) & 15).reshape(*w.shape[:-1], -1).double()
+    return c * s.double().repeat_interleave(64, -1) + b.double().repeat_interleave(64, -1)
+
+
 @pytest.mark.parametrize("norm", [True, False])
 @pytest.mark.parametrize("T,k,E,K,I", [(1, 8, 128, 2048, 768), (3, 1, 1, 2048, 6), (16, 64, 64, 2048, 33),
                                        (2, 10, 600, 4096, 64), (5, 20, 256, 4096, 12)])
@@ -50,8 +57,10 @@ def test_block_decode_over_mlx_weights(dev, T, resident, I, shared):
     ref = block.experts(x, idx, sc)
     if not shared:
         assert torch.equal(y, ref)
-    else:  # one rounding of the sum where the parts' sum has two
-        both = ref.double() + block.shared_expert(x).double()
+    else:  # the routed part's rounding, h's and the sum's, against the shared expert in 64 bits
+        a, u = (x.double() @ _deq64(sgu)[0].t()).chunk(2, dim=-1)
+        mlp = (torch.nn.functional.silu(a) * u) @ _deq64(sdn)[0].t()
+        both = ref.double() + torch.sigmoid(x.double() @ gate.double().t()) * mlp
         assert bool(((y.double() - both).abs() <= 2.0 ** -7 * both.abs().max()).all())
 
 

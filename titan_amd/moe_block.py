@@ -52,7 +52,7 @@ from dataclasses import dataclass
 
 import torch
 
-from . import ops
+from . import _lib, ops
 
 __all__ = ["SparseMoeBlock", "SharedExpert", "DECODE_MAX_PAIRS", "ROUTER_GEMV_MAX_T", "TILE_DECODE_MAX_K",
            "tile_decode_supported"]
@@ -252,6 +252,8 @@ class SparseMoeBlock:
             gu_t, dn_t = self._shared_tiles
             tiles = ops.build_tiles(torch.zeros(T, dtype=torch.int32, device=x2.device), 1)
             return ops.gather_qmm_sorted_tiles(ops.gather_qmm_swiglu_sorted_tiles(x2, gu_t, tiles), dn_t, tiles)
+        if T > 16:
+            raise ops.QmoeUnsupported(_lib.ERR_UNSUPPORTED, "the shared expert's decode kernels take at most 16 tokens")
         zeros, ones = self._zeros[:T], self._ones[:T]
         if self._shared_decode_tiles:
             gu_t, dn_t = self._shared_tiles
@@ -262,24 +264,8 @@ class SparseMoeBlock:
 
     def shared_expert(self, x2: torch.Tensor) -> torch.Tensor:
         """sigmoid(x w_gate) * SwiGLU-MLP(x) (language.py:81-89)."""
-        sh = self.shared
-        T = x2.shape[0]
-        zeros = torch.zeros(T, 1, dtype=torch.int32, device=x2.device)
-        ones = torch.ones(T, 1, dtype=torch.float32, device=x2.device)
-        if T <= 16 and self._shared_decode_tiles:  # the fused down kernel takes up to 16 tokens
-            gu_t, dn_t = self._shared_tiles
-            h = ops.gate_up_silu_tiles(x2, gu_t, zeros)
-            y = ops.down_wsum_tiles(h, dn_t, zeros, ones)
-        elif T <= 16 or self._shared_tiles is None:
-            h = ops.gate_up_silu(x2, *sh.gate_up, zeros, self.group_size, self.bits)
-            y = ops.down_wsum(h, *sh.down, zeros, ones, self.group_size, self.bits)
-        else:
-            gu_t, dn_t = self._shared_tiles
-            tiles = ops.build_tiles(zeros.reshape(-1), 1)
-            h = ops.gather_qmm_swiglu_sorted_tiles(x2, gu_t, tiles)
-            y = ops.gather_qmm_sorted_tiles(h, dn_t, tiles)
-        z = ops.router_logits(x2, sh.gate_weight)
-        return (torch.sigmoid(z) * y.float()).to(torch.bfloat16)
+        z = ops.router_logits(x2, self.shared.gate_weight)
+        return (torch.sigmoid(z) * self._shared_mlp(x2).float()).to(torch.bfloat16)
 
     def decodes_with_topk(self, T: int) -> bool:
         """Does a call with T tokens take the gate_up decode kernel that picks
