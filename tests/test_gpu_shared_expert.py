@@ -267,3 +267,58 @@ def test_shared_expert_with_a_quantized_gate(dev, T, S, resident):
     bound = 2.0 ** -9 * (3 * shared.norm() + (routed + shared).norm())
     print(f"[parity] err/bound {float(err / bound):.3g}", flush=True)
     assert float(err) <= float(bound)
+
+
+@pytest.mark.parametrize("T", [2, 40])
+@pytest.mark.parametrize("resident,shared", [("tiles", True), ("both", True), ("both", False)])
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
+def test_replaced_steps_are_called(dev, T, resident, shared, how, monkeypatch):
+    """route, experts and shared_expert of a subclass, an instance or the patched
+    class run where the block's own would, and make the result."""
+    print(f"[case] replaced steps T={T} {resident} shared={shared} {how}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T)
+    E, H, I, k = 32, 2048, 512, 4
+    router, gu, dn = _block_weights(g, dev, E, H, I)
+    sh = SharedExpert(_quant(g, (1, 2 * I), H, dev), _quant(g, (1, H), I, dev),
+                      (torch.randn(1, H, device=dev, generator=g) * H ** -0.5).to(torch.bfloat16)) if shared else None
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    plain = SparseMoeBlock(router, gu, dn, k, resident=resident, shared=sh)
+    calls = []
+
+    def route(self, x2):
+        calls.append("route")
+        idx, scores = SparseMoeBlock_route(self, x2)
+        return idx.flip(-1).contiguous(), 0.5 * scores
+
+    def experts(self, x2, idx, scores):
+        calls.append("experts")
+        return 2 * SparseMoeBlock_experts(self, x2, idx, scores)
+
+    def shared_expert(self, x2):
+        calls.append("shared_expert")
+        return 3 * SparseMoeBlock_shared(self, x2)
+
+    SparseMoeBlock_route, SparseMoeBlock_experts = SparseMoeBlock.route, SparseMoeBlock.experts
+    SparseMoeBlock_shared = SparseMoeBlock.shared_expert
+    steps = {"route": route, "experts": experts, "shared_expert": shared_expert}
+    block = plain
+    if how == "subclass":
+        block = type("Mine", (SparseMoeBlock,), steps)(router, gu, dn, k, resident=resident, shared=sh)
+    elif how == "class":
+        for name, step in steps.items():
+            monkeypatch.setattr(SparseMoeBlock, name, step)
+    else:
+        for name, step in steps.items():
+            monkeypatch.setattr(block, name, lambda *a, step=step: step(block, *a))
+    y = block(x)
+    # the tile-layout decode call has its two launches in the place of route and experts
+    routed = not (resident == "tiles" and T == 2)
+    assert calls == ["route", "experts"] * routed + ["shared_expert"] * shared
+    if routed:
+        idx, scores = SparseMoeBlock_route(block, x)
+        ref = 2 * SparseMoeBlock_experts(block, x, idx.flip(-1).contiguous(), 0.5 * scores)
+    else:
+        ref = SparseMoeBlock_experts(block, x, *SparseMoeBlock_route(block, x))
+    if shared:
+        ref = (ref.float() + (3 * SparseMoeBlock_shared(block, x)).float()).to(torch.bfloat16)
+    assert torch.equal(y, ref)
