@@ -140,7 +140,11 @@ def test_route_block_matches_route(dev, T, k, E):
             assert m == nt and t.rows == n
 
 
-@pytest.mark.parametrize("T,E", [(17, 4), (128, 3), (129, 3), (300, 40)])
+# (tile kernel; then, at six rows per expert or fewer, the rows kernel up to 320
+# rows and either kernel past them, the shared expert's tiles of one to four
+# subtiles and two tiles)
+@pytest.mark.parametrize("T,E", [(17, 4), (128, 3), (129, 3), (300, 40), (17, 40), (33, 60), (65, 40), (100, 60),
+                                 (129, 100), (140, 200), (200, 300)])
 def test_gemm_with_shared_expert_is_the_two_gemms(dev, T, E):
     """Both epilogues over a table whose last expert is a tensor of its own:
     bit for bit the routed GEMM and the shared expert's own."""
