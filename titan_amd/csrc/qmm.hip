@@ -4,14 +4,16 @@
 //
 // The GEMV (qmv.hip) streams the weights once per row of x; here each weight
 // is read once per 16 * MT rows.  The codes go to the matrix cores as they
-// are -- 4-bit codes as the bf16 values 128 + q (0x4300 | q), 8-bit codes as
+// are -- 4-bit codes as the bf16 values 1 + q / 128 (0x3F80 | q), 8-bit codes as
 // the integers 0..255, all exact -- and the group's scale and bias are applied
 // to the products' sums in fp32, so nothing is rounded to bf16 before the
 // result, as in the GEMV:
 //   acc += s * sum_k x q + b * sum_k x            per group
 // with sum_k x from the same matrix instruction over a constant: for 4 bits
-// the constant is -128, so that the sum is also what the products start from
-// (sum x (128 + q) - 128 sum x).
+// the constant is -1, so that the sum is also what the products start from
+// (sum x (1 + q / 128) - sum x), and the scale is multiplied by 128.  (128 + q
+// would do without that and give the same bits, but 128 sum x overflows from
+// sums of 2.7e36 on.)
 //
 // Work: a block owns 16 output columns of 16 * MT rows and its eight waves
 // take the K = 256 batches (four 64-column units) in turn; their partial sums
@@ -67,9 +69,9 @@ __device__ __forceinline__ u32x4_t pair_nibbles(const u32x4_t& a) {
   return u32x4_t{__builtin_amdgcn_perm(a[2], a[0], 0x05040100u), __builtin_amdgcn_perm(a[2], a[0], 0x07060302u),
                  __builtin_amdgcn_perm(a[3], a[1], 0x05040100u), __builtin_amdgcn_perm(a[3], a[1], 0x07060302u)};
 }
-// the eight 4-bit codes of a word as bf16 128 + q, in that order
+// the eight 4-bit codes of a word as bf16 1 + q / 128, in that order
 __device__ __forceinline__ u32x4_t codes4(uint32_t v) {
-  constexpr uint32_t m = 0x000F000Fu, c = 0x43004300u;
+  constexpr uint32_t m = 0x000F000Fu, c = 0x3F803F80u;
   return u32x4_t{(v & m) | c, ((v >> 4) & m) | c, ((v >> 8) & m) | c, ((v >> 12) & m) | c};
 }
 // eight 8-bit codes of two words as bf16 integers (exact: the float's top half)
@@ -159,7 +161,7 @@ __global__ __launch_bounds__(64 * kWaves) void qmm_kernel(QmmArgs a) {
     }
   };
 
-  const uint32_t one = BITS == 4 ? 0xC300C300u : 0x3F803F80u;  // bf16 -128 or 1
+  const uint32_t one = BITS == 4 ? 0xBF80BF80u : 0x3F803F80u;  // bf16 -1 or 1
   const u32x4_t ones = {one, one, one, one};
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   f32x4_t acc[MT];
@@ -232,8 +234,8 @@ __global__ __launch_bounds__(64 * kWaves) void qmm_kernel(QmmArgs a) {
 #pragma unroll
         for (int sg = 0; sg < SG; ++sg) {
           const uint32_t w = live ? sbj[j][sg] : 0u;
-          const float s = __uint_as_float(w << 16);
-          const float b = __uint_as_float(w & 0xFFFF0000u) * (BITS == 4 ? -0.0078125f : 1.0f);  // exact
+          const float s = __uint_as_float(w << 16) * (BITS == 4 ? 128.0f : 1.0f);  // exact
+          const float b = BITS == 4 ? -__uint_as_float(w & 0xFFFF0000u) : __uint_as_float(w & 0xFFFF0000u);
 #pragma unroll
           for (int i = 0; i < MT; ++i) {
             u32x4_t xf[2];
