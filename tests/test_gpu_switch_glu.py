@@ -72,3 +72,17 @@ def test_layer_over_its_kernels_and_without(dev, T, how, monkeypatch):
     y, ref = y.detach(), ref.detach()
     err = (y.double() - ref.double()).norm() / ref.double().norm()
     assert float(err) < 2.0 ** -9  # single ULPs of h, seldom
+
+
+@pytest.mark.parametrize("rows", [1, 63])
+def test_ids_of_more_rows_than_x_has_are_refused(dev, rows):
+    g = torch.Generator(device=dev).manual_seed(rows)
+    E, K, I, k = 16, 512, 256, 2
+    layer = SwitchGLU(QuantizedSwitchLinear(*_quant(g, (E, K), I, dev)),
+                      gate_up_proj=QuantizedSwitchLinear(*_quant(g, (E, 2 * I), K, dev)))
+    x = torch.randn(64, K, device=dev, generator=g).to(torch.bfloat16)
+    idx = torch.randint(0, E, (64, k), dtype=torch.int32, device=dev, generator=g)
+    with pytest.raises(IndexError, match="rows"):
+        layer(x[:rows], idx)
+    # more rows than ids are ignored, as indexing by the ids' rows does
+    assert torch.equal(layer(x, idx[:40]), layer(x[:40], idx[:40]))

@@ -19,6 +19,8 @@ use torch's stable argsort and the stock gather.
 
 from __future__ import annotations
 
+import math
+
 import torch
 from torch.autograd import forward_ad
 
@@ -60,6 +62,9 @@ def _gather_sort(x: torch.Tensor, indices: torch.Tensor, num_experts: int):
     (None off the GPU)."""
     M = indices.shape[-1]
     flat = indices.reshape(-1)
+    rows = math.prod(x.shape[:-2])
+    if flat.numel() > rows * M:
+        raise IndexError(f"ids of {flat.numel() // M} rows of {M}, x has {rows}")
     if flat.is_cuda:
         r = ops.route(flat, num_experts)
         order, inv, ids, tiles = r.order, r.inv_order, r.sorted_ids, r.tiles
