@@ -86,3 +86,30 @@ def test_ids_of_more_rows_than_x_has_are_refused(dev, rows):
         layer(x[:rows], idx)
     # more rows than ids are ignored, as indexing by the ids' rows does
     assert torch.equal(layer(x, idx[:40]), layer(x[:40], idx[:40]))
+
+
+@pytest.mark.parametrize("T", [3, 90])
+@pytest.mark.parametrize("what", ["function", "call"])
+def test_a_replaced_default_activation_runs(dev, T, what, monkeypatch):
+    """swiglu and SwiGLU.__call__ put in the place of the module's own."""
+    g = torch.Generator(device=dev).manual_seed(T)
+    E, K, I, k = 16, 512, 256, 4
+    layer = SwitchGLU(QuantizedSwitchLinear(*_quant(g, (E, K), I, dev)),
+                      gate_up_proj=QuantizedSwitchLinear(*_quant(g, (E, 2 * I), K, dev)))
+    x = torch.randn(T, K, device=dev, generator=g).to(torch.bfloat16)
+    idx = torch.randint(0, E, (T, k), dtype=torch.int32, device=dev, generator=g)
+    calls = []
+
+    def mine(gate, x):
+        calls.append(tuple(gate.shape))
+        return x - gate
+
+    if what == "function":
+        monkeypatch.setattr(switch_layers, "swiglu", mine)
+    else:
+        monkeypatch.setattr(SwiGLU, "__call__", lambda self, x, gate: mine(gate, x))
+    y = layer(x, idx)
+    assert len(calls) == 1
+    monkeypatch.undo()
+    layer.activation = lambda x, gate: x - gate
+    assert torch.equal(y, layer(x, idx))

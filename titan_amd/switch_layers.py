@@ -44,6 +44,15 @@ class SwiGLU:
         return swiglu(gate, x)
 
 
+def _default(activation) -> bool:
+    """Is ``activation`` the default module with nothing put in the place of its
+    expression, which ops.swiglu computes?"""
+    return type(activation) is SwiGLU and (SwiGLU.__call__, swiglu) == _DEFAULT
+
+
+_DEFAULT = (SwiGLU.__call__, swiglu)
+
+
 def _plain(t: torch.Tensor, width: int) -> bool:
     """May a kernel read ``t`` as it is, rows of ``width`` elements?  bf16 in GPU
     memory, contiguous, whole aligned 16-byte units per row, and nothing that has
@@ -172,7 +181,7 @@ class SwitchGLU:
             x, idx, inv_order, tiles = _gather_sort(x, indices, self.num_experts)
         if self.gate_up_proj is not None:
             gu = self.gate_up_proj(x, idx, sorted_indices=do_sort, tiles=tiles)
-            if type(self.activation) is SwiGLU and gu.shape[-1] % 2 == 0 and _plain(gu, gu.shape[-1] // 2):
+            if _default(self.activation) and gu.shape[-1] % 2 == 0 and _plain(gu, gu.shape[-1] // 2):
                 h = ops.swiglu(gu)
             else:
                 x_gate, x_up = gu.chunk(2, dim=-1)
