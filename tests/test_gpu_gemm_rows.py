@@ -74,3 +74,36 @@ def test_either_kernel_is_the_tile_kernel(dev, rows, E, N):
         y = gemm(x[:R], ops.repack_tiles(*w, swiglu_pairs=pairs), many_t)
         ref = gemm(x, ops.repack_tiles(*sub, swiglu_pairs=pairs), past_t)
         assert torch.equal(y, ref[:R])
+
+
+# T tokens of two experts each, one of them with an infinity or a NaN
+@pytest.mark.parametrize("v", ["inf", "-inf", "nan"])
+@pytest.mark.parametrize("T,E", [(40, 100), (170, 200)])
+def test_rows_kernel_with_infinities(dev, T, E, v):
+    """Such a row of x takes its own results with it and no other's, in the rows
+    kernel and in the one that holds both, as in the tile kernel."""
+    print(f"[case] rows kernel with {v} T={T} E={E}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T)
+    K, N, k = 256, 512, 2
+    x = torch.randn(T, K, device=dev, generator=g).to(torch.bfloat16)
+    idx = torch.randint(0, E, (T, k), dtype=torch.int32, device=dev, generator=g)
+    x_rows, _, few = ops.route_block(idx, E)
+    # the same rows in a table past the limit: many more of the last expert after them
+    more = 6 * E + 6
+    ids = torch.cat([idx.reshape(-1).long().sort()[0], torch.full((more,), E - 1, device=dev)]).to(torch.int32)
+    many = ops.build_tiles(ids, E)
+    rows2 = torch.cat([x_rows, torch.zeros(more, dtype=torch.int32, device=dev)])
+    w = _quant(g, (E, N), K, dev)
+    bad = x_rows == T // 2
+    for pairs in (False, True):
+        tw = ops.repack_tiles(*w, swiglu_pairs=pairs)
+        gemm = ops.gather_qmm_swiglu_sorted_tiles if pairs else ops.gather_qmm_sorted_tiles
+        y0 = gemm(x, tw, few, x_rows=x_rows)
+        xb = x.clone()
+        xb[T // 2, 5] = float(v)
+        y = gemm(xb, tw, few, x_rows=x_rows)
+        ref = gemm(xb, tw, many, x_rows=rows2)[:T * k]
+        assert torch.equal(y[~bad], y0[~bad])
+        assert torch.equal(y[bad].view(torch.int16), ref[bad].view(torch.int16))
+        if not pairs:  # (silu takes a gate of minus infinity to zero or NaN)
+            assert not bool(torch.isfinite(y[bad]).any())

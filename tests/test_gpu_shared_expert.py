@@ -326,3 +326,69 @@ def test_replaced_steps_are_called(dev, T, resident, shared, how, monkeypatch):
     if shared:
         ref = (ref.float() + (3 * SparseMoeBlock_shared(block, x)).float()).to(torch.bfloat16)
     assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("v", ["inf", "-inf", "nan"])
+def test_shared_slot_decode_with_infinities(dev, v):
+    """A token with an infinity or a NaN takes its own result with it and no
+    other's; its shared score is the sigmoid's limit, or NaN."""
+    print(f"[case] shared slot with {v}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(9)
+    E, H, I, k, T = 24, 2048, 512, 4, 5
+    router, gu, dn = _block_weights(g, dev, E, H, I)
+    sgu, sdn = _quant(g, (1, 2 * I), H, dev), _quant(g, (1, H), I, dev)
+    gate = (torch.randn(1, H, device=dev, generator=g) * H ** -0.5).to(torch.bfloat16)
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    logits = torch.randn(T, E, device=dev, generator=g)
+    tw, stw = ops.repack_tiles(*gu, swiglu_pairs=True), ops.repack_tiles(*sgu, swiglu_pairs=True)
+    td, std = ops.repack_tiles(*dn), ops.repack_tiles(*sdn)
+
+    def run(x):
+        h, idx, sc = ops.gate_up_silu_tiles_topk_shared(x, tw, logits, k, stw, gate)
+        return h, idx, sc, ops.down_wsum_tiles_shared(h, td, idx, sc, std)
+
+    h0, idx0, sc0, y0 = run(x)
+    xb = x.clone()
+    xb[2, 7] = float(v)
+    h, idx, sc, y = run(xb)
+    assert torch.equal(idx, idx0) and torch.equal(sc[:, :k], sc0[:, :k])
+    rest = torch.tensor([0, 1, 3, 4], device=dev)
+    assert torch.equal(h[rest], h0[rest]) and torch.equal(sc[rest], sc0[rest]) and torch.equal(y[rest], y0[rest])
+    z = float(v) * float(gate[0, 7])  # the rest of the logit is finite
+    lim = torch.sigmoid(torch.tensor(z))
+    assert bool(torch.isnan(sc[2, k])) if v == "nan" else float(sc[2, k]) == float(lim)
+    # the kernel that takes ids, slot for slot
+    hi = ops.gate_up_silu_tiles(xb, tw, idx[:, :k].contiguous())
+    assert torch.equal(h[:, :k].contiguous().view(torch.int16), hi.view(torch.int16))
+    assert not bool(torch.isfinite(y[2]).any())
+
+
+@pytest.mark.parametrize("E", [100, 600])
+def test_selection_of_infinite_and_nan_logits(dev, E):
+    """The kernels that select by themselves choose as router_topk does where
+    logits are NaN, infinite, the lowest value or all equal."""
+    print(f"[case] selection of infinite logits E={E}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(E)
+    H, I, k, T = 2048, 512, 6, 8
+    gu, sgu = _quant(g, (E, 2 * I), H, dev), _quant(g, (1, 2 * I), H, dev)
+    gate = torch.randn(1, H, device=dev, generator=g).to(torch.bfloat16)
+    x = torch.randn(T, H, device=dev, generator=g).to(torch.bfloat16)
+    lg = torch.randn(T, E, device=dev, generator=g)
+    lg[0, ::2] = float("nan")
+    lg[1, 1:] = float("nan")
+    lg[2, 5:] = float("-inf")
+    lg[3] = float("-inf")
+    lg[4, [1, 7]] = float("inf")
+    lg[5] = torch.finfo(torch.float32).min
+    lg[6] = 0.0
+    lg[7] = float("nan")
+    for norm in (True, False):
+        idx, sc = ops.router_topk(lg, k, norm)
+        bits = sc.view(torch.int32)
+        _, i1, s1 = ops.gate_up_silu_topk(x, *gu, lg, k, norm)
+        assert torch.equal(i1, idx) and torch.equal(s1.view(torch.int32), bits)
+        tw, stw = ops.repack_tiles(*gu, swiglu_pairs=True), ops.repack_tiles(*sgu, swiglu_pairs=True)
+        _, i2, s2 = ops.gate_up_silu_tiles_topk_shared(x, tw, lg, k, stw, gate, norm)
+        assert torch.equal(i2[:, :k], idx) and torch.equal(s2[:, :k].contiguous().view(torch.int32), bits)
+        i3, s3 = ops.router_topk_shared(lg, k, x, gate, norm)
+        assert torch.equal(i3, idx) and torch.equal(s3[:, :k].contiguous().view(torch.int32), bits)

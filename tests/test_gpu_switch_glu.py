@@ -113,3 +113,38 @@ def test_a_replaced_default_activation_runs(dev, T, what, monkeypatch):
     monkeypatch.undo()
     layer.activation = lambda x, gate: x - gate
     assert torch.equal(y, layer(x, idx))
+
+
+def test_plain_tensors_only(dev, monkeypatch):
+    """What keeps a tensor from the layer's own kernels."""
+    from torch.autograd import forward_ad
+
+    plain = switch_layers._plain
+    t = torch.zeros(4, 64, dtype=torch.bfloat16, device=dev)
+    assert plain(t, 64) and plain(t[2:], 64) and plain(torch.zeros(0, 64, dtype=torch.bfloat16, device=dev), 64)
+    assert not plain(t.cpu(), 64)
+    assert not plain(t.float(), 64)
+    assert not plain(t[:, :32], 32)                      # a stride
+    assert not plain(t.reshape(-1)[4:68].reshape(1, 64), 64)  # 8-byte alignment
+    assert not plain(torch.zeros(4, 60, dtype=torch.bfloat16, device=dev), 60)
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert not plain(t.as_subclass(Sub), 64)
+    p = t.clone().requires_grad_(True)
+    assert not plain(p, 64)
+    with torch.no_grad():
+        assert plain(p, 64)
+    with forward_ad.dual_level():
+        assert not plain(t, 64)
+        assert not plain(forward_ad.make_dual(t, t), 64)
+    seen = []
+    torch.func.vmap(lambda r: seen.append(plain(r, 64)) or r)(t)
+    torch.func.grad(lambda r: seen.append(plain(r, 64)) or r.float().sum())(t)
+    torch.func.jvp(lambda r: seen.append(plain(r, 64)) or r * 2, (t,), (t,))
+    torch.func.functionalize(lambda r: seen.append(plain(r, 64)) or r * 2)(t)
+    torch.jit.trace(lambda r: seen.append(plain(r, 64)) or r * 2, (t,), check_trace=False)
+    assert len(seen) == 5 and not any(seen)
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    assert not plain(t, 64)
