@@ -64,11 +64,13 @@ def test_block_decode_over_mlx_weights(dev, T, resident, I, shared):
         assert bool(((y.double() - both).abs() <= 2.0 ** -7 * both.abs().max()).all())
 
 
-# both sides of the lines between the selecting gate_up and a top-k launch: 256 |
-# 257 experts, top-16 | 17 and 64 pairs below, top-4 | 5 and 16 pairs above
+# both sides of the lines between the selecting gate_up and a top-k launch: up to
+# 256 experts top-32 and 63 pairs, up to 512 top-4 and 64 pairs x top-k, above
+# top-16 and 24 pairs
 @pytest.mark.parametrize("E,k,T,selects", [
-    (256, 10, 6, True), (256, 16, 3, True), (256, 17, 1, False), (64, 8, 8, False), (64, 63, 1, False),
-    (257, 4, 4, True), (257, 4, 5, False), (512, 5, 1, False), (512, 10, 1, False), (1024, 1, 16, True)])
+    (256, 10, 6, True), (256, 32, 1, True), (256, 33, 1, False), (64, 21, 3, True), (64, 8, 8, False),
+    (257, 4, 4, True), (257, 4, 5, False), (512, 5, 1, False), (512, 10, 1, False), (512, 1, 16, True),
+    (513, 16, 1, True), (513, 17, 1, False), (1024, 8, 3, True), (1024, 5, 5, False)])
 def test_block_decode_over_mlx_weights_selects_where_it_pays(dev, E, k, T, selects, monkeypatch):
     print(f"[case] MLX-layout block decode E={E} k={k} T={T}", flush=True)
     g = torch.Generator(device=dev).manual_seed(E + k + T)

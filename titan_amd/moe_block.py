@@ -279,15 +279,15 @@ class SparseMoeBlock:
         """Does a decode call over the MLX tensors let the gate_up kernel pick the
         experts?  Each wave of slot j walks j + 1 rounds of the selection, over 4
         logits per lane up to 256 experts and 16 above, against one launch of
-        router_topk.  The launches' time with / without it, hidden 2048 and 4096,
-        widths 512 to 1536, below 64 pairs: up to 256 experts 0.72-1.00 to top-10,
-        0.75-1.02 at top-16, 0.80-1.07 at top-32, 0.93-1.23 at top-64 (from 64 pairs on
-        0.88-1.11 to top-16); 512 experts 0.76-0.94 up to 16 pairs of top-4 at most,
-        0.86-1.07 beyond these, 0.94-1.27 at top-8 and top-10."""
+        router_topk, which takes 8 up to 512.  The launches' time with / without
+        it (hidden 2048 and 4096, widths 512 to 1536, 1 to 16 tokens, top-1 to
+        top-64): 0.72-1.02 inside these lines, 0.84-3.66 outside."""
         pairs = T * self.top_k
-        if self.num_experts <= 256:
-            return self.top_k <= 16 and pairs < 64
-        return self.top_k <= 4 and pairs <= 16
+        if self.num_experts <= 256:  # outside, 0.88-1.45
+            return self.top_k <= 32 and pairs < 64
+        if self.num_experts <= 512:  # 0.85-3.66, top-8 and top-10 0.94-1.35
+            return self.top_k <= 4 and pairs * self.top_k <= 64
+        return self.top_k <= 16 and pairs <= 24  # 0.84-2.59
 
     def _own(self, *steps: str) -> bool:
         """Are these methods the ones defined here?  A launch that does the work of
