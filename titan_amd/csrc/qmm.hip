@@ -39,7 +39,8 @@
 // A launch and its first dependent read take ~2.8 us of each; the error against
 // 64-bit products is the GEMV's to four digits (0.0016 to 0.0017, the result's
 // bf16 rounding).  Twice the units of x staged at a time measured 2-25% slower
-// (one block per CU then).
+// (144 KB of LDS and more: one block per CU.  The 8-bit form's 96 KB allow no
+// second one as it is, but for three row tiles, 80 KB.)
 #include "qmm.h"
 
 #include "gemm_common.h"
@@ -313,6 +314,9 @@ bool takes(int64_t M, int64_t N, int64_t K, int group_size, int bits) {
   // 4096 x 2048 but 5.2/5.6 for 2048 x 4096) and between two and three of 8-bit
   // ones (at three 7.1/4.9 and 7.5/6.1); group 32, whose units cost it twice
   // the matrix work, at up to eight (4.1/4.2 at 1000 x 2048) and five rows.
+  // Larger K, and K with a tail chunk for the GEMV, meet earlier: at four rows of
+  // 4-bit codes 9.6/6.8 for 5120 x 2560 and 11.8/7.5 for 4096 x 6144, 6.8/6.8 and
+  // 8.2/7.5 at two; the line, drawn by the rows alone, leaves those to the GEMV.
   // Below a few MB of weight reads both are launch-bound and the GEMV's chain
   // is the shorter one.
   const int64_t min_rows = bits == 4 ? (group_size == 32 ? 8 : 5) : (group_size == 32 ? 5 : 3);

@@ -488,7 +488,7 @@ __global__ __launch_bounds__(kScanThreads) void tiles_from_sorted_kernel(const i
 
 // The whole routing step in one block, for up to kFusedMaxN pairs and
 // kFusedMaxE experts.  Wave w owns the contiguous row segment w of
-// kFusedWaves and holds its ids in registers (at most kFusedSteps steps of 64
+// the block's W and holds its ids in registers (at most kFusedSteps steps of 64
 // rows, read once); its histogram row in LDS counts the segment, one block
 // scan in (expert, wave) order turns the rows into each wave's first slot per
 // expert, and the wave then walks its segment in order ranking equal ids with

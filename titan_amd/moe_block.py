@@ -29,8 +29,8 @@ The optional shared expert (language.py:81-89: a dense SwiGLU MLP gated by
 sigmoid(x w_gate)), when it has the routed experts' shape, is one more slot of
 the two decode kernels and one more expert of the prefill's GEMMs, with its
 score from the top-k kernel and its rows added by the weighted sum, so it takes
-no launch of its own; otherwise it runs through the same kernels as a
-one-expert table.  Up to 16 tokens its weights are always the exact affine
+no launch of its own; otherwise (another width, a gate of codes, MLX-layout
+decode, a replaced step) it runs through the same kernels as a one-expert table.  Up to 16 tokens its weights are always the exact affine
 ones, so a sorted call that narrow runs it through the decode kernels.
 
 Resident weights (``resident``): by default one copy, in the tile layout --
@@ -39,9 +39,12 @@ construction and keeps only those, since every path it runs, decode GEMVs and
 prefill grouped GEMMs, has a tile-layout kernel.  The tile layout is made for
 the GEMMs (one contiguous 2 KiB chunk per 64 columns and group); the decode
 GEMVs read it slower than the MLX layout (at one token x top-10 of 256
-experts, hidden 2048: gate_up 5.7 against 5.0 us, down at 8 tokens 14.4
+experts, hidden 2048: gate_up 5.4 against 4.9 us, down at 8 tokens 12.3
 against 11.1 us), so ``resident="both"`` keeps the MLX tensors too and
-decodes from them, at twice the memory.  Shapes outside the tile-layout
+decodes from them, at twice the memory: the one-token block without a shared
+expert takes 11.3 against 12.6 us.  With a shared expert of the routed shape
+the tile layout is the faster one, 14.0 against 20.5 us (its decode kernels take
+it as a slot: three launches instead of six).  Shapes outside the tile-layout
 decode kernels' envelope (hidden a multiple of 2048 up to 8192, intermediate
 512, top-k up to 16) keep the MLX tensors for decode either way.
 """
@@ -104,7 +107,8 @@ class SparseMoeBlock:
     once, here (gate_up in the gate/up-paired row order of the SwiGLU kernels).
     ``resident``: "tiles" keeps only that copy when the tile-layout decode
     kernels take the shape (:func:`tile_decode_supported`); "both" also keeps
-    the MLX tensors and decodes from them (faster GEMVs, twice the memory);
+    the MLX tensors and decodes from them (faster without a shared expert, twice the
+    memory);
     ``prefill_tiles=False`` keeps only the MLX tensors and takes decode widths
     only.  ``nbytes`` reports what stays resident.
 
