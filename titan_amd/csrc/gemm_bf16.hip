@@ -671,14 +671,14 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmA
 // Beyond about six rows per expert (kRowsMaxPerExpert) the activation reads, a
 // row's line per lane and wave where the tile kernel copies each row once per
 // workgroup, are what bounds it.  They do so at fewer rows when these go to few
-// experts: 150 tokens that all choose the same 10 of 512 experts take 107 / 43
-// us (hidden 4096) against the tile kernel's 86 / 21.  Up to kRowsAlways rows
-// even the most uneven routing leaves this kernel ahead (320 rows of 10 to 64
-// experts: at most 0.85 of the tile kernel's time); past them only the device
-// knows, and gemm_either_kernel holds both and goes by the rows per tile: up to
-// 16 the rows kernel (24 to 30 rows per tile: 1.1 to 1.6 times the tile
-// kernel's time at the 4096-column down shape, 0.6 to 1.0 at the others), more
-// the tile kernel.  Against the tile kernel alone over 370 routings (8 to 150
+// experts: 150 tokens on 32 of 512 experts (hidden 4096) take 68.3 / 32.9 us
+// against the tile kernel's 64.7 / 17.7.  Up to kRowsAlways rows even the most
+// uneven routing leaves this kernel ahead (320 rows of 10 to 512 experts: at
+// most 0.88 of the tile kernel's time); past them only the device knows, and
+// gemm_either_kernel holds both and goes by the rows per tile: up to 16 the
+// rows kernel (20 to 30 rows per tile: 1.0 to 1.6 times the tile kernel's time
+// at the 4096-column down shape, 0.6 to 1.2 at the others), more the tile
+// kernel.  Against the tile kernel alone over 370 routings (8 to 150
 // tokens, 10 to all experts used, the three layer shapes 256 x 512 x 2048, 128
 // x 768 x 2048 and 512 x 512 x 4096) the geometric mean is 0.78 and the
 // largest ratio 1.07 (64 experts of 15 rows at that down shape).
@@ -687,7 +687,7 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmA
 //
 // The grid has blocks for the rows there can be (RowsGrid), not for every
 // subtile of max_tiles tiles: 2^15 blocks that return at once cost the
-// 512-expert down launch 9 us of 17.  Past kRowsAlways it is kept at
+// 512-expert down launch 9 us of 17 (8 tokens on 10 experts).  Past kRowsAlways it is kept at
 // kRowsMaxBlocks a subtile, and blocks take further tiles in turn.
 //
 // Two or four groups ahead, and two or four waves per SIMD, measured within 5%
