@@ -46,7 +46,7 @@ def test_rows_kernel_is_the_tile_kernel(dev, rows, N, K, gathered):
 
 # What decides between the two kernels, and the rows kernel's grid, on either
 # side: the rows of a call (320 | more), the rows per tile (16 | more), more
-# tiles and more 33-row tiles than a round of the grid has blocks for, and a
+# tiles and more 33-row tiles than the grid has blocks for at once, and a
 # table past the limit of rows per expert.  (rows per used expert, experts, N)
 @pytest.mark.parametrize("rows,E,N", [
     ((32,) * 10, 100, 512), ((33,) + (32,) * 9, 100, 512),   # 320 and 321 rows
@@ -54,7 +54,7 @@ def test_rows_kernel_is_the_tile_kernel(dev, rows, N, K, gathered):
     ((16,) * 30, 100, 256), ((17,) + (16,) * 29, 100, 256),  # 16 rows per tile and a little more
     ((1,) * 40 + (100, 300, 33), 80, 512),                   # few rows per tile, several large tiles
     ((1,) * 2300, 2400, 256),                                # more tiles than 2048 blocks of one column block
-    ((33, 1, 1) * 150, 900, 4096),                           # more large tiles than the 128 of a round
+    ((33, 1, 1) * 150, 900, 4096),                           # more large tiles than the 128 of one pass
 ])
 def test_either_kernel_is_the_tile_kernel(dev, rows, E, N):
     print(f"[case] rows {len(rows)} x {max(rows)} of {E} experts, N={N}", flush=True)

@@ -687,8 +687,9 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void gemm_bf16_kernel(GemmA
 //
 // The grid has blocks for the rows there can be (RowsGrid), not for every
 // subtile of max_tiles tiles: 2^15 blocks that return at once cost the
-// 512-expert down launch 9 us of 17 (8 tokens on 10 experts).  Past kRowsAlways it is kept at
-// kRowsMaxBlocks a subtile, and blocks take further tiles in turn.
+// 512-expert down launch 9 us of 17 (8 tokens on 10 experts).  Past
+// kRowsAlways it is kept at kRowsMaxBlocks a subtile, and blocks take further
+// tiles in turn.
 //
 // Two or four groups ahead, and two or four waves per SIMD, measured within 5%
 // of three and three; a 32-column unit twice as often (half the dequantisation
@@ -725,7 +726,7 @@ __device__ int large_tile(const Tiles& t, int ntiles, int rows, int j) {
     const int i = ntiles - 1 - base - (int)threadIdx.x;
     const bool f = i >= 0 && tile_rows_of(t, i).valid > rows;
     const uint64_t m = __ballot(f);
-    __syncthreads();  // every wave is done with the last round's counts and result
+    __syncthreads();  // every wave is done with the counts and result before
     if (lane == 0) cnt[wave] = __popcll(m);
     __syncthreads();
     int before = 0, total = 0;
@@ -861,7 +862,7 @@ __device__ __forceinline__ void rows_block(const GemmArgs& a, const RowsGrid& gr
     }
   if (back >= step) return;  // a grid rounded up
   const int ntiles = a.ntiles[0];
-  // one round, unless a caller's own table holds empty or overlapping tiles
+  // one pass, unless a caller's own table holds empty or overlapping tiles
   for (;; back += step) {
     const int tile = sub == 0 ? ntiles - 1 - back
                               : large_tile(Tiles{a.offsets, a.tile_row, a.tile_exp, a.ntiles, a.n_rows, a.num_experts},
